@@ -178,3 +178,17 @@ def test_autotune_leaves_state_untouched(gpu_available):
     b.close()
     for g in gs:
         g.close()
+
+
+def test_untuned_batch_starts_with_whole_wavefronts(gpu_available):
+    """Without autotuning every tunable kernel runs full 64-wide rows of
+    several wavefronts (a batch used to start with 1 x 1 workgroups)."""
+    import fwgpu
+    states = members("sp", kinds=("reg",), n_each=1)
+    print("\n[batch] default workgroup shapes", flush=True)
+    gs = [fwgpu.Solver(st, "sp") for st in states]
+    b = fwgpu.Batch(gs)
+    assert b.shapes() == {"disp": (64, 8), "src_huv": (64, 4), "cell": (64, 4), "mask_brk": (64, 8)}
+    b.close()
+    for g in gs:
+        g.close()
