@@ -23,8 +23,8 @@
 // (FIXED_DT halving, misc.F:283-288) stops with FW_BATCH_DT_CHANGED before
 // the step; one that blows up stops after it.  The UPDATE_MASK and
 // WAVE_BREAKING buffers swap each stage; the launches take that parity as an
-// argument, so one step, recorded once per starting parity, replays from a
-// hipGraph.
+// argument, so one step, recorded once per starting parity (and once more as
+// the first step of a call), replays from a hipGraph.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -204,19 +204,16 @@ __global__ void __launch_bounds__(WideLB<R>::wg256) kb_huv(FWB_ARGS, int pm, int
   huv_body<R, true, P2, XD>(d, M.g, M.p, al, be, M.clk[0], AA, tile_blk(e));
 }
 
-// lines per workgroup of the line solves, as in fw_step (FP64 in 48-row
-// chunks, so that its LDS tile fits)
-constexpr int kTridLines = 16;
-template <class R, int L, int CH>
-__global__ void __launch_bounds__(256) kb_trid_lds(FWB_ARGS, int pm, int pa) {
+template <class R>
+__global__ void __launch_bounds__(kTridThreads) kb_trid_fac(FWB_ARGS, int pm, int pa) {
   FWB_HEAD
-  trid_lds_body<R, L, CH>(mdev(M, pm, pa), M.g, e.aux, tile_blk(e));
+  trid_fac_body<R>(mdev(M, pm, pa), M.g, M.p, e.aux, tile_blk(e));
 }
 
-template <class R>
-__global__ void kb_trid(FWB_ARGS, int pm, int pa) {
+template <class R, bool RES, bool PER>
+__global__ void __launch_bounds__(kTridThreads) kb_trid_solve(FWB_ARGS, int pm, int pa) {
   FWB_HEAD
-  trid_body<R>(mdev(M, pm, pa), M.g, M.p, e.aux, tile_blk(e));
+  trid_lines_body<R, RES, PER>(mdev(M, pm, pa), M.g, e.aux, tile_blk(e));
 }
 
 template <class R>
@@ -306,7 +303,7 @@ struct fw_batch {
   bool periodic = false, disp = false, pow2 = false;
   std::string err;
   hipStream_t stream = nullptr, side = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_fac = nullptr;
   void *members = nullptr;     // Member<R>[n] on the device
   std::vector<char> members_h;  // host image
   void *clk = nullptr;         // n x 4 R
@@ -320,9 +317,11 @@ struct fw_batch {
   size_t pinned_bytes = 0;
   // queues
   std::map<std::string, Queue> q;
+  TridGrid trid{};  // LDS of the line solves
   dim3 shape[G_COUNT] = {kGroupShape[0], kGroupShape[1], kGroupShape[2], kGroupShape[3]};
-  // graphs of one step per starting parity
-  hipGraphExec_t gx[2] = {nullptr, nullptr};
+  // graphs of one step per starting parity, and of the first step of a call
+  hipGraphExec_t gx[3] = {nullptr, nullptr, nullptr};
+  bool trid_fixed = false;  // trid_fixed() holds for every member
   bool use_graph = true;
   int parity = 0;  // stages run so far in this call, mod 2
   std::vector<int> status;
@@ -532,16 +531,22 @@ int build_queues(fw_batch *b) {
   if ((rc = make_line(b, "one1024", dim3(1024), [](int) { return 1; }, [](int) { return 0; }))) return rc;
   auto chunks = [&](int m) { return (int)std::min<size_t>(2048, (mem(m).pe + 2047) / 2048); };
   if ((rc = make_line(b, "copy", dim3(256), chunks, chunks))) return rc;
-  if (b->periodic) {
-    auto nx = [&](int m) { const Geo &g = mem(m).g; return (g.Je - g.Jb + 1 + 63) / 64; };
-    auto ny = [&](int m) { const Geo &g = mem(m).g; return (g.Ie - g.Ib + 1 + 63) / 64; };
-    if ((rc = make_line(b, "trid", dim3(64), [&](int m) { return nx(m) + ny(m); }, nx))) return rc;
+  auto nx = [&](int m) { return trid_grid<R>(mem(m).g, b->periodic).nx; };
+  auto nxy = [&](int m) { const TridGrid t = trid_grid<R>(mem(m).g, b->periodic); return t.nx + t.ny; };
+  if ((rc = make_line(b, "trid", dim3(kTridThreads), nxy, nx))) return rc;
+  if (b->periodic) {  // c' of the x lines only
+    if ((rc = make_line(b, "trid_fac", dim3(kTridThreads), nx, nx))) return rc;
   } else {
-    constexpr int L = kTridLines;
-    auto nx = [&](int m) { const Geo &g = mem(m).g; return (g.Je - g.Jb + 1 + L - 1) / L; };
-    auto ny = [&](int m) { const Geo &g = mem(m).g; return (g.Ie - g.Ib + 1 + L - 1) / L; };
-    if ((rc = make_line(b, "trid", dim3(256), [&](int m) { return nx(m) + ny(m); }, nx))) return rc;
+    if ((rc = make_line(b, "trid_fac", dim3(kTridThreads), nxy, nx))) return rc;
   }
+  int rows = 0;  // of the longest line over all members
+  for (int m = 0; m < b->n; m++) {
+    const Geo &g = mem(m).g;
+    rows = std::max(rows, b->periodic ? g.Ie - g.Ib + 1 : std::max(g.Ie - g.Ib + 1, g.Je - g.Jb + 1));
+  }
+  b->trid = trid_lds<R>(rows);
+  b->trid_fixed = true;
+  for (int m = 0; m < b->n; m++) b->trid_fixed = b->trid_fixed && trid_fixed(mem(m).p);
   if ((rc = make_halo_queue<R>(b, "halo_x", 0))) return rc;
   if ((rc = make_halo_queue<R>(b, "halo_xf", 1))) return rc;
   if ((rc = make_halo_queue<R>(b, "halo_d", 2))) return rc;
@@ -554,10 +559,14 @@ int build_queues(fw_batch *b) {
 // the precision)
 namespace {
 template <class R, typename K, typename... A>
-void bl(fw_batch *b, hipStream_t s, const char *qname, K k, A... args) {
+void bl_lds(fw_batch *b, hipStream_t s, const char *qname, size_t lds, K k, A... args) {
   Queue &Q = b->q[qname];
   if (!Q.n) return;
-  hipLaunchKernelGGL(k, dim3(Q.n), Q.block, 0, s, (const Member<R> *)b->members, (const QEnt *)Q.d, args...);
+  hipLaunchKernelGGL(k, dim3(Q.n), Q.block, lds, s, (const Member<R> *)b->members, (const QEnt *)Q.d, args...);
+}
+template <class R, typename K, typename... A>
+void bl(fw_batch *b, hipStream_t s, const char *qname, K k, A... args) {
+  bl_lds<R>(b, s, qname, 0, k, args...);
 }
 
 // EXCHANGE (+ SPONGE_DAMPING when sponge) at buffer parity par
@@ -574,9 +583,10 @@ void rec_exchange(fw_batch *b, int par, int sponge) {
   bl<R>(b, s, "cell", kb_mask_mul<R>, par, par, sponge, 1);
 }
 
-// one whole step, starting at buffer parity p0 (do_step's sequence)
+// one whole step, starting at buffer parity p0 (do_step's sequence); first:
+// the first step of a call, whose first two stages form the line solves' c'
 template <class R, bool P2>
-int rec_step(fw_batch *b, int p0) {
+int rec_step(fw_batch *b, int p0, bool first) {
   hipStream_t s = b->stream, sd = b->side;
   const R alpha[3] = {(R)0, (R)3 / (R)4, (R)1 / (R)3};
   const R beta[3] = {(R)1, (R)1 / (R)4, (R)2 / (R)3};
@@ -586,6 +596,13 @@ int rec_step(fw_batch *b, int p0) {
   bl<R>(b, s, "dt", kb_dt_partial<R>, par, par);
   bl<R>(b, s, "one", kb_dt_final<R>);
   for (int st = 0; st < 3; st++) {
+    const bool fac = b->disp && ((first && st < 2) || !b->trid_fixed);
+    if (fac) {  // beside the dispersion and the fluxes
+      BCHK(b, hipEventRecord(b->ev_fork, s));
+      BCHK(b, hipStreamWaitEvent(sd, b->ev_fork, 0));
+      bl<R>(b, sd, "trid_fac", kb_trid_fac<R>, par, par);
+      BCHK(b, hipEventRecord(b->ev_fac, sd));
+    }
     if (b->disp && !b->periodic) {
       bl<R>(b, s, "dispf", kb_disp_fused<R, P2>, par, par);
     } else if (b->disp) {
@@ -607,14 +624,19 @@ int rec_step(fw_batch *b, int p0) {
       if (b->disp) bl<R>(b, s, "flux_y", kb_flux_y<R, true, FluxYK<R>::K>, par, par);
       else bl<R>(b, s, "flux_y", kb_flux_y<R, false, FluxYK<R>::K>, par, par);
     }
+    if (fac) BCHK(b, hipStreamWaitEvent(s, b->ev_fac, 0));
     if (b->disp && !b->periodic) bl<R>(b, s, "huv", kb_huv<R, P2, true>, par, par, alpha[st], beta[st]);
     else bl<R>(b, s, "huv", kb_huv<R, P2>, par, par, alpha[st], beta[st]);
     // line solves and the velocity tail beside UPDATE_MASK + WAVE_BREAKING
     BCHK(b, hipEventRecord(b->ev_fork, s));
     BCHK(b, hipStreamWaitEvent(sd, b->ev_fork, 0));
     if (b->disp) {
-      if (b->periodic) bl<R>(b, s, "trid", kb_trid<R>, par, par);
-      else bl<R>(b, s, "trid", kb_trid_lds<R, kTridLines, sizeof(R) == 4 ? 64 : 48>, par, par);
+      auto solve = [&](auto kres, auto kstream) {
+        if (b->trid.res) bl_lds<R>(b, s, "trid", b->trid.lds, kres, par, par);
+        else bl_lds<R>(b, s, "trid", b->trid.lds, kstream, par, par);
+      };
+      if (b->periodic) solve(kb_trid_solve<R, true, true>, kb_trid_solve<R, false, true>);
+      else solve(kb_trid_solve<R, true, false>, kb_trid_solve<R, false, false>);
     }
     bl<R>(b, s, "cell", kb_uv_final<R>, par, par);
     if (!b->disp) bl<R>(b, s, "copy", kb_ubar_from_hu<R>);
@@ -632,8 +654,8 @@ int rec_step(fw_batch *b, int p0) {
 }
 
 template <class R>
-int rec_step_any(fw_batch *b, int p0) {
-  return b->pow2 ? rec_step<R, true>(b, p0) : rec_step<R, false>(b, p0);
+int rec_step_any(fw_batch *b, int p0, bool first) {
+  return b->pow2 ? rec_step<R, true>(b, p0, first) : rec_step<R, false>(b, p0, first);
 }
 
 int destroy_graphs(fw_batch *b) {
@@ -648,14 +670,14 @@ int destroy_graphs(fw_batch *b) {
 template <class R>
 int build_graphs(fw_batch *b) {
   destroy_graphs(b);
-  for (int p0 = 0; p0 < 2; p0++) {
+  for (int k = 0; k < 3; k++) {
     hipGraph_t g = nullptr;
     BCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    int rc = rec_step_any<R>(b, p0);
+    int rc = rec_step_any<R>(b, k & 1, k == 2);
     hipError_t e = hipStreamEndCapture(b->stream, &g);
     if (rc) return rc;
     if (e != hipSuccess) return bfail(b, FW_E_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
-    e = hipGraphInstantiate(&b->gx[p0], g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(&b->gx[k], g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     if (e != hipSuccess) return bfail(b, FW_E_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
   }
@@ -765,11 +787,12 @@ int run_steps(fw_batch *b, int nsteps, double *ms) {
       timing_started = true;
     }
     for (int k = 0; k < cnt; k++) {
-      const int p0 = b->parity;
+      const int p0 = b->parity;  // 0 at the first step of a call
+      const bool first = done + k == 0;
       if (b->use_graph) {
-        BCHK(b, hipGraphLaunch(b->gx[p0], b->stream));
+        BCHK(b, hipGraphLaunch(b->gx[first ? 2 : p0], b->stream));
       } else {
-        if ((rc = rec_step_any<R>(b, p0))) return rc;
+        if ((rc = rec_step_any<R>(b, p0, first))) return rc;
       }
       b->parity ^= 1;  // three stages: the parity flips once per step
     }
@@ -984,7 +1007,8 @@ int fw_batch_create(fw_ctx *const *members, int n, fw_batch **out) {
     if (hipSetDevice(c0->device) != hipSuccess || hipStreamCreate(&b->stream) != hipSuccess ||
         hipStreamCreate(&b->side) != hipSuccess ||
         hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming) != hipSuccess)
+        hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&b->ev_fac, hipEventDisableTiming) != hipSuccess)
       rc = bfail(b, FW_E_HIP, "stream/event creation failed");
   }
   // the members' own queued work (uploads) completes first
@@ -1010,6 +1034,7 @@ int fw_batch_destroy(fw_batch *b) {
   if (b->pinned) (void)hipHostFree(b->pinned);
   if (b->ev_fork) (void)hipEventDestroy(b->ev_fork);
   if (b->ev_join) (void)hipEventDestroy(b->ev_join);
+  if (b->ev_fac) (void)hipEventDestroy(b->ev_fac);
   if (b->side) (void)hipStreamDestroy(b->side);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;

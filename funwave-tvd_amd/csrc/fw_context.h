@@ -57,7 +57,7 @@ struct fw_ctx {
   // third while the line solves run (the three share no array; see
   // do_src_huv); cur is the stream launch() uses
   hipStream_t side = nullptr, side2 = nullptr, cur = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_brk = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_brk = nullptr, ev_fac = nullptr;
   int device = 0;
   std::vector<void *> allocs;
   std::vector<size_t> alloc_sizes;  // bytes of each allocation (snapshots)
@@ -107,6 +107,42 @@ inline size_t plane_elems(const Geo &g) { return (size_t)g.P * (size_t)(g.N + 1)
 
 inline void hadd(HaloList &L, void *p, int vtype, int isint = 0, int spec = 0) {
   L.a[L.n++] = HaloArr{p, vtype, isint, spec};
+}
+
+// Line-solve launch: workgroups of x and y lines, whether the lines' d' fit
+// into LDS (TridCfg), dynamic LDS bytes.  n: rows of the longest line.
+struct TridGrid {
+  int nx, ny;
+  bool res;
+  size_t lds;
+};
+template <class R>
+inline TridGrid trid_lds(int n) {
+  TridGrid t{};
+  t.res = TridCfg<R>::bytes(n, true) <= TridCfg<R>::lds_max;
+  t.lds = TridCfg<R>::bytes(n, t.res);
+  return t;
+}
+template <class R>
+inline TridGrid trid_grid(const Geo &g, bool periodic) {
+  const int nx = g.Ie - g.Ib + 1, ny = g.Je - g.Jb + 1;
+  TridGrid t = trid_lds<R>(periodic ? nx : (nx > ny ? nx : ny));
+  t.nx = (ny + kTridL - 1) / kTridL;
+  t.ny = periodic ? (nx + kTridThreads - 1) / kTridThreads : (nx + kTridL - 1) / kTridL;
+  return t;
+}
+
+// Whether the line solves' c' stay the same from the second stage of a call
+// of whole steps on (the first two stages always form them).  They depend on
+// Depth, MASK9 and, where the diagonal 1 - gm (c_c + c_d) dep^2 is exactly 0,
+// MASK.  A step changes none of these but MASK9 and MASK, in UPDATE_MASK; with
+// the viscosity breaking model that sets MASK9 to 1 over the whole interior,
+// whatever it was (masks.F:165-205), and with -(c_c + c_d) > 0 (any Beta_ref
+// in (-2, 0); the reference's is -0.531) the diagonal is at least 1.  Without
+// either, every stage forms them.
+template <class R>
+inline bool trid_fixed(const Prm<R> &p) {
+  return p.VISC_BRK && p.G1 >= (R)0 && -p.cxc - p.cxd > (R)0 && -p.cyc - p.cyd > (R)0;
 }
 
 // ---- wavemaker tables (host, C library, working precision) ----------------

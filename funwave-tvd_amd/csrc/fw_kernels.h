@@ -1711,9 +1711,21 @@ __global__ void k_sources(Dev<R> d, Geo g, Prm<R> p, R AA) {
 }
 
 // --------------------------------------------------------------------------
+// d/a of one line-solve row as k_trid_solve reads it (d in a kept row)
+template <class R>
+__device__ __forceinline__ R trid_da(R gm, R dep, R dl, int mk, R ka, R kb, R kc, R kd, R t4, bool first) {
+  const R t1 = gm * (ka * dep * dep + kb * dl * dep);
+  const R t2 = (R)1 + gm * (-(kc * dep * dep) - kd * dep * dep);
+  const bool on = t2 != (R)0 || mk > 0;
+  const R a = on ? ddiv(t1, t2) : (R)0, dd = on ? ddiv(t4, t2) : (R)0;
+  return first || !(a != (R)0) ? dd : ddiv(dd, a);
+}
+
+// --------------------------------------------------------------------------
 // ESTIMATE_HUV (etauv_solver.F:53-351): SSP-RK3 update of Eta, Ubar, Vbar;
 // then H = Eta*Gamma3 + Depth on all cells (GET_Eta_U_V_HU_HV :373) and the
-// normalised tridiagonal rows of both line systems (:400-539).
+// right-hand sides of both line systems (:400-539; with FUSED, a and c
+// are formed by k_trid_fac).
 // FUSED: SourceTerms of the cell are formed here (source_terms) instead of
 // read back, which is the same arithmetic on the same inputs: SourceTerms
 // reads nothing ESTIMATE_HUV writes.
@@ -1752,8 +1764,7 @@ __device__ __forceinline__ void huv_body(Dev<R> d, Geo g, Prm<R> p, R al, R be, 
     const bool disp = p.DISPERSION;
     const int mk = d.MASK[o];
     const R m9 = (R)(disp ? d.MASK9 : d.MASK)[o];
-    const R dxl = d.Depth[disp ? IX(i - 1, j) : o], dxr = d.Depth[disp ? IX(i + 1, j) : o];
-    const R dyl = d.Depth[disp ? IX(i, j - 1) : o], dyr = d.Depth[disp ? IX(i, j + 1) : o];
+    const R dxl = d.Depth[disp ? IX(i - 1, j) : o], dyl = d.Depth[disp ? IX(i, j - 1) : o];
     R vxy, dvxy, uxy, duxy, u1p = (R)0, v1p = (R)0;
     if constexpr (XD) {
       // (64-bit addresses here: this kernel is at its register limit, and
@@ -1826,29 +1837,30 @@ __device__ __forceinline__ void huv_body(Dev<R> d, Geo g, Prm<R> p, R al, R be, 
       const R b2 = p.b2;
       const R gm = p.G1 * m9;
       R dep = rmax(depth, mdf);
+      // fw_step's solve takes d/a; fw_estimate_huv's sweep and the periodic y
+      // solve take a, c, d themselves
+      auto raw = [&](R *A, R *C, R *D, R dl, R dr, R ka, R kb, R kc, R kd, R t4) {
+        const R t1 = gm * (ka * dep * dep + kb * dl * dep);
+        const R t2 = (R)1 + gm * (-(kc * dep * dep) - kd * dep * dep);
+        const R t3 = gm * (ka * dep * dep + kb * dep * dr);
+        const bool on = t2 != (R)0 || mk > 0;
+        A[o] = on ? ddiv(t1, t2) : (R)0;
+        C[o] = on ? ddiv(t3, t2) : (R)0;
+        D[o] = on ? ddiv(t4, t2) : (R)0;
+      };
       {
-        R depl = rmax(dxl, mdf), depr = rmax(dxr, mdf);
-        R t1 = gm * (p.cxa * dep * dep + p.cxb * depl * dep);
-        R t2 = (R)1 + gm * (-(p.cxc * dep * dep) - p.cxd * dep * dep);
-        R t3 = gm * (p.cxa * dep * dep + p.cxb * dep * depr);
-        R t4 = ddiv(ub * (R)mk, rmax(h, mdf)) + gm * (-(p.b1h * dep * dep * vxy) - b2 * dep * dvxy);
-        if (t2 != (R)0 || mk > 0) {
-          d.xa[o] = ddiv(t1, t2); d.xc[o] = ddiv(t3, t2); d.xd[o] = ddiv(t4, t2);
-        } else {
-          d.xa[o] = (R)0; d.xc[o] = (R)0; d.xd[o] = (R)0;
-        }
+        const R t4 = ddiv(ub * (R)mk, rmax(h, mdf)) + gm * (-(p.b1h * dep * dep * vxy) - b2 * dep * dvxy);
+        if (FUSED)
+          d.xd[o] = trid_da(gm, dep, rmax(dxl, mdf), mk, p.cxa, p.cxb, p.cxc, p.cxd, t4, i == g.Ib);
+        else
+          raw(d.xa, d.xc, d.xd, rmax(dxl, mdf), rmax(d.Depth[IX(i + 1, j)], mdf), p.cxa, p.cxb, p.cxc, p.cxd, t4);
       }
       {
-        R depl = rmax(dyl, mdf), depr = rmax(dyr, mdf);
-        R t1 = gm * (p.cya * dep * dep + p.cyb * depl * dep);
-        R t2 = (R)1 + gm * (-(p.cyc * dep * dep) - p.cyd * dep * dep);
-        R t3 = gm * (p.cya * dep * dep + p.cyb * dep * depr);
-        R t4 = ddiv(vb * (R)mk, rmax(h, mdf)) + gm * (-(p.b1h * dep * dep * uxy) - b2 * dep * duxy);
-        if (t2 != (R)0 || mk > 0) {
-          d.ya[o] = ddiv(t1, t2); d.yc[o] = ddiv(t3, t2); d.yd[o] = ddiv(t4, t2);
-        } else {
-          d.ya[o] = (R)0; d.yc[o] = (R)0; d.yd[o] = (R)0;
-        }
+        const R t4 = ddiv(vb * (R)mk, rmax(h, mdf)) + gm * (-(p.b1h * dep * dep * uxy) - b2 * dep * duxy);
+        if (FUSED && (XD || !p.PERIODIC))
+          d.yd[o] = trid_da(gm, dep, rmax(dyl, mdf), mk, p.cya, p.cyb, p.cyc, p.cyd, t4, j == g.Jb);
+        else
+          raw(d.ya, d.yc, d.yd, rmax(dyl, mdf), rmax(d.Depth[IX(i, j + 1)], mdf), p.cya, p.cyb, p.cyc, p.cyd, t4);
       }
     } else {
       d.U[o] = ddiv(ub, rmax(h, mdf));
@@ -1863,106 +1875,90 @@ __global__ void __launch_bounds__(WideLB<R>::wg256) k_huv(Dev<R> d, Geo g, Prm<R
   huv_body<R, FUSED, P2, XD>(d, g, p, al, be, DT, AA, grid_blk());
 }
 
-// TRIDx_ser / TRIDy_ser (tridiagnal.F:338-398): Thomas sweeps on rows
-// normalised by the diagonal; a row with A == 0 is left as it is.  One
-// thread per line; x lines walk along the contiguous direction, y lines are
-// coalesced across threads.
-template <class R>
-__device__ __forceinline__ void thomas(R *A, R *C, R *D, R *Z, size_t o0, ptrdiff_t s, int n) {
-  R cprev = C[o0], dprev = D[o0];
-  for (int k = 1; k < n; k++) {
-    size_t o = o0 + k * s;
-    R a = A[o];
-    R c = C[o], dd = D[o];
-    if (a != (R)0) {
-      R den = ddiv((R)1, a) - cprev;
-      c = ddiv(ddiv(c, a), den);
-      dd = ddiv(ddiv(dd, a) - dprev, ddiv((R)1, a) - cprev);
-      C[o] = c;
-      D[o] = dd;
-    }
-    cprev = c;
-    dprev = dd;
-  }
-  size_t ol = o0 + (n - 1) * s;
-  R z = D[ol];
-  Z[ol] = z;
-  for (int k = n - 2; k >= 0; k--) {
-    size_t o = o0 + k * s;
-    z = D[o] - C[o] * z;
-    Z[o] = z;
-  }
+// --------------------------------------------------------------------------
+// Line solves (TRIDx_ser / TRIDy_ser, tridiagnal.F:338-398): Thomas sweeps on
+// rows normalised by the diagonal; the first row and a row with A == 0 are
+// left as they are.  The elimination step of row k (tridiagnal.F:383-388) is
+//   den = 1/a - c'_prev,  c' = (c/a) / den,  d' = (d/a - d'_prev) / den
+// and back substitution is z = d' - c' z_next.
+//
+// The rows' a and c depend on Depth, MASK9 and MASK only, so the work is split
+// in two kernels:
+//   k_trid_fac   forms a, c and runs the c' recurrence, leaving den and c'
+//                (planes xa, xc and ya, yc).  Nothing it reads is written by
+//                FLUXES or ESTIMATE_HUV: it runs on another stream beside
+//                them, and in fw_step only for the stages whose masks may
+//                have changed (do_step).
+//   k_trid_solve runs d' and the back substitution.  The RK update stores
+//                d/a (d in a kept row) in xd, yd.
+// What bounds them is the dependent chain of one row after another, on as
+// many lanes as a workgroup has lines, whatever the occupancy.  In one sweep
+// the c' chain (12 dependent operations, the correctly rounded division
+// among them, ~116 cycles per row) set the pace and d' followed; with den
+// known ahead, the quotient d' is four dependent operations (below).
+// Measured at 2048 x 2048 rows, FP32, x and y lines together: 164 -> 117 us per
+// solve beside UPDATE_MASK and WAVE_BREAKING (106 alone); k_trid_fac takes
+// 157 us beside the dispersion and the fluxes of two stages per call.  1024 x 4
+// periodic (x lines one per thread before): 456 -> 40 us; 96 x 72: 43 -> 11;
+// FP64 1021 x 770: 105 -> 70.
+constexpr int kTridL = 16;    // lines per workgroup: 2 x 2042 lines fill the 256 CUs once
+constexpr int kTridNS = 256;  // staging threads (four waves)
+constexpr int kTridThreads = 64 + kTridNS;
+
+// The mark of a kept row in the denominators' plane: a NaN that no operation
+// forms by itself.
+__device__ __forceinline__ float trid_kept(float) { return __uint_as_float(0x7fc0beefu); }
+__device__ __forceinline__ double trid_kept(double) { return __longlong_as_double(0x7ff8c0be00000000ll); }
+__device__ __forceinline__ bool is_trid_kept(float x) { return __float_as_uint(x) == 0x7fc0beefu; }
+__device__ __forceinline__ bool is_trid_kept(double x) { return __double_as_longlong(x) == 0x7ff8c0be00000000ll; }
+
+// A workgroup's block of lines.  Workgroups go to the XCDs in turn; handing
+// each XCD a contiguous run of line blocks keeps the two blocks of columns
+// that share a 128-byte line (16 FP32 columns are 64 bytes) on one L2.
+__device__ __forceinline__ int line_block(const Blk &B) {
+  if (!B.remap) return B.x;
+  const int xcd = B.x & 7, k = B.x >> 3, per = B.gx >> 3, rem = B.gx & 7;
+  return xcd * per + min(xcd, rem) + k;
 }
 
+// The lines of a workgroup: direction, count, rows and addresses.
 template <class R>
-__device__ __forceinline__ void trid_body(Dev<R> d, Geo g, Prm<R> p, int nxblk, const Blk &B) {
-  const int nx = g.Ie - g.Ib + 1, ny = g.Je - g.Jb + 1;
-  if ((int)B.x < nxblk) {
-    int j = g.Jb + B.x * blockDim.x + threadIdx.x;
-    if (j > g.Je) return;
-    thomas(d.xa, d.xc, d.xd, d.U, IX(g.Ib, j), 1, nx);
-    return;
+struct TridLines {
+  bool x;
+  int line0, nl, n;
+  __device__ __forceinline__ TridLines(const Geo &g, int nxblk, const Blk &B) {
+    const int b = line_block(B);
+    x = b < nxblk;
+    line0 = (x ? b : b - nxblk) * kTridL;
+    nl = min(kTridL, (x ? g.Je - g.Jb + 1 : g.Ie - g.Ib + 1) - line0);
+    n = x ? g.Ie - g.Ib + 1 : g.Je - g.Jb + 1;
   }
-  int i = g.Ib + (B.x - nxblk) * blockDim.x + threadIdx.x;
-  if (i > g.Ie) return;
-  const ptrdiff_t s = (ptrdiff_t)g.P;
-  if (!p.PERIODIC) {
-    thomas(d.ya, d.yc, d.yd, d.V, IX(i, g.Jb), s, ny);
-    return;
+  __device__ __forceinline__ size_t at(const Geo &g, int l, int k) const {
+    return x ? (size_t)(g.Jb + line0 + l - 1) * g.P + (size_t)(g.Ib + k - 1)
+             : (size_t)(g.Jb + k - 1) * g.P + (size_t)(g.Ib + line0 + l - 1);
   }
-  // TRIDy_periodic (tridiagnal.F:59-325, serial path): Sherman-Morrison
-  R *a = d.ya, *c = d.yc, *dd = d.yd;
-  size_t ob = IX(i, g.Jb), oe = IX(i, g.Je);
-  R abeg = a[ob], cend = c[oe];
-  c[ob] = ddiv(c[ob], (R)1 + cend);
-  dd[ob] = ddiv(dd[ob], (R)1 + cend);
-  a[oe] = ddiv(a[oe], (R)1 + abeg);
-  dd[oe] = ddiv(dd[oe], (R)1 + abeg);
-  for (int k = 0; k < ny; k++) d.c1[ob + k * s] = c[ob + k * s];
-  thomas(a, d.c1, dd, d.y1, ob, s, ny);
-  for (int k = 0; k < ny; k++) dd[ob + k * s] = (R)0;
-  dd[ob] = ddiv((R)1, (R)1 + cend);
-  dd[oe] = -ddiv((R)1, (R)1 + abeg);
-  thomas(a, c, dd, d.y2, ob, s, ny);
-  R beta = ddiv(cend * d.y1[ob] - abeg * d.y1[oe], (R)1 - (cend * d.y2[ob] - abeg * d.y2[oe]));
-  for (int k = 0; k < ny; k++) {
-    size_t o = ob + k * s;
-    d.V[o] = d.y1[o] + beta * d.y2[o];
+  // staging slot e of a chunk of CH rows: consecutive threads take
+  // consecutive addresses, along a row for x lines, across columns for y
+  template <int CH>
+  __device__ __forceinline__ void slot(int e, int &l, int &k) const {
+    if (x) { l = e / CH; k = e % CH; } else { l = e % kTridL; k = e / kTridL; }
   }
-}
-template <class R>
-__global__ void k_trid(Dev<R> d, Geo g, Prm<R> p, int nxblk) {
-  trid_body<R>(d, g, p, nxblk, grid_blk());
-}
-
-// Line solves staged through LDS.  A workgroup of 256 threads owns L lines
-// of one direction, processed in chunks of CH rows.  The elimination step of
-// tridiagnal.F:383-388 is
-//   c' = (c/a) / (1/a - c'_prev),  d' = (d/a - d'_prev) / (1/a - c'_prev)
-// (rows with a == 0, and the first row, keep c, d).  1/a, c/a and d/a do not
-// depend on the previous row, so the staging waves form them; what is left
-// are two recurrences, c' alone and d' driven by the denominators of c'.
-// They run on two waves, lane l on line l:
-//   wave 0 eliminates c' of chunk ch and leaves the denominator beside it,
-//   wave 1 eliminates d' of chunk ch-1 from those denominators,
-//   waves 2-3 put chunk ch+1 (loaded during the previous chunk) into LDS,
-//   load chunk ch+2 and write the results of chunk ch-2 back to c, d
-// (coalesced: consecutive threads take consecutive addresses, along a row
-// for x lines and across columns for y lines), with one barrier per chunk
-// and three LDS buffers in rotation.  Back substitution
-// (tridiagnal.F:390-394) runs on wave 0 over the chunks in reverse, the
-// last three still in LDS, while waves 2-3 restage the others.  Every
-// quantity is the same correctly rounded operation on the same operands as
-// in the row-by-row sweep, so results are bitwise the same.  The forward
-// results of all but the last chunk go back to the c, d arrays.
-template <class R>
-struct alignas(4 * sizeof(R)) TridRow {
-  R r, ca, da, keep;  // 1/a, c/a, d/a (or c, d where keep is set, keep_on)
 };
-// A kept row (the first, or A == 0) takes its c, d unchanged.  In FP32 the
-// flag is an all-ones bit mask and the choice one v_bfi_b32 on the serial
-// chain (a compare there would wait for VCC, which the division uses);
-// FP64 keeps 1 / 0 and a select.
+
+// a, c of one row (GET_Eta_U_V_HU_HV, etauv_solver.F:400-539): dl, dr the
+// neighbours' max(Depth, MinDepthFrc) along the line; t2 also normalises d
+template <class R>
+__device__ __forceinline__ void trid_ac(R gm, R dep, R dl, R dr, int mk, R ka, R kb, R kc, R kd, R &a, R &c) {
+  const R t1 = gm * (ka * dep * dep + kb * dl * dep);
+  const R t2 = (R)1 + gm * (-(kc * dep * dep) - kd * dep * dep);
+  const R t3 = gm * (ka * dep * dep + kb * dep * dr);
+  const bool on = t2 != (R)0 || mk > 0;
+  a = on ? ddiv(t1, t2) : (R)0;
+  c = on ? ddiv(t3, t2) : (R)0;
+}
+// A kept row takes its c unchanged.  In FP32 the flag is an all-ones bit mask
+// and the choice one v_bfi_b32 on the serial chain (a compare there would
+// wait for VCC, which the division uses); FP64 keeps 1 / 0 and a select.
 __device__ __forceinline__ float keep_on(float) { return __uint_as_float(0xffffffffu); }
 __device__ __forceinline__ double keep_on(double) { return 1.0; }
 __device__ __forceinline__ float keep_sel(float keep, float kept, float x) {
@@ -1970,16 +1966,6 @@ __device__ __forceinline__ float keep_sel(float keep, float kept, float x) {
   return __uint_as_float((__float_as_uint(kept) & m) | (__float_as_uint(x) & ~m));
 }
 __device__ __forceinline__ double keep_sel(double keep, double kept, double x) { return keep != 0.0 ? kept : x; }
-template <class R>
-struct alignas(2 * sizeof(R)) TridCD {
-  R c, d;  // during elimination d first holds the denominator 1/a - c'_prev
-};
-template <class R, int L, int CH>
-struct TridTile {
-  TridRow<R> v[3][L][CH + 1];  // forward input
-  TridCD<R> o[3][L][CH + 1];   // forward output = backward input
-  R z[2][L][CH + 1];           // backward output
-};
 
 // The serial lanes issue every instruction on their own (one wave per
 // SIMD), so their loops carry no per-row bookkeeping: rows go in groups of
@@ -2014,6 +2000,515 @@ __device__ __forceinline__ void trid_rows(int cnt, Ld ld, Grp grp, Op op) {
 }
 
 constexpr int TG = 8;
+
+// ---- c' and the denominators: wave 0 runs the recurrence of chunk t from
+// LDS, lane l on line l, the other waves form the rows of chunk t+1 and write
+// back chunk t-1; one barrier per chunk.
+constexpr int kFacCH = 32;
+template <class R>
+struct alignas(4 * sizeof(R)) FacRow {
+  R r, ca, keep, pad;  // 1/a, c/a (c where keep is set)
+};
+template <class R>
+struct alignas(2 * sizeof(R)) FacOut {
+  R c, den;
+};
+
+template <class R>
+__device__ __forceinline__ void trid_fac_body(const Dev<R> &d, const Geo &g, const Prm<R> &p, int nxblk, const Blk &B) {
+  constexpr int L = kTridL, CH = kFacCH, PER = L * CH / kTridNS;
+  __shared__ FacRow<R> in[2][L][CH + 1];
+  __shared__ FacOut<R> out[2][L][CH + 1];
+  const TridLines<R> T(g, nxblk, B);
+  R *DEN = T.x ? d.xa : d.ya, *CP = T.x ? d.xc : d.yc;
+  const R ka = T.x ? p.cxa : p.cya, kb = T.x ? p.cxb : p.cyb, kc = T.x ? p.cxc : p.cyc, kd = T.x ? p.cxd : p.cyd;
+  const size_t s = T.x ? 1 : (size_t)g.P;
+  const int t = threadIdx.x, lane = t & 63, st = t - 64;
+  const int nch = (T.n + CH - 1) / CH;
+  auto put = [&](int ch) {
+    R dep[PER], dl[PER], dr[PER];
+    int m9[PER], mk[PER];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {  // every load first, unused slots from the block's first row
+      int l, k;
+      T.template slot<CH>(st + q * kTridNS, l, k);
+      k += ch * CH;
+      const size_t o = l < T.nl && k < T.n ? T.at(g, l, k) : T.at(g, 0, 0);
+      dep[q] = d.Depth[o]; dl[q] = d.Depth[o - s]; dr[q] = d.Depth[o + s];
+      m9[q] = d.MASK9[o]; mk[q] = d.MASK[o];
+    }
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      int l, k;
+      T.template slot<CH>(st + q * kTridNS, l, k);
+      R a, c;
+      trid_ac(p.G1 * (R)m9[q], rmax(dep[q], p.MDF), rmax(dl[q], p.MDF), rmax(dr[q], p.MDF), mk[q], ka, kb, kc, kd, a, c);
+      FacRow<R> v;
+      if (ch * CH + k == 0 || !(a != (R)0)) v = FacRow<R>{(R)0, c, keep_on((R)0), (R)0};
+      else v = FacRow<R>{ddiv((R)1, a), ddiv(c, a), (R)0, (R)0};
+      in[ch & 1][l][k] = v;
+    }
+  };
+  auto store = [&](int ch) {
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      int l, k;
+      T.template slot<CH>(st + q * kTridNS, l, k);
+      if (l < T.nl && ch * CH + k < T.n) {
+        const FacOut<R> v = out[ch & 1][l][k];
+        const size_t o = T.at(g, l, ch * CH + k);
+        DEN[o] = v.den;
+        CP[o] = v.c;
+      }
+    }
+  };
+  if (st >= 0) put(0);
+  __syncthreads();
+  R cprev = (R)0;
+  for (int ch = 0; ch <= nch; ch++) {
+    if (st < 0) {
+      if (ch < nch && lane < T.nl) {
+        const FacRow<R> *row = in[ch & 1][lane];
+        FacOut<R> *o = out[ch & 1][lane];
+        const int cnt = min(CH, T.n - ch * CH);
+        // rows read from LDS one group of TG ahead, two register sets in turn
+        trid_rows<TG>(
+            cnt, [&](int k) { return row[k]; },
+            [&](int k0, const FacRow<R>(&V)[TG]) {
+#pragma unroll
+              for (int q = 0; q < TG; q++) {
+                const R den = V[q].r - cprev;
+                cprev = keep_sel(V[q].keep, V[q].ca, ddiv(V[q].ca, den));
+                o[k0 + q] = FacOut<R>{cprev, keep_sel(V[q].keep, trid_kept((R)0), den)};
+              }
+            },
+            [&](int k, const FacRow<R> &v) {
+              const R den = v.r - cprev;
+              cprev = keep_sel(v.keep, v.ca, ddiv(v.ca, den));
+              o[k] = FacOut<R>{cprev, keep_sel(v.keep, trid_kept((R)0), den)};
+            });
+      }
+    } else {
+      if (ch + 1 < nch) put(ch + 1);
+      if (ch >= 1) store(ch - 1);
+    }
+    __syncthreads();
+  }
+}
+template <class R>
+__global__ void __launch_bounds__(kTridThreads) k_trid_fac(Dev<R> d, Geo g, Prm<R> p, int nxblk) {
+  trid_fac_body<R>(d, g, p, nxblk, grid_blk());
+}
+
+// ---- d' and back substitution.
+// The quotient a/den of the d' chain, a = d/a - d'_prev, by Markstein's
+// method with y = RN(1/den) formed ahead by the staging waves:
+//   FP32: q = RN(a y), q' = RN(q + RN(a - den q) y)  (see mdiv)
+//   FP64: one more such correction, so that the estimate the last one starts
+//         from is within an ulp whatever the operands, which is what the
+//         method's theorem asks for.
+// It is the correctly rounded quotient where nothing under- or overflows and
+// den < 0 (then zeros come out with the right sign too: q + RN(+0 y) with
+// y < 0).  The staging waves raise a flag for a group of G rows with a
+// kept row or a denominator outside [-den_hi, -den_lo]; the serial wave tracks
+// the smallest nonzero |a| of a group beside the chain.  (Large ones need no
+// check: |den| >= 1/2, so a quotient that overflows is one whose exact value
+// does, and it leaves a NaN behind, as an infinite a does.)  A group that
+// fails either, or ends in a NaN, is formed again with the division.
+// Denominators are 1/a - c' with a in (-1/2, 0), c' in (-1, 0): far inside
+// the range unless rows are kept (MASK9 = 0).  The numerators leave it where
+// d' decays to nothing ahead of a wave front or behind the shoreline, for a
+// group or two per line.
+template <class R> struct TridRange;
+template <> struct TridRange<float> {
+  static constexpr float den_lo = 0.5f, den_hi = 0x1p40f;
+};
+template <> struct TridRange<double> {
+  static constexpr double den_lo = 0.5, den_hi = 0x1p40;
+};
+// FP32: |a| >= 2^-80 or a == 0 (the quotient stays above 2^-120 and the
+// residual's last bit above 2^-149); FP64: |a| >= 2^-801 or a == 0
+struct TridTrackF {
+  uint32_t lo = 0xffffffffu;
+  __device__ __forceinline__ void add(float a) {
+    lo = min(lo, (__float_as_uint(a) << 1) - 1u);  // a zero wraps to the largest
+  }
+  __device__ __forceinline__ bool bad() const { return lo < (__float_as_uint(0x1p-80f) << 1) - 1u; }
+};
+struct TridTrackD {
+  int lo = 0;
+  __device__ __forceinline__ void add(double a) { lo = min(lo, __builtin_amdgcn_frexp_exp(a)); }  // 0 for a zero
+  __device__ __forceinline__ bool bad() const { return lo < -800; }
+};
+__device__ __forceinline__ float trid_quot(float a, float den, float y) {
+  const float q = a * y;
+  return __builtin_fmaf(__builtin_fmaf(-den, q, a), y, q);
+}
+__device__ __forceinline__ double trid_quot(double a, double den, double y) {
+  const double q = a * y;
+  const double q1 = __builtin_fma(__builtin_fma(-den, q, a), y, q);
+  return __builtin_fma(__builtin_fma(-den, q1, a), y, q1);
+}
+// RN(1/den): v_rcp_f32 and one Newton step give it for every significand
+// (mdiv); FP64 takes the division
+__device__ __forceinline__ float trid_rcp(float den) {
+  const float y = __builtin_amdgcn_rcpf(den);
+  return __builtin_fmaf(__builtin_fmaf(-den, y, 1.0f), y, y);
+}
+__device__ __forceinline__ double trid_rcp(double den) { return 1.0 / den; }
+
+// Layout in LDS.  Rows are staged in chunks of CH into rings of two buffers;
+// a lane reads and writes the rows of its line 16 bytes at a time, and the
+// line strides are 4 mod 64 words, so that the 16 lanes cover all 64 banks.
+// RES: the d' (then z) of whole lines stay in LDS, 16 x stride(n) values, so
+// that a solve moves 16 B per row and direction in FP32; without room for
+// them (FP32 beyond 2112 rows, FP64 beyond 1024) d' goes back to xd, yd and
+// is read again.
+template <class R>
+struct TridCfg {
+  static constexpr int CH = sizeof(R) == 4 ? 64 : 32;
+  static constexpr int ST = CH + 16 / (int)sizeof(R);
+  static constexpr int G = 64 / (int)sizeof(R);  // rows between two range checks
+  static constexpr int ring = 2 * kTridL * ST;  // values of one ring
+  static constexpr int V = 16 / (int)sizeof(R); // rows of one LDS access
+  static __host__ __device__ constexpr int stride(int n) { return (n + 63) / 64 * 64 + V; }
+  static __host__ __device__ constexpr size_t bytes(int n, bool res) {
+    return (size_t)(3 * ring + (res ? kTridL * stride(n) : ring)) * sizeof(R);
+  }
+  static constexpr size_t lds_max = 160 * 1024 - 256;  // 160 KB less the static flags
+};
+template <class R>
+struct alignas(16) Vec16 {
+  R v[16 / sizeof(R)];
+};
+
+template <class R, bool RES>
+__device__ __forceinline__ void trid_solve_body(const Dev<R> &d, const Geo &g, int nxblk, const Blk &B, char *smem) {
+  using C = TridCfg<R>;
+  constexpr int L = kTridL, CH = C::CH, ST = C::ST, V = C::V, G = C::G, NG = CH / G, NV = G / V, PER = L * CH / kTridNS;
+  R *sA = (R *)smem, *sN = sA + C::ring, *sY = sN + C::ring, *S = sY + C::ring;
+  __shared__ int flag[2][NG];
+  const TridLines<R> T(g, nxblk, B);
+  const R *DEN = T.x ? d.xa : d.ya, *CP = T.x ? d.xc : d.yc;
+  R *DP = T.x ? d.xd : d.yd, *Z = T.x ? d.U : d.V;
+  const int n = T.n, nch = (n + CH - 1) / CH, str = C::stride(n);
+  const int t = threadIdx.x, lane = t & 63, st = t - 64;
+  if (t < 2 * NG) flag[t / NG][t % NG] = 0;
+  // staging slots of this thread
+  int sl[PER], sk[PER];
+#pragma unroll
+  for (int q = 0; q < PER; q++) T.template slot<CH>(max(st, 0) + q * kTridNS, sl[q], sk[q]);
+  const size_t osafe = T.at(g, 0, 0);
+  auto ok = [&](int q, int ch) { return sl[q] < T.nl && ch * CH + sk[q] < n; };
+  // (loads unconditional: an unused slot reads the block's first row)
+  auto addr = [&](int q, int ch) { return ok(q, ch) ? T.at(g, sl[q], ch * CH + sk[q]) : osafe; };
+  auto rix = [&](int b, int q) { return (b * L + sl[q]) * ST + sk[q]; };
+  // Items: forward chunk i for i < nch, then backward chunk 2 nch - 1 - i.
+  // Item i uses ring buffer and register set i & 1; a set is loaded two
+  // items before it is put into LDS.
+  R r0[2][PER], r1[2][PER];
+  auto load = [&](auto SET, int i) {
+    constexpr int s = decltype(SET)::value;
+    if (i < nch) {
+#pragma unroll
+      for (int q = 0; q < PER; q++) {
+        const size_t o = addr(q, i);
+        r0[s][q] = DP[o];
+        r1[s][q] = DEN[o];
+      }
+    } else {
+      const int ch = 2 * nch - 1 - i;
+      if (ch < 0) return;
+#pragma unroll
+      for (int q = 0; q < PER; q++) {
+        const size_t o = addr(q, ch);
+        if (!RES) r0[s][q] = DP[o];
+        r1[s][q] = CP[o];
+      }
+    }
+  };
+  auto put = [&](auto SET, int i) {
+    constexpr int s = decltype(SET)::value;
+    if (i < nch) {
+#pragma unroll
+      for (int q = 0; q < PER; q++) {
+        const bool on = ok(q, i);
+        const R den = on ? r1[s][q] : (R)-1;
+        sA[rix(s, q)] = on ? r0[s][q] : (R)0;
+        sN[rix(s, q)] = den;
+        sY[rix(s, q)] = trid_rcp(den);
+        if (!(den <= -TridRange<R>::den_lo && den >= -TridRange<R>::den_hi)) flag[s][sk[q] / G] = 1;
+      }
+    } else {
+      const int ch = 2 * nch - 1 - i;
+      if (ch < 0) return;
+#pragma unroll
+      for (int q = 0; q < PER; q++) {
+        const bool on = ok(q, ch);
+        // the last row's z is its d': c' counts as 0 there and past it
+        sN[rix(s, q)] = on && ch * CH + sk[q] < n - 1 ? r1[s][q] : (R)0;
+        if (!RES) sA[rix(s, q)] = on ? r0[s][q] : (R)0;
+      }
+    }
+  };
+  // results of item i: d' back to xd, yd (without RES), z to U, V
+  auto store = [&](auto SET, int i) {
+    constexpr int s = decltype(SET)::value;
+    if (i < 0 || (RES && i < nch)) return;
+    const int ch = i < nch ? i : 2 * nch - 1 - i;
+    R *dst = i < nch ? DP : Z;
+#pragma unroll
+    for (int q = 0; q < PER; q++)
+      if (ok(q, ch)) dst[T.at(g, sl[q], ch * CH + sk[q])] = RES ? S[sl[q] * str + ch * CH + sk[q]] : S[rix(s, q)];
+  };
+  R dp = (R)0, z = (R)0;
+  auto ld = [&](const R *a, Vec16<R>(&x)[NV]) {
+#pragma unroll
+    for (int u = 0; u < NV; u++) x[u] = *(const Vec16<R> *)(a + u * V);
+  };
+  auto forward = [&](auto SET, int i) {
+    constexpr int s = decltype(SET)::value;
+    const R *a = sA + (s * L + lane) * ST, *dn = sN + (s * L + lane) * ST, *yy = sY + (s * L + lane) * ST;
+    R *out = RES ? S + lane * str + i * CH : S + (s * L + lane) * ST;
+    const int ng = (min(CH, n - i * CH) + G - 1) / G;
+    // one group: the rows of the next one are read ahead of this one's chain
+    Vec16<R> A[2][NV], N[2][NV], Y[2][NV];
+    int fl[2];
+    auto rd = [&](auto BUF, int k) {
+      constexpr int c = decltype(BUF)::value;
+      fl[c] = flag[s][k];
+      ld(a + k * G, A[c]); ld(dn + k * G, N[c]); ld(yy + k * G, Y[c]);
+    };
+    auto group = [&](auto BUF, auto NEXT, int k) {
+      constexpr int c = decltype(BUF)::value;
+      rd(NEXT, min(k + 1, NG - 1));
+      const R start = dp;
+      std::conditional_t<sizeof(R) == 4, TridTrackF, TridTrackD> tr;
+      Vec16<R> o[NV];
+#pragma unroll
+      for (int u = 0; u < NV; u++) {
+#pragma unroll
+        for (int v = 0; v < V; v++) {
+          const R num = A[c][u].v[v] - dp;
+          tr.add(num);
+          dp = trid_quot(num, N[c][u].v[v], Y[c][u].v[v]);
+          o[u].v[v] = dp;
+        }
+      }
+      if (__builtin_expect(__any(tr.bad() || fl[c] || dp != dp), 0)) {
+        dp = start;
+#pragma unroll
+        for (int u = 0; u < NV; u++) {
+#pragma unroll
+          for (int v = 0; v < V; v++) {
+            const R num = A[c][u].v[v], den = N[c][u].v[v], q = ddiv(num - dp, den);
+            dp = is_trid_kept(den) ? num : q;
+            o[u].v[v] = dp;
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < NV; u++) *(Vec16<R> *)(out + k * G + u * V) = o[u];
+    };
+    using B0 = std::integral_constant<int, 0>;
+    using B1 = std::integral_constant<int, 1>;
+    rd(B0{}, 0);
+    for (int k = 0; k < ng; k += 2) {
+      group(B0{}, B1{}, k);
+      if (k + 1 >= ng) break;
+      group(B1{}, B0{}, k + 1);
+    }
+  };
+  auto backward = [&](auto SET, int i) {
+    constexpr int s = decltype(SET)::value;
+    const int ch = 2 * nch - 1 - i;
+    const R *cc = sN + (s * L + lane) * ST;
+    R *io = RES ? S + lane * str + ch * CH : nullptr;
+    const R *in = RES ? io : sA + (s * L + lane) * ST;
+    R *out = RES ? io : S + (s * L + lane) * ST;
+    const int ng = (min(CH, n - ch * CH) + G - 1) / G;
+    Vec16<R> D[2][NV], Cc[2][NV];
+    ld(in + (NG - 1) * G, D[(NG - 1) & 1]); ld(cc + (NG - 1) * G, Cc[(NG - 1) & 1]);
+#pragma unroll
+    for (int k = NG - 1; k >= 0; k--) {
+      const int b = k & 1;
+      if (k > 0) {
+        ld(in + (k - 1) * G, D[b ^ 1]); ld(cc + (k - 1) * G, Cc[b ^ 1]);
+      }
+      if (k >= ng) continue;
+#pragma unroll
+      for (int u = NV - 1; u >= 0; u--) {
+        Vec16<R> o;
+#pragma unroll
+        for (int v = V - 1; v >= 0; v--) {
+          z = D[b][u].v[v] - Cc[b][u].v[v] * z;
+          o.v[v] = z;
+        }
+        *(Vec16<R> *)(out + k * G + u * V) = o;
+      }
+    }
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  auto turn = [&](auto SET, auto OTHER, int i) {
+    if (st < 0) {
+      if (lane < T.nl) {
+        if (i < nch) forward(SET, i);
+        else backward(SET, i);
+        if (RES && i == nch - 1)  // the rows past the last one, read by the first group backward
+          for (int k = n; k < (n + G - 1) / G * G; k++) S[lane * str + k] = (R)0;
+      }
+      if (lane < NG) flag[decltype(SET)::value][lane] = 0;
+    } else {
+      // (without RES the backward rows need the stored d': a new start there)
+      if (RES || i + 1 != nch) put(OTHER, i + 1);
+      if (RES || i + 3 < nch || i >= nch) load(OTHER, i + 3);
+      if (RES || i != nch) store(OTHER, i - 1);
+    }
+    __syncthreads();
+  };
+  if (st >= 0) {
+    load(S0{}, 0);
+    if (RES || nch > 1) load(S1{}, 1);
+  }
+  __syncthreads();  // the flags are cleared
+  if (st >= 0) {
+    put(S0{}, 0);
+    if (RES || nch > 2) load(S0{}, 2);
+  } else {
+    __builtin_amdgcn_s_setprio(3);  // one wave carries the chain
+  }
+  __syncthreads();
+  for (int i = 0; i < nch; i += 2) {
+    turn(S0{}, S1{}, i);
+    if (i + 1 < nch) turn(S1{}, S0{}, i + 1);
+  }
+  if (!RES) {
+    if (st >= 0) {
+      if (nch & 1) store(S0{}, nch - 1); else store(S1{}, nch - 1);
+    }
+    __syncthreads();
+    if (st >= 0) {  // items nch and nch + 1
+      if (nch & 1) { load(S1{}, nch); load(S0{}, nch + 1); put(S1{}, nch); load(S1{}, nch + 2); }
+      else { load(S0{}, nch); load(S1{}, nch + 1); put(S0{}, nch); load(S0{}, nch + 2); }
+    }
+    __syncthreads();
+  }
+  for (int i = nch & ~1; i < 2 * nch; i += 2) {
+    if (i >= nch) turn(S0{}, S1{}, i);
+    if (i + 1 >= nch && i + 1 < 2 * nch) turn(S1{}, S0{}, i + 1);
+  }
+  if (st >= 0) store(S1{}, 2 * nch - 1);
+}
+
+// TRIDy_periodic (tridiagnal.F:59-325, serial path): Sherman-Morrison, one
+// thread per line (its lines are short).  The RK update keeps a, c, d
+// themselves in ya, yc, yd for it.
+template <class R>
+__device__ __forceinline__ void thomas(R *A, R *C, R *D, R *Z, size_t o0, ptrdiff_t s, int n) {
+  R cprev = C[o0], dprev = D[o0];
+  for (int k = 1; k < n; k++) {
+    size_t o = o0 + k * s;
+    R a = A[o];
+    R c = C[o], dd = D[o];
+    if (a != (R)0) {
+      R den = ddiv((R)1, a) - cprev;
+      c = ddiv(ddiv(c, a), den);
+      dd = ddiv(ddiv(dd, a) - dprev, ddiv((R)1, a) - cprev);
+      C[o] = c;
+      D[o] = dd;
+    }
+    cprev = c;
+    dprev = dd;
+  }
+  size_t ol = o0 + (n - 1) * s;
+  R z = D[ol];
+  Z[ol] = z;
+  for (int k = n - 2; k >= 0; k--) {
+    size_t o = o0 + k * s;
+    z = D[o] - C[o] * z;
+    Z[o] = z;
+  }
+}
+template <class R>
+__device__ __forceinline__ void trid_per_body(const Dev<R> &d, const Geo &g, int blk) {
+  const int ny = g.Je - g.Jb + 1;
+  const int i = g.Ib + blk * blockDim.x + threadIdx.x;
+  if (i > g.Ie) return;
+  const ptrdiff_t s = (ptrdiff_t)g.P;
+  R *a = d.ya, *c = d.yc, *dd = d.yd;
+  size_t ob = IX(i, g.Jb), oe = IX(i, g.Je);
+  R abeg = a[ob], cend = c[oe];
+  c[ob] = ddiv(c[ob], (R)1 + cend);
+  dd[ob] = ddiv(dd[ob], (R)1 + cend);
+  a[oe] = ddiv(a[oe], (R)1 + abeg);
+  dd[oe] = ddiv(dd[oe], (R)1 + abeg);
+  for (int k = 0; k < ny; k++) d.c1[ob + k * s] = c[ob + k * s];
+  thomas(a, d.c1, dd, d.y1, ob, s, ny);
+  for (int k = 0; k < ny; k++) dd[ob + k * s] = (R)0;
+  dd[ob] = ddiv((R)1, (R)1 + cend);
+  dd[oe] = -ddiv((R)1, (R)1 + abeg);
+  thomas(a, c, dd, d.y2, ob, s, ny);
+  R beta = ddiv(cend * d.y1[ob] - abeg * d.y1[oe], (R)1 - (cend * d.y2[ob] - abeg * d.y2[oe]));
+  for (int k = 0; k < ny; k++) {
+    size_t o = ob + k * s;
+    d.V[o] = d.y1[o] + beta * d.y2[o];
+  }
+}
+// PER: the y lines are periodic (workgroups from nxblk on)
+template <class R, bool RES, bool PER>
+__device__ __forceinline__ void trid_lines_body(const Dev<R> &d, const Geo &g, int nxblk, const Blk &B) {
+  extern __shared__ __attribute__((aligned(16))) char trid_smem[];
+  if (PER) {
+    const int b = line_block(B);
+    if (b >= nxblk) {
+      trid_per_body<R>(d, g, b - nxblk);
+      return;
+    }
+  }
+  trid_solve_body<R, RES>(d, g, nxblk, B, trid_smem);
+}
+template <class R, bool RES, bool PER>
+__global__ void __launch_bounds__(kTridThreads) k_trid_solve(Dev<R> d, Geo g, int nxblk) {
+  trid_lines_body<R, RES, PER>(d, g, nxblk, grid_blk());
+}
+
+// ---- the whole solve in one sweep, for fw_estimate_huv, where a, c and d all
+// come from the RK update of the same call (k_trid_fac and k_trid_solve one
+// after the other take 20 % longer there).  A workgroup of 256 threads owns L lines
+// of one direction, processed in chunks of CH rows.  The elimination step of
+// tridiagnal.F:383-388 is
+//   c' = (c/a) / (1/a - c'_prev),  d' = (d/a - d'_prev) / (1/a - c'_prev)
+// (rows with a == 0, and the first row, keep c, d).  1/a, c/a and d/a do not
+// depend on the previous row, so the staging waves form them; what is left
+// are two recurrences, c' alone and d' driven by the denominators of c'.
+// They run on two waves, lane l on line l:
+//   wave 0 eliminates c' of chunk ch and leaves the denominator beside it,
+//   wave 1 eliminates d' of chunk ch-1 from those denominators,
+//   waves 2-3 put chunk ch+1 (loaded during the previous chunk) into LDS,
+//   load chunk ch+2 and write the results of chunk ch-2 back to c, d
+// (coalesced: consecutive threads take consecutive addresses, along a row
+// for x lines and across columns for y lines), with one barrier per chunk
+// and three LDS buffers in rotation.  Back substitution
+// (tridiagnal.F:390-394) runs on wave 0 over the chunks in reverse, the
+// last three still in LDS, while waves 2-3 restage the others.  Every
+// quantity is the same correctly rounded operation on the same operands as
+// in the row-by-row sweep, so results are bitwise the same.  The forward
+// results of all but the last chunk go back to the c, d arrays.
+template <class R>
+struct alignas(4 * sizeof(R)) TridRow {
+  R r, ca, da, keep;  // 1/a, c/a, d/a (or c, d where keep is set, keep_on)
+};
+template <class R>
+struct alignas(2 * sizeof(R)) TridCD {
+  R c, d;  // during elimination d first holds the denominator 1/a - c'_prev
+};
+template <class R, int L, int CH>
+struct TridTile {
+  TridRow<R> v[3][L][CH + 1];  // forward input
+  TridCD<R> o[3][L][CH + 1];   // forward output = backward input
+  R z[2][L][CH + 1];           // backward output
+};
 
 template <class R>
 struct TridDIn {
@@ -2206,8 +2701,13 @@ __device__ __forceinline__ void trid_lds_body(Dev<R> d, Geo g, int nxblk, const 
   }
   if (w >= 2) bwd_store(0, 0);
 }
-template <class R, int L, int CH>
+// PER: the y lines are periodic (256 per workgroup from nxblk on)
+template <class R, int L, int CH, bool PER>
 __global__ void __launch_bounds__(256) k_trid_lds(Dev<R> d, Geo g, int nxblk) {
+  if (PER && (int)blockIdx.x >= nxblk) {
+    trid_per_body<R>(d, g, blockIdx.x - nxblk);
+    return;
+  }
   trid_lds_body<R, L, CH>(d, g, nxblk, grid_blk());
 }
 

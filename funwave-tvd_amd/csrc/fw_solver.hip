@@ -63,19 +63,24 @@ hipEvent_t get_event(fw_ctx *c) {
   return e;
 }
 
+// lds: bytes of dynamic LDS
 template <typename K, typename... A>
-void launch(fw_ctx *c, const char *name, K k, dim3 grid, dim3 block, A... args) {
+void launch_lds(fw_ctx *c, const char *name, K k, dim3 grid, dim3 block, size_t lds, A... args) {
   hipEvent_t a = nullptr, b = nullptr;
   if (c->prof) {
     a = get_event(c);
     b = get_event(c);
     (void)hipEventRecord(a, c->cur);
   }
-  hipLaunchKernelGGL(k, grid, block, 0, c->cur, args...);
+  hipLaunchKernelGGL(k, grid, block, lds, c->cur, args...);
   if (c->prof) {
     (void)hipEventRecord(b, c->cur);
     c->pending.push_back({name, a, b});
   }
+}
+template <typename K, typename... A>
+void launch(fw_ctx *c, const char *name, K k, dim3 grid, dim3 block, A... args) {
+  launch_lds(c, name, k, grid, block, 0, args...);
 }
 
 int collect_profile(fw_ctx *c) {
@@ -471,7 +476,39 @@ int do_sources(fw_ctx *c) {
 }
 
 template <class R>
-int do_solve(fw_ctx *c);
+int do_solve(fw_ctx *c, bool fac);
+
+// The line solves' c' and denominators.  Lines of more than kFacFork rows:
+// on the second stream, beside whatever the main stream does next, which
+// waits for ev_fac before the solve (join_factor).  A pair of cross-stream
+// waits costs about 25 us of host and queue time, k_trid_fac about 75 ns per
+// row, so that shorter lines are faster in line on the main stream.
+constexpr int kFacFork = 400;
+template <class R>
+bool factor_forks(fw_ctx *c) {
+  const Geo &g = c->g;
+  return std::max(g.Ie - g.Ib, c->cfg.PERIODIC ? 0 : g.Je - g.Jb) + 1 > kFacFork;
+}
+template <class R>
+int fork_factor(fw_ctx *c) {
+  const TridGrid tg = trid_grid<R>(c->g, c->cfg.PERIODIC);
+  const dim3 gr(tg.nx + (c->cfg.PERIODIC ? 0 : tg.ny));
+  const bool fork = factor_forks<R>(c);
+  if (fork) {
+    HIPCHK(c, hipEventRecord(c->ev_fork, c->stream));
+    HIPCHK(c, hipStreamWaitEvent(c->side, c->ev_fork, 0));
+    c->cur = c->side;
+  }
+  launch(c, "trid_fac", k_trid_fac<R>, gr, dim3(kTridThreads), c->dev<R>(), c->g, c->prm<R>(), tg.nx);
+  c->cur = c->stream;
+  if (fork) HIPCHK(c, hipEventRecord(c->ev_fac, c->side));
+  return FW_OK;
+}
+template <class R>
+int join_factor(fw_ctx *c) {
+  if (factor_forks<R>(c)) HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_fac, 0));
+  return FW_OK;
+}
 
 template <class R>
 int do_huv(fw_ctx *c, int istage) {
@@ -484,7 +521,7 @@ int do_huv(fw_ctx *c, int istage) {
   // (the unfused update divides by no spacing)
   launch(c, "huv", k_huv<R, false, false>, grid2(g.M, g.N, kBH), kBH, d, g, c->prm<R>(), alpha[istage - 1],
          beta[istage - 1], (R)c->dt, (R)0);
-  return do_solve<R>(c);
+  return do_solve<R>(c, false);
 }
 
 // SourceTerms fused into ESTIMATE_HUV (the whole-step path)
@@ -525,7 +562,7 @@ int do_src_huv(fw_ctx *c, int istage, bool overlap) {
       launch(c, "src_huv", k_huv<R, true, false>, grid2(g.M, g.N, kBH), kBH, d, g, c->prm<R>(), alpha[istage - 1],
              beta[istage - 1], (R)c->dt, AA);
   }
-  if (!overlap) return do_solve<R>(c);
+  if (!overlap) return do_solve<R>(c, true);
   // UPDATE_MASK reads Eta, Depth, H and the old MASK and writes MASKn,
   // MASK9, DepthX/Y; WAVE_BREAKING reads Eta, Depth, H, the dispersion
   // slopes and AGE and writes AGEn, nu_break; the line solves and the
@@ -537,7 +574,7 @@ int do_src_huv(fw_ctx *c, int istage, bool overlap) {
   HIPCHK(c, hipEventRecord(c->ev_fork, c->stream));
   HIPCHK(c, hipStreamWaitEvent(c->side, c->ev_fork, 0));
   HIPCHK(c, hipStreamWaitEvent(c->side2, c->ev_fork, 0));
-  if ((rc = do_solve<R>(c))) return rc;
+  if ((rc = do_solve<R>(c, true))) return rc;
   c->cur = c->side;
   rc = do_mask<R>(c);
   if (rc == FW_OK) {
@@ -563,24 +600,31 @@ template <class R>
 int froude_cap_on_host(fw_ctx *c);
 
 // line solves and the final velocities (GET_Eta_U_V_HU_HV after the
-// coefficient assembly)
+// coefficient assembly); fac: c' has been formed by k_trid_fac (fw_step)
 template <class R>
-int do_solve(fw_ctx *c) {
+int do_solve(fw_ctx *c, bool fac) {
   Dev<R> &d = c->dev<R>();
   const Geo &g = c->g;
-  if (c->cfg.DISPERSION) {
-    int ny = g.Je - g.Jb + 1, nx = g.Ie - g.Ib + 1;
-    if (c->cfg.PERIODIC) {  // short periodic y lines: Sherman-Morrison per thread
-      int bs = 64;
-      int nxblk = (ny + bs - 1) / bs, nyblk = (nx + bs - 1) / bs;
-      launch(c, "trid", k_trid<R>, dim3(nxblk + nyblk), dim3(bs), d, g, c->prm<R>(), nxblk);
+  if (c->cfg.DISPERSION && !fac) {
+    // 16 lines per workgroup; FP64 rows take twice the LDS, so its chunks are
+    // 48 rows (125 KB)
+    constexpr int L = kTridL, CH = sizeof(R) == 4 ? 64 : 48;
+    const int ny = g.Je - g.Jb + 1, nx = g.Ie - g.Ib + 1, nxblk = (ny + L - 1) / L;
+    if (c->cfg.PERIODIC)
+      launch(c, "trid", k_trid_lds<R, L, CH, true>, dim3(nxblk + (nx + 255) / 256), dim3(256), d, g, nxblk);
+    else
+      launch(c, "trid", k_trid_lds<R, L, CH, false>, dim3(nxblk + (nx + L - 1) / L), dim3(256), d, g, nxblk);
+  } else if (c->cfg.DISPERSION) {
+    const TridGrid tg = trid_grid<R>(g, c->cfg.PERIODIC);
+    const dim3 gr(tg.nx + tg.ny), b(kTridThreads);
+    if (c->cfg.PERIODIC) {
+      if (tg.res) launch_lds(c, "trid", k_trid_solve<R, true, true>, gr, b, tg.lds, d, g, tg.nx);
+      else launch_lds(c, "trid", k_trid_solve<R, false, true>, gr, b, tg.lds, d, g, tg.nx);
     } else {
-      // 16 lines per workgroup (2 x 2048 lines: one workgroup per CU);
-      // FP64 rows take twice the LDS, so its chunks are 48 rows (125 KB)
-      constexpr int L = 16, CH = sizeof(R) == 4 ? 64 : 48;
-      int nxblk = (ny + L - 1) / L, nyblk = (nx + L - 1) / L;
-      launch(c, "trid", k_trid_lds<R, L, CH>, dim3(nxblk + nyblk), dim3(256), d, g, nxblk);
+      if (tg.res) launch_lds(c, "trid", k_trid_solve<R, true, false>, gr, b, tg.lds, d, g, tg.nx);
+      else launch_lds(c, "trid", k_trid_solve<R, false, false>, gr, b, tg.lds, d, g, tg.nx);
     }
+    HIPCHK(c, hipGetLastError());  // (the only launch with more than 64 KB of dynamic LDS)
   }
   launch(c, "uv_final", k_uv_final<R>, grid2(g.M, g.N, kB2), kB2, d, g, c->prm<R>());
   if (c->prm<R>().host_math) {
@@ -683,8 +727,11 @@ int do_step(fw_ctx *c, int nsteps) {
     if ((rc = do_exchange<R>(c, false))) return rc;
     if ((rc = do_estimate_dt<R>(c, true))) return rc;
     for (int st = 1; st <= 3; st++) {
+      const bool fac = f.DISPERSION && (3 * s + st <= 2 || !trid_fixed(c->prm<R>()));
+      if (fac && (rc = fork_factor<R>(c))) return rc;
       if (f.DISPERSION && (rc = do_dispersion<R>(c, true))) return rc;
       if ((rc = do_fluxes<R>(c))) return rc;
+      if (fac && (rc = join_factor<R>(c))) return rc;
       if ((rc = do_src_huv<R>(c, st, true))) return rc;
       if ((rc = do_exchange<R>(c, f.DIRECT_SPONGE != 0))) return rc;
     }
@@ -817,6 +864,7 @@ int fw_create(const fw_config *cfg, fw_ctx **out) {
       hipStreamCreate(&c->side) != hipSuccess || hipStreamCreate(&c->side2) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&c->ev_fac, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_brk, hipEventDisableTiming) != hipSuccess) {
     fw_destroy(c);
     return FW_E_HIP;
@@ -866,6 +914,7 @@ int fw_destroy(fw_ctx *c) {
   if (c->pinned) (void)hipHostFree(c->pinned);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
+  if (c->ev_fac) (void)hipEventDestroy(c->ev_fac);
   if (c->ev_brk) (void)hipEventDestroy(c->ev_brk);
   if (c->side) (void)hipStreamDestroy(c->side);
   if (c->side2) (void)hipStreamDestroy(c->side2);

@@ -1,0 +1,81 @@
+"""The line solves (k_trid_fac, k_trid_solve) at the sizes where their
+chunking can go wrong, against the oracle: lines shorter than one check
+group, of whole and partial chunks (32 and 64 rows) and groups (8 and 16),
+longer than what fits into LDS (FP32 beyond 2112 rows, FP64 beyond 1024),
+partial blocks of 16 lines, rows that are kept (MASK9 = 0) and numerators
+that decay to zero.  Every quantity is the same correctly rounded operation
+as the oracle's, so the tolerance is none: every array bit for bit (with the
+Froude cap's per-cell ATAN2, COS and SIN left to the host, as there)."""
+import numpy as np
+import pytest
+
+from common import bitwise_mismatch
+
+pytestmark = pytest.mark.gpu
+
+KEYS = ["Eta", "U", "V", "HU", "HV", "Ubar", "Vbar", "H", "MASK", "MASK9", "U4", "V4", "P", "Q", "nu_break"]
+
+
+def _state(m, n, prec, visc, quiet, periodic=False):
+    """A sloping beach that dries at its east end, with random small waves in
+    its western part only when quiet is set (still water elsewhere)."""
+    import fwcases
+    import fwsetup
+    c = fwcases.beach_1d(mglob=m, nglob=n, xslp=0.4 * m, xc_wk=0.2 * m, sponge_west=min(10.0, 0.1 * m))
+    x = np.arange(m) + 0.5
+    c.depth = np.tile(np.where(x > 0.4 * m, 4.0 - 8.0 * (x / m - 0.4), 4.0), (n, 1))
+    c.params.update({"DEPTH_TYPE": "DATA", "PERIODIC": periodic, "VISCOSITY_BREAKING": visc, "WAVEMAKER": "NONE",
+                     "DIRECT_SPONGE": False})
+    st = fwsetup.build_state(c, prec)
+    rng = np.random.default_rng(m * 1000 + n)
+    on = st["MASK"] * (st["Depth"] > 1.0)
+    if quiet:
+        on = on * (np.arange(m + 6) < 0.3 * (m + 6))[None, :]
+    rdt = st["Depth"].dtype
+    for k, a in (("Eta", 0.05), ("U", 0.1), ("V", 0.1)):
+        st[k] = np.where(on > 0, (a * rng.standard_normal(on.shape)), st.get(k, 0)).astype(rdt)
+    st["H"] = np.where(on > 0, st["Eta"] + st["Depth"], st["H"]).astype(rdt)
+    st["HU"], st["HV"] = (st["H"] * st["U"]).astype(rdt), (st["H"] * st["V"]).astype(rdt)
+    st["Ubar"], st["Vbar"] = st["HU"].copy(), st["HV"].copy()
+    return st
+
+
+SIZES = [(3, 3), (9, 17), (16, 15), (31, 33), (64, 16), (65, 129), (127, 48), (200, 3), (1023, 5), (1025, 7),
+         (2048, 3), (2113, 4), (5, 2300)]
+
+
+@pytest.mark.parametrize("prec", ["sp", "dp"])
+@pytest.mark.parametrize("m,n", SIZES)
+def test_lines_match_oracle(m, n, prec, gpu_available):
+    import fwgpu
+    import oracle
+    for visc, quiet in ((True, True), (False, False)):
+        print(f"\n[line solves] {m} x {n} {prec} viscosity={visc} quiet={quiet}", flush=True)
+        st = _state(m, n, prec, visc, quiet)
+        g, o = fwgpu.Solver(st, prec, host_math=True), oracle.OracleSolver(st)
+        for steps in (1, 2):
+            assert g.step(steps) == (o.run(steps), (o.dt.value, o.time.value))[1]
+            bad = {k: bitwise_mismatch(g.download(k), o[k]) for k in KEYS}
+            assert not any(bad.values()), bad
+        # and routine by routine: c' beside ESTIMATE_HUV's own kernel
+        g.dispersion(); o.dispersion()
+        g.fluxes(); o.fluxes()
+        g.sources(); o.sources()
+        g.estimate_huv(2); o.estimate_huv(2)
+        bad = {k: bitwise_mismatch(g.download(k), o[k]) for k in ("Eta", "U", "V", "HU", "HV")}
+        assert not any(bad.values()), bad
+        g.close()
+
+
+@pytest.mark.parametrize("prec", ["sp", "dp"])
+@pytest.mark.parametrize("m,n", [(40, 3), (333, 4), (64, 21)])
+def test_periodic_lines_match_oracle(m, n, prec, gpu_available):
+    import fwgpu
+    import oracle
+    print(f"\n[line solves] periodic {m} x {n} {prec}", flush=True)
+    st = _state(m, n, prec, True, False, periodic=True)
+    g, o = fwgpu.Solver(st, prec, host_math=True), oracle.OracleSolver(st)
+    assert g.step(3) == (o.run(3), (o.dt.value, o.time.value))[1]
+    bad = {k: bitwise_mismatch(g.download(k), o[k]) for k in KEYS}
+    assert not any(bad.values()), bad
+    g.close()
