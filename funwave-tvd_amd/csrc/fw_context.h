@@ -76,6 +76,10 @@ struct fw_ctx {
   hipEvent_t slot_ev[kStageSlots]{};
   int slot_next = 0;
   void *scal = nullptr;  // device scalars
+  // values the step kernels hand to the host: [0] DT, [1] max |eta| and the
+  // breaking flag (pinned memory, as the host and as the device see it)
+  fw::Pub *pub = nullptr, *pub_dev = nullptr;
+  unsigned pub_seq = 0;
   std::string err;
   bool prof = false;
   std::vector<PendingEvent> pending;

@@ -62,6 +62,10 @@ struct Dev {
   // (U1pp + U2) + U3 and (V1pp + V2) + V3, the only form in which the fused
   // RK update reads the nonlinear dispersive terms
   R *sumU, *sumV;
+  // where ESTIMATE_HUV leaves the new Eta: Eta itself, or (whole steps of a
+  // non-periodic domain) a plane of its own, so that k_tail can read it around
+  // a cell while it writes Eta
+  R *EtaW, *eta2;
   // reductions and breaking candidates
   R *red;          // block partials
   double *red64;   // FP64 partials (stats)

@@ -198,6 +198,40 @@ template <class R>
 __global__ void k_halo(HaloList L, Geo g, int mode) {
   halo_body<R>(L.a[blockIdx.y], g, mode, grid_blk());
 }
+// Periodic fill of one cell array (modes 1 and 2 in one pass).  An x-ghost
+// cell of an interior row first gives the value it holds to the y-ghost rows
+// that copy its row, as the reference's y copy does before its x fill, and
+// then takes its mirror value; the y-ghost rows of the interior columns copy
+// interior cells, which nothing here writes.
+template <class R>
+__device__ __forceinline__ void halo_per_body(const HaloArr &A, const Geo &g, const Blk &B) {
+  int t = B.x * blockDim.x + threadIdx.x;
+  const int nx = g.Ie - g.Ib + 1, ny = g.Je - g.Jb + 1;
+  auto fill = [&](auto *ph) {
+    if (t < 6 * nx) {
+      const int r = t / nx, i = g.Ib + t % nx;
+      const int j = r < 3 ? 1 + r : g.Je - 2 + r;  // 1..3, Je+1..Je+3
+      ph[IX(i, j)] = ph[IX(i, r < 3 ? g.Je - 3 + j : 3 + (j - g.Je))];
+      return;
+    }
+    t -= 6 * nx;
+    if (t >= 6 * ny) return;
+    const int r = t % 6, j = g.Jb + t / 6;
+    const int i = r < 3 ? 1 + r : g.Ie - 2 + r;
+    const auto old = ph[IX(i, j)], v = ph[IX(r < 3 ? 2 * g.Ib - 1 - i : 2 * g.Ie + 1 - i, j)];
+    if (j > g.Je - 3) ph[IX(i, j - (g.Je - 3))] = old;
+    if (j < g.Jb + 3) ph[IX(i, j - 3 + g.Je)] = old;
+    ph[IX(i, j)] = A.vtype == 2 ? -v : v;
+  };
+  if (A.isint) fill((int *)A.p);
+  else fill((R *)A.p);
+}
+// cell arrays of L periodic, face arrays of Lf mirrored
+template <class R>
+__global__ void k_halo_per(HaloList L, HaloList Lf, Geo g) {
+  if ((int)blockIdx.y < L.n) halo_per_body<R>(L.a[blockIdx.y], g, grid_blk());
+  else halo_body<R>(Lf.a[blockIdx.y - L.n], g, 0, grid_blk());
+}
 
 // --------------------------------------------------------------------------
 // ESTIMATE_DT (misc.F:216-296) over all cells including ghosts; the block
@@ -248,6 +282,15 @@ __global__ void k_dt_partial(Dev<R> d, Geo g, Prm<R> p, int copy_uv) {
   dt_partial_body<R>(d, g, p, copy_uv, grid_blk());
 }
 
+// DT from the smallest dx / (|u| + c) (misc.F:270-288)
+template <class R>
+__device__ __forceinline__ R dt_of(const Prm<R> &p, R least) {
+  const R dtt = p.CFL * least;
+  if (!p.FIXED_DT) return dtt;
+  R dt = p.DTF;
+  while (dt > dtt) dt = ddiv(dt, (R)2);
+  return dt;
+}
 template <class R>
 __device__ __forceinline__ void dt_final_body(Dev<R> d, Prm<R> p, int nblk, R *out, const Blk &B) {
   __shared__ R sm[256];
@@ -259,21 +302,54 @@ __device__ __forceinline__ void dt_final_body(Dev<R> d, Prm<R> p, int nblk, R *o
     if (threadIdx.x < s) sm[threadIdx.x] = rmin(sm[threadIdx.x], sm[threadIdx.x + s]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    R dtt = p.CFL * sm[0];
-    R dt;
-    if (p.FIXED_DT) {
-      dt = p.DTF;
-      while (dt > dtt) dt = ddiv(dt, (R)2);
-    } else {
-      dt = dtt;
-    }
-    out[0] = dt;
-  }
+  if (threadIdx.x == 0) out[0] = dt_of(p, sm[0]);
 }
 template <class R>
 __global__ void k_dt_final(Dev<R> d, Prm<R> p, int nblk, R *out) {
   dt_final_body<R>(d, p, nblk, out, grid_blk());
+}
+// A value handed to the host through pinned memory: the host spins on seq
+// (a few us) instead of a copy and a stream synchronisation (12 us).
+struct Pub {
+  double val;
+  int flag;
+  unsigned seq;
+};
+__device__ __forceinline__ void publish(Pub *pub, double val, int flag, unsigned seq) {
+  pub->val = val;
+  pub->flag = flag;
+  __threadfence_system();
+  __hip_atomic_store(&pub->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// the extreme of n block extremes, by one workgroup of 1024 threads (eight
+// loads of a thread in flight together); the result in thread 0
+template <class R, bool MAX>
+__device__ __forceinline__ R extreme1024(const R *red, int n, R none) {
+  __shared__ R sm[1024];
+  R m = none;
+  for (int k0 = threadIdx.x; k0 < n; k0 += 8 * 1024) {
+    R a[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) a[k] = red[min(k0 + k * 1024, n - 1)];
+#pragma unroll
+    for (int k = 0; k < 8; k++) m = MAX ? rmax(m, a[k]) : rmin(m, a[k]);
+  }
+  sm[threadIdx.x] = m;
+  __syncthreads();
+  for (int s = 512; s > 0; s >>= 1) {
+    if ((int)threadIdx.x < s)
+      sm[threadIdx.x] = MAX ? rmax(sm[threadIdx.x], sm[threadIdx.x + s]) : rmin(sm[threadIdx.x], sm[threadIdx.x + s]);
+    __syncthreads();
+  }
+  return sm[0];
+}
+template <class R>
+__global__ void __launch_bounds__(1024) k_dt_pub(Dev<R> d, Prm<R> p, int nblk, R *out, Pub *pub, unsigned seq) {
+  const R least = extreme1024<R, false>(d.red, nblk, Lit<R>::large());
+  if (threadIdx.x == 0) {
+    out[0] = dt_of(p, least);
+    publish(pub, (double)out[0], 0, seq);
+  }
 }
 
 // max |eta| over the interior (CHECK_BLOWUP, misc.F:394-433)
@@ -323,6 +399,11 @@ __device__ __forceinline__ void max_final_body(Dev<R> d, int nblk, R *out, const
 template <class R>
 __global__ void k_max_final(Dev<R> d, int nblk, R *out) {
   max_final_body<R>(d, nblk, out, grid_blk());
+}
+template <class R>
+__global__ void __launch_bounds__(1024) k_max_pub(Dev<R> d, int nblk, Pub *pub, unsigned seq) {
+  const R m = extreme1024<R, true>(d.red, nblk, (R)0);
+  if (threadIdx.x == 0) publish(pub, (double)m, d.flags[0], seq);
 }
 
 // plain copies of whole pitched arrays (Eta0 := Eta etc.)
@@ -527,9 +608,11 @@ __device__ __forceinline__ void disp_deriv_body(Dev<R> d, Geo g, Prm<R> p, R DT,
     d.DVtxy[o] = wall ? (R)0 : gfxy<R>(DVT, i, j, dx, dy) * m9;
   }
 }
+// (dtp: DT where ESTIMATE_DT left it on the device, for launches queued before
+// the host has it)
 template <class R, bool P2>
-__global__ void __launch_bounds__(WideLB<R>::wg512) k_disp_deriv(Dev<R> d, Geo g, Prm<R> p, R DT) {
-  disp_deriv_body<R, P2>(d, g, p, DT, grid_blk());
+__global__ void __launch_bounds__(WideLB<R>::wg512) k_disp_deriv(Dev<R> d, Geo g, Prm<R> p, R DT, const R *dtp) {
+  disp_deriv_body<R, P2>(d, g, p, dtp ? *dtp : DT, grid_blk());
 }
 
 // CAL_DISPERSION part 2: U4, V4, U1p, V1p on all cells (:293-330) and the
@@ -699,8 +782,8 @@ __device__ __forceinline__ void disp_terms_body(Dev<R> d, Geo g, Prm<R> p, R DT,
   disp_terms_at<R, P2>(d, g, p, DT, i, j, S);
 }
 template <class R, bool P2>
-__global__ void __launch_bounds__(WideLB<R>::wg512) k_disp_terms(Dev<R> d, Geo g, Prm<R> p, R DT) {
-  disp_terms_body<R, P2>(d, g, p, DT, grid_blk());
+__global__ void __launch_bounds__(WideLB<R>::wg512) k_disp_terms(Dev<R> d, Geo g, Prm<R> p, R DT, const R *dtp) {
+  disp_terms_body<R, P2>(d, g, p, dtp ? *dtp : DT, grid_blk());
 }
 
 // --------------------------------------------------------------------------
@@ -841,8 +924,8 @@ __device__ __forceinline__ void disp_fused_body(Dev<R> d, Geo g, Prm<R> p, R DT,
   }
 }
 template <class R, bool P2>
-__global__ void __launch_bounds__(kDispTX * kDispTY) k_disp_fused(Dev<R> d, Geo g, Prm<R> p, R DT) {
-  disp_fused_body<R, P2>(d, g, p, DT, grid_blk());
+__global__ void __launch_bounds__(kDispTX * kDispTY) k_disp_fused(Dev<R> d, Geo g, Prm<R> p, R DT, const R *dtp) {
+  disp_fused_body<R, P2>(d, g, p, dtp ? *dtp : DT, grid_blk());
 }
 
 // --------------------------------------------------------------------------
@@ -1829,7 +1912,7 @@ __device__ __forceinline__ void huv_body(Dev<R> d, Geo g, Prm<R> p, R al, R be, 
     R r3 = -(p.rDX * (gx1 * nr + gx0 * nl)) - p.rDY * (gy1 * nr + gy0 * nl) + srcy;
     R vb = al * vbar0 + be * (vbar + DT * r3);
     R h = eta * p.G3 + depth;
-    d.Eta[o] = eta;
+    d.EtaW[o] = eta;
     d.Ubar[o] = ub;
     d.Vbar[o] = vb;
     d.H[o] = h;
@@ -1868,6 +1951,7 @@ __device__ __forceinline__ void huv_body(Dev<R> d, Geo g, Prm<R> p, R al, R be, 
     }
   } else {
     d.H[o] = eta * p.G3 + d.Depth[o];
+    if (FUSED) d.EtaW[o] = eta;  // (its own value where EtaW is Eta)
   }
 }
 template <class R, bool FUSED, bool P2, bool XD = false>
@@ -2788,13 +2872,13 @@ __device__ __forceinline__ int new_mask(const Dev<R> &d, const Geo &g, int i, in
   int m = d.MASK[o];
   if (i < g.Ib - 2 || i > g.Ie + 2 || j < g.Jb - 2 || j > g.Je + 2) return m;
   if (d.MASK_STRUC[o] != 1) return m;
-  R e = d.Eta[o];
+  R e = d.EtaW[o];
   if (m < 1) {
     if (e > -d.Depth[o]) m = 1;
-    if (d.MASK[IX(i - 1, j)] == 1 && d.Eta[IX(i - 1, j)] > e) m = 1;
-    if (d.MASK[IX(i + 1, j)] == 1 && d.Eta[IX(i + 1, j)] > e) m = 1;
-    if (d.MASK[IX(i, j - 1)] == 1 && d.Eta[IX(i, j - 1)] > e) m = 1;
-    if (d.MASK[IX(i, j + 1)] == 1 && d.Eta[IX(i, j + 1)] > e) m = 1;
+    if (d.MASK[IX(i - 1, j)] == 1 && d.EtaW[IX(i - 1, j)] > e) m = 1;
+    if (d.MASK[IX(i + 1, j)] == 1 && d.EtaW[IX(i + 1, j)] > e) m = 1;
+    if (d.MASK[IX(i, j - 1)] == 1 && d.EtaW[IX(i, j - 1)] > e) m = 1;
+    if (d.MASK[IX(i, j + 1)] == 1 && d.EtaW[IX(i, j + 1)] > e) m = 1;
   } else {
     if (e < -d.Depth[o]) m = 0;
   }
@@ -2932,18 +3016,17 @@ __device__ __forceinline__ R brk_prop(const Dev<R> &d, const Geo &g, const BrkIn
   return t ? DT : own;
 }
 template <class R>
-__device__ __forceinline__ R brk_nu(const Dev<R> &d, const Geo &g, const Prm<R> &p, const BrkIn<R> &b, size_t o, int i,
-                                    int j, R age) {
+__device__ __forceinline__ R brk_nu(const Prm<R> &p, const Geo &g, const BrkIn<R> &b, int i, int j, R age, R dep, R eta) {
   R xmk = (R)(i - g.Ib) * p.DX, ymk = (R)(j - g.Jb) * p.DY;
   if (dabs(xmk - p.XC) < p.WW && dabs(ymk - p.YC) < half(p.YW)) {
     if (b.et > rmin(b.t2, p.WKC * b.t3)) {
-      R cap1 = (R)1 * (rmax(d.Depth[o], p.MDF) + d.Eta[o]);
+      R cap1 = (R)1 * (rmax(dep, p.MDF) + eta);
       return cap1 * p.WKC * b.t3 + p.NUB;
     }
     return (R)0 + p.NUB;
   }
   if (age > (R)0 && age < p.TBRK && b.et > b.t2) {
-    R cap1 = (R)1 * (rmax(d.Depth[o], p.MDF) + d.Eta[o]);
+    R cap1 = (R)1 * (rmax(dep, p.MDF) + eta);
     return cap1 * b.t2 + p.NUB;
   }
   return (R)0 + p.NUB;
@@ -2984,27 +3067,30 @@ __global__ void k_roller(Dev<R> d, Geo g, Prm<R> p) {
   d.UNDERTOW_V[o] = -(rf * sn);
 }
 
+// First pass of one cell: its new age and viscosity from the old ages.  Only a
+// cell that may take the propagation branch forms the angle and the travel
+// times (brk_in: an ATAN2 and four divisions).
 template <class R>
-__device__ __forceinline__ void brk1_body(Dev<R> d, Geo g, Prm<R> p, R DT, const Blk &B) {
-  const Tile tb = xcd_tile(B);
-  int i = 1 + tb.x * blockDim.x + threadIdx.x;
-  int j = 1 + tb.y * blockDim.y + threadIdx.y;
-  if (i > g.M || j > g.N) return;
-  size_t o = IX(i, j);
-  R age = d.AGE_BREAKING[o];
-  if (i < g.Ib - 1 || i > g.Ie + 1 || j < g.Jb - 1 || j > g.Je + 1) {
+__device__ __forceinline__ void brk1_cell(const Dev<R> &d, const Geo &g, const Prm<R> &p, R DT, int i, int j, size_t o,
+                                          bool ring, R age, R et, R h, R dep, R eta) {
+  if (!ring) {
     d.AGEn[o] = age;
     return;
   }
-  BrkIn<R> b = brk_in(d, g, p, o);
+  BrkIn<R> b;
+  b.t3 = dsqrt(GRAV * rmax(p.MDF, h));
+  b.t1 = p.C1 * b.t3;
+  b.t2 = p.C2 * b.t3;
+  b.et = et;
   R na;
-  if (b.et >= b.t1 && (age == (R)0 || age > p.TBRK)) {
+  if (et >= b.t1 && (age == (R)0 || age > p.TBRK)) {
     na = DT;
   } else if (age > (R)0) {
     na = age + DT;
   } else {
     na = age;
-    if (b.et >= b.t2) {
+    if (et >= b.t2) {
+      b = brk_in(d, g, p, o);
       int q = brk_quad(b.ang);
       if (q != 0) {
         na = brk_prop(d, g, b, q, i, j, d.AGE_BREAKING, d.AGE_BREAKING, DT, age);
@@ -3019,7 +3105,17 @@ __device__ __forceinline__ void brk1_body(Dev<R> d, Geo g, Prm<R> p, R DT, const
     }
   }
   d.AGEn[o] = na;
-  d.nu_break[o] = brk_nu(d, g, p, b, o, i, j, na);
+  d.nu_break[o] = brk_nu(p, g, b, i, j, na, dep, eta);
+}
+template <class R>
+__device__ __forceinline__ void brk1_body(Dev<R> d, Geo g, Prm<R> p, R DT, const Blk &B) {
+  const Tile tb = xcd_tile(B);
+  int i = 1 + tb.x * blockDim.x + threadIdx.x;
+  int j = 1 + tb.y * blockDim.y + threadIdx.y;
+  if (i > g.M || j > g.N) return;
+  const size_t o = IX(i, j);
+  const bool ring = i >= g.Ib - 1 && i <= g.Ie + 1 && j >= g.Jb - 1 && j <= g.Je + 1;
+  brk1_cell(d, g, p, DT, i, j, o, ring, d.AGE_BREAKING[o], d.ETAT[o], d.H[o], d.Depth[o], d.Eta[o]);
 }
 template <class R>
 __global__ void k_brk1(Dev<R> d, Geo g, Prm<R> p, R DT) {
@@ -3027,7 +3123,7 @@ __global__ void k_brk1(Dev<R> d, Geo g, Prm<R> p, R DT) {
 }
 
 template <class R>
-__device__ __forceinline__ void brk2_body(Dev<R> d, Geo g, Prm<R> p, R DT, const Blk &B) {
+__device__ __forceinline__ void brk2_body(const Dev<R> &d, const Geo &g, const Prm<R> &p, R DT, const Blk &B) {
   __shared__ int changed;
   const int n = *d.cand_n;
   if (n == 0) return;
@@ -3064,7 +3160,7 @@ __device__ __forceinline__ void brk2_body(Dev<R> d, Geo g, Prm<R> p, R DT, const
     const R *ci = d.cinf + 8 * (size_t)k;
     BrkIn<R> b;
     b.et = ci[4]; b.t2 = ci[5]; b.t3 = ci[6];
-    d.nu_break[o] = brk_nu(d, g, p, b, o, i, j, d.AGEn[o]);
+    d.nu_break[o] = brk_nu(p, g, b, i, j, d.AGEn[o], d.Depth[o], d.EtaW[o]);
   }
   __syncthreads();
   if (threadIdx.x == 0) *d.cand_n = 0;
@@ -3119,8 +3215,347 @@ __global__ void k_mask_mul(Dev<R> d, Geo g, Prm<R> p, int sponge, int mul) {
   mask_mul_body<R>(d, g, p, sponge, mul, grid_blk());
 }
 
+// --------------------------------------------------------------------------
+// Whole steps of the production path (fw_step, fw_batch).  On small domains a
+// step's time is its launches (about 3.5 us each) and cross-stream waits
+// (about 25 us a pair), on large ones the planes each kernel reads again, so
+// what follows the line solves is one pass, k_tail, and what precedes the
+// first stage another, k_begin.  Each ghost cell is a pure function of one
+// interior cell (PHI_COLL), so the thread of that interior cell writes its
+// ghost cells too, and nothing has to wait for a fill.
+//
+// f(ti, tj, nx, ny) for every ghost cell (ti, tj) that mirrors (i, j); nx, ny:
+// across a wall normal to x, y (the sign of arrays odd in that direction)
+template <class F>
+__device__ __forceinline__ void mirrors(int i, int j, int Ib, int Ie, int Jb, int Je, F f) {
+  const int tx[3] = {i, i < Ib + 3 ? 2 * Ib - 1 - i : 0, i > Ie - 3 ? 2 * Ie + 1 - i : 0};
+  const int ty[3] = {j, j < Jb + 3 ? 2 * Jb - 1 - j : 0, j > Je - 3 ? 2 * Je + 1 - j : 0};
+#pragma unroll
+  for (int b = 0; b < 3; b++)
+#pragma unroll
+    for (int a = 0; a < 3; a++)
+      if (a + b > 0 && tx[a] > 0 && ty[b] > 0) f(tx[a], ty[b], a > 0, b > 0);
+}
+// ghost fill of the fluxes P, Q (bc.F:631-1272 on face arrays) by the threads
+// of the interior faces
+template <class R>
+__device__ __forceinline__ void mirror_faces(const Dev<R> &d, const Geo &g, int i, int j) {
+  if (i >= g.Ib && i <= g.Ie + 1 && j >= g.Jb && j <= g.Je &&
+      (i < g.Ib + 3 || i > g.Ie - 2 || j < g.Jb + 3 || j > g.Je - 3)) {
+    const R v = d.P[IX(i, j)];
+    mirrors(i, j, g.Ib, g.Ie + 1, g.Jb, g.Je, [&](int a, int b, bool, bool) { d.P[IX(a, b)] = v; });
+  }
+  if (i >= g.Ib && i <= g.Ie && j >= g.Jb && j <= g.Je + 1 &&
+      (i < g.Ib + 3 || i > g.Ie - 3 || j < g.Jb + 3 || j > g.Je - 2)) {
+    const R v = d.Q[IX(i, j)];
+    mirrors(i, j, g.Ib, g.Ie, g.Jb, g.Je + 1, [&](int a, int b, bool, bool) { d.Q[IX(a, b)] = v; });
+  }
+}
+// block minimum / maximum of one value per thread (64 x up to 8 threads),
+// left in out[block] by thread 0
+template <class R, bool MAX>
+__device__ __forceinline__ void block_extreme(R m, R *out) {
+  __shared__ R sm[8];
+  const int lane = threadIdx.x, w = threadIdx.y;
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) {
+    const R v = __shfl_xor(m, s);
+    m = MAX ? rmax(m, v) : rmin(m, v);
+  }
+  if (lane == 0) sm[w] = m;
+  __syncthreads();
+  if (lane == 0 && w == 0) {
+    for (int k = 1; k < (int)blockDim.y; k++) m = MAX ? rmax(m, sm[k]) : rmin(m, sm[k]);
+    *out = m;
+  }
+}
+
+// Start of a step of a non-periodic domain in one pass: Eta0, Ubar0, Vbar0 :=
+// Eta, Ubar, Vbar (main.F:295-297), EXCHANGE (bc.F:426-529), the partial
+// minima of ESTIMATE_DT over all cells, ghosts included (misc.F:216-296), and
+// U0, V0 := U, V (main.F:331-332).  HBM-bound: 12 planes, 201 MB at 2048 x 2048
+// FP32, in 45 us (4.5 TB/s); the copy, fill, mask multiply and reduction it
+// replaces took 62 and read U, V, MASK, H again.
+template <class R>
+__device__ __forceinline__ void begin_body(const Dev<R> &d, const Geo &g, const Prm<R> &p, const Blk &B) {
+  const int i = 1 + B.x * 64 + threadIdx.x;
+  const int j = 1 + B.y * blockDim.y + threadIdx.y;
+  R t3 = Lit<R>::large();
+  if (i <= g.M && j <= g.N) {
+    const size_t o = IX(i, j);
+    const R ub = d.Ubar[o], vb = d.Vbar[o];
+    if (i >= g.Ib && i <= g.Ie && j >= g.Jb && j <= g.Je) {
+      const R eta = d.Eta[o], u0 = d.U[o], v0 = d.V[o], h = d.H[o];
+      const int mk = d.MASK[o];
+      auto cell_dt = [&](R u, R v, R hc) {
+        const R c = dsqrt(GRAV * rmax(hc, p.MDF));
+        R t1 = dabs(u) + c;
+        R t2 = (t1 < SMALL) ? ddiv(p.DX, SMALL) : ddiv(p.DX, t1);
+        if (t2 < t3) t3 = t2;
+        t1 = dabs(v) + c;
+        t2 = (t1 < SMALL) ? ddiv(p.DY, SMALL) : ddiv(p.DY, t1);
+        if (t2 < t3) t3 = t2;
+      };
+      const bool mul = mk != 1;  // x*1 leaves every bit of x
+      const R m = (R)mk;
+      const R u = mul ? u0 * m : u0, v = mul ? v0 * m : v0;
+      const bool edge = i < g.Ib + 3 || i > g.Ie - 3 || j < g.Jb + 3 || j > g.Je - 3;
+      d.Eta0[o] = eta;
+      d.U0[o] = u;
+      d.V0[o] = v;
+      cell_dt(u, v, h);
+      if (mul || edge) {
+        const R hu0 = d.HU[o], hv0 = d.HV[o];
+        const R hu = mul ? hu0 * m : hu0, hv = mul ? hv0 * m : hv0;
+        if (!bits_equal(u, u0)) d.U[o] = u;
+        if (!bits_equal(v, v0)) d.V[o] = v;
+        if (!bits_equal(hu, hu0)) d.HU[o] = hu;
+        if (!bits_equal(hv, hv0)) d.HV[o] = hv;
+        if (edge) {
+          const bool brk = p.VISC_BRK;
+          const R age = brk ? d.AGE_BREAKING[o] : (R)0, nu = brk ? d.nu_break[o] : (R)0;
+          mirrors(i, j, g.Ib, g.Ie, g.Jb, g.Je, [&](int a, int b, bool nx, bool ny) {
+            const size_t q = IX(a, b);
+            const R gu = nx ? -u : u, gv = ny ? -v : v;
+            d.Eta0[q] = d.Eta[q];
+            d.Eta[q] = eta;
+            d.MASK[q] = mk;
+            d.U[q] = gu;
+            d.V[q] = gv;
+            d.HU[q] = nx ? -hu : hu;
+            d.HV[q] = ny ? -hv : hv;
+            d.U0[q] = gu;
+            d.V0[q] = gv;
+            if (brk) {
+              d.AGE_BREAKING[q] = age;
+              d.nu_break[q] = nu;
+            }
+            cell_dt(gu, gv, d.H[q]);
+          });
+        }
+      }
+    }
+    if (p.VISC_BRK || p.DIFF_SPONGE) mirror_faces(d, g, i, j);
+    d.Ubar0[o] = ub;
+    d.Vbar0[o] = vb;
+  }
+  block_extreme<R, false>(t3, d.red + (size_t)B.y * B.gx + B.x);
+}
+template <class R>
+__global__ void __launch_bounds__(256) k_begin(Dev<R> d, Geo g, Prm<R> p) {
+  begin_body<R>(d, g, p, grid_blk());
+}
+
+// What follows the line solves in a stage, in one pass: UPDATE_MASK
+// (mask_body), the first pass of WAVE_BREAKING (brk1_body), the velocity tail
+// (uv_final_body) and, with FILL (non-periodic), EXCHANGE and SPONGE_DAMPING.
+// Eta is read around the cell from EtaW, where the RK update left it, and
+// written to Eta, so that no cell reads what another one writes; MASK and the
+// ages are double-buffered.  The ages' and viscosities' ghost cells are left
+// to k_brk2_fill, which may still change them.  With last, the block maxima
+// of |eta| (CHECK_BLOWUP) go to red.
+// HBM-bound on about 20 planes: 70 us at 2048 x 2048 FP32; in kernels of their
+// own UPDATE_MASK (93) and WAVE_BREAKING (58) beside the solve, the velocity
+// tail (23), ghost fill (6) and mask multiply (15) after it.  At 96 x 72 cells
+// the step with k_begin and k_tail takes 250 us against 390.
+template <class R, bool FILL>
+__device__ __forceinline__ void tail_body(const Dev<R> &d, const Geo &g, const Prm<R> &p, R DT, int sponge, int last,
+                                          const Blk &B) {
+  const Tile tb = xcd_tile(B);
+  const int i = 1 + tb.x * 64 + threadIdx.x;
+  const int j = 1 + tb.y * blockDim.y + threadIdx.y;
+  R emax = (R)0;
+  if (i <= g.M + 1 && j <= g.N + 1) {
+    const int lo_i = g.Ib - 2, hi_i = g.Ie + 2, lo_j = g.Jb - 2, hi_j = g.Je + 2;
+    const bool cell = i <= g.M && j <= g.N;
+    const bool inner = i >= g.Ib && i <= g.Ie && j >= g.Jb && j <= g.Je;
+    const bool ring = i >= g.Ib - 1 && i <= g.Ie + 1 && j >= g.Jb - 1 && j <= g.Je + 1;
+    const bool brk = p.SHOW_BRK;
+    // every load first, from indices clamped into the array
+    const int ic = i <= g.M ? i : g.M, jc = j <= g.N ? j : g.N;
+    const int im = ic > 1 ? ic - 1 : 1, ip = ic < g.M ? ic + 1 : g.M;
+    const int jm = jc > 1 ? jc - 1 : 1, jp = jc < g.N ? jc + 1 : g.N;
+    const int im1 = i - 1 >= 1 ? i - 1 : 1, jm1 = j - 1 >= 1 ? j - 1 : 1;
+    const size_t o = IX(ic, jc);
+    const R *E = d.EtaW;
+    const int m0 = d.MASK[o], mw = d.MASK[IX(im, jc)], me = d.MASK[IX(ip, jc)];
+    const int ms = d.MASK[IX(ic, jm)], mn = d.MASK[IX(ic, jp)];
+    const int mfw = d.MASK[IX(im1, jc)], mfs = d.MASK[IX(ic, jm1)];
+    const R e0 = E[o], ew = E[IX(im, jc)], ee = E[IX(ip, jc)], es = E[IX(ic, jm)], en = E[IX(ic, jp)];
+    const R h0 = d.Depth[o], hw = d.Depth[IX(im1, jc)], hs = d.Depth[IX(ic, jm1)];
+    const int strc = d.MASK_STRUC[o], m9_old = d.MASK9[o];
+    const R u_in = d.U[o], v_in = d.V[o], h = d.H[o];
+    const R sp = FILL && sponge ? d.SPONGE[o] : (R)1;
+    const R age = (brk ? d.AGE_BREAKING : d.H)[o], et = (brk ? d.ETAT : d.H)[o];
+    // UPDATE_MASK: DepthX/DepthY at faces of dry cells (masks.F:152-161)
+    if (j <= g.N && j >= lo_j && j <= hi_j) {
+      R v;
+      bool w = false;
+      if (i - 1 >= lo_i && i - 1 <= hi_i && mfw < 1) { v = h0; w = true; }
+      if (i >= lo_i && i <= hi_i && m0 < 1) { v = hw; w = true; }
+      if (w) d.DepthX[IX(i, j)] = v;
+    }
+    if (i <= g.M && i >= lo_i && i <= hi_i) {
+      R v;
+      bool w = false;
+      if (j - 1 >= lo_j && j - 1 <= hi_j && mfs < 1) { v = h0; w = true; }
+      if (j >= lo_j && j <= hi_j && m0 < 1) { v = hs; w = true; }
+      if (w) d.DepthY[IX(i, j)] = v;
+    }
+    if (cell) {
+      // the new mask of the cell (masks.F:79-135)
+      int m = m0;
+      if (i >= lo_i && i <= hi_i && j >= lo_j && j <= hi_j && strc == 1) {
+        if (m0 < 1) {
+          if (e0 > -h0) m = 1;
+          if (mw == 1 && ew > e0) m = 1;
+          if (me == 1 && ee > e0) m = 1;
+          if (ms == 1 && es > e0) m = 1;
+          if (mn == 1 && en > e0) m = 1;
+        } else {
+          if (e0 < -h0) m = 0;
+        }
+      }
+      int m9 = 0;
+      if (ring) {
+        if (p.VISC_BRK) {
+          m9 = 1;
+        } else {
+          m9 = m * new_mask(d, g, i - 1, j) * new_mask(d, g, i + 1, j) * new_mask(d, g, i + 1, j + 1) *
+               new_mask(d, g, i, j + 1) * new_mask(d, g, i - 1, j + 1) * new_mask(d, g, i + 1, j - 1) *
+               new_mask(d, g, i, j - 1) * new_mask(d, g, i - 1, j - 1);
+          if (ddiv(dabs(e0), rmax(h0, p.MDF)) > p.SWE) m9 = 0;
+        }
+      }
+      if (m9 != m9_old) d.MASK9[o] = m9;
+      if (!FILL) d.MASKn[o] = m;
+      if (brk) brk1_cell(d, g, p, DT, i, j, o, ring, age, et, h, h0, e0);
+      if (inner) {
+        // the velocity tail with the old mask
+        R u = (R)0, v = (R)0, hu = (R)0, hv = (R)0;
+        if (m0 < 1) {
+          d.Ubar[o] = (R)0;
+          d.Vbar[o] = (R)0;
+        } else {
+          const R hm = rmax(h, p.MDF);
+          u = u_in;
+          v = v_in;
+          hu = hm * u;
+          hv = hm * v;
+          const R ut = dsqrt(u * u + v * v);
+          const R fr = dsqrt(GRAV * hm);
+          if (ddiv(ut, fr) > p.FCAP) {
+            const R th = datan2(v, u);
+            u = p.FCAP * fr * dcos(th);
+            v = p.FCAP * fr * dsin(th);
+            hu = u * hm;
+            hv = v * hm;
+          }
+        }
+        const bool disp = p.DISPERSION;
+        if (!disp) {
+          d.Ubar[o] = hu;
+          d.Vbar[o] = hv;
+        }
+        if constexpr (!FILL) {
+          if (!bits_equal(u, u_in)) d.U[o] = u;
+          if (!bits_equal(v, v_in)) d.V[o] = v;
+          d.HU[o] = hu;
+          d.HV[o] = hv;
+        } else {
+          // EXCHANGE: U, V, HU, HV times the new mask, Eta, U, V over the
+          // sponge (bc.F:491-494, sponge.F:52-66), here and in the ghost
+          // cells that mirror this one (each with its own SPONGE)
+          const R mr = (R)m;
+          const bool mul = m != 1;
+          const R um = mul ? u * mr : u, vm = mul ? v * mr : v;
+          const R hum = mul ? hu * mr : hu, hvm = mul ? hv * mr : hv;
+          auto damp = [&](R x, R s) { return s == (R)1 ? x : ddiv(x, s); };
+          const R uf = damp(um, sp), vf = damp(vm, sp);
+          const R ef = mr > (R)0 ? damp(e0, sp) : e0;
+          const bool edge = i < g.Ib + 3 || i > g.Ie - 3 || j < g.Jb + 3 || j > g.Je - 3;
+          if (edge)
+            mirrors(i, j, g.Ib, g.Ie, g.Jb, g.Je, [&](int a, int b, bool nx, bool ny) {
+              const size_t q = IX(a, b);
+              const R s = sponge ? d.SPONGE[q] : (R)1;
+              if (!disp) {
+                d.Ubar[q] = d.HU[q];
+                d.Vbar[q] = d.HV[q];
+              }
+              d.Eta[q] = mr > (R)0 ? damp(e0, s) : e0;
+              d.U[q] = damp(nx ? -um : um, s);
+              d.V[q] = damp(ny ? -vm : vm, s);
+              d.HU[q] = nx ? -hum : hum;
+              d.HV[q] = ny ? -hvm : hvm;
+              d.MASKn[q] = m;
+            });
+          d.Eta[o] = ef;
+          if (!bits_equal(uf, u_in)) d.U[o] = uf;
+          if (!bits_equal(vf, v_in)) d.V[o] = vf;
+          d.HU[o] = hum;
+          d.HV[o] = hvm;
+          d.MASKn[o] = m;
+          emax = dabs(ef);
+          if (!(emax > (R)0)) emax = (R)0;  // (a NaN counts as 0, as in the comparison of k_maxeta_partial)
+        }
+      }
+      if (FILL && (p.VISC_BRK || p.DIFF_SPONGE)) mirror_faces(d, g, i, j);
+    }
+  }
+  if (FILL && last) block_extreme<R, true>(emax, d.red + (size_t)tb.y * B.gx + tb.x);
+}
+template <class R, bool FILL>
+__global__ void __launch_bounds__(256) k_tail(Dev<R> d, Geo g, Prm<R> p, R DT, int sponge, int last) {
+  tail_body<R, FILL>(d, g, p, DT, sponge, last, grid_blk());
+}
+
+// The rest of WAVE_BREAKING by one workgroup: the candidates' fixed point
+// (brk2_body), then the ghost cells of the new ages and viscosities
+// (EXCHANGE; non-periodic).  With pub, the maximum of the nblk block maxima
+// and the breaking flag go to the host.
+template <class R>
+__device__ __forceinline__ void brk2_fill_body(const Dev<R> &d, const Geo &g, const Prm<R> &p, R DT, const Blk &B) {
+  if (p.SHOW_BRK) brk2_body<R>(d, g, p, DT, B);
+  if (!p.VISC_BRK) return;
+  __syncthreads();
+  const HaloSpec s = halo_spec(g, 0);
+  const int cnt = 6 * g.M + 6 * (g.Je - g.Jb + 1);
+  R *arr[2] = {p.SHOW_BRK ? d.AGEn : d.AGE_BREAKING, d.nu_break};
+  constexpr int K = 4;  // ghost cells of a thread in flight together
+  for (int t0 = threadIdx.x; t0 < cnt; t0 += K * blockDim.x) {
+    size_t dst[K];
+    R va[K], vn[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      int i, j;
+      const int t = min(t0 + k * (int)blockDim.x, cnt - 1);
+      halo_pos(s, t, 0, i, j);
+      const int si = i < g.Ib ? 2 * g.Ib - 1 - i : (i > g.Ie ? 2 * g.Ie + 1 - i : i);
+      const int sj = j < g.Jb ? 2 * g.Jb - 1 - j : (j > g.Je ? 2 * g.Je + 1 - j : j);
+      dst[k] = IX(i, j);
+      va[k] = arr[0][IX(si, sj)];
+      vn[k] = arr[1][IX(si, sj)];
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      if (t0 + k * (int)blockDim.x >= cnt) continue;
+      arr[0][dst[k]] = va[k];
+      arr[1][dst[k]] = vn[k];
+    }
+  }
+}
+template <class R>
+__global__ void __launch_bounds__(1024) k_brk2_fill(Dev<R> d, Geo g, Prm<R> p, R DT, int nblk, Pub *pub, unsigned seq) {
+  brk2_fill_body<R>(d, g, p, DT, grid_blk());
+  if (!pub) return;
+  __threadfence_system();  // the ghost cells, before the host is told
+  __syncthreads();
+  const R m = extreme1024<R, true>(d.red, nblk, (R)0);
+  if (threadIdx.x == 0) publish(pub, (double)m, d.flags[0], seq);
+}
+
 // FP64 budget (mass, energy, extrema) over the interior.
-// FP64 budget terms of one wet interior cell (fw_stats): total depth,
+// Terms of one wet interior cell (fw_stats): total depth,
 // volume and energy formed in FP64
 struct StatAcc {
   double mass = 0, en = 0, mx = -1e300, mn = 1e300, mu = 0, mv = 0, wet = 0;

@@ -3,6 +3,8 @@
 // per-routine entry points and the whole-step driver behind include/fwgpu.h.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -101,6 +103,11 @@ int collect_profile(fw_ctx *c) {
 
 inline dim3 grid2(int nx, int ny, dim3 b) { return dim3((nx + b.x - 1) / b.x, (ny + b.y - 1) / b.y); }
 const dim3 kB2(64, 4);
+// workgroups of the largest kernel that leaves one partial per workgroup
+inline size_t red_blocks(const Geo &g) {
+  const dim3 n = grid2(g.M + 1, g.N + 1, kB2);
+  return (size_t)n.x * n.y;
+}
 // taller tiles for kernels reading j-1/j+1 neighbours: fewer rows fetched
 // twice by vertically adjacent workgroups
 const dim3 kBT(64, 8);
@@ -185,7 +192,7 @@ int alloc_state(fw_ctx *c) {
 #undef FW_ALLOC
   void **rs[] = {(void **)&d.AGEn, (void **)&d.xa, (void **)&d.xc, (void **)&d.xd, (void **)&d.ya,
                  (void **)&d.yc,   (void **)&d.yd, (void **)&d.c1, (void **)&d.y1, (void **)&d.y2,
-                 (void **)&d.sumU, (void **)&d.sumV};
+                 (void **)&d.sumU, (void **)&d.sumV, (void **)&d.eta2};
   for (void **q : rs)
     if ((rc = get(pe * sizeof(R), q)) != FW_OK) return rc;
   void **is[] = {(void **)&d.MASK, (void **)&d.MASK9, (void **)&d.MASK_STRUC, (void **)&d.MASKn, (void **)&d.cand};
@@ -195,7 +202,9 @@ int alloc_state(fw_ctx *c) {
   if ((rc = get(64 * sizeof(int), (void **)&d.cand_n)) != FW_OK) return rc;
   d.flags = d.cand_n + 16;
   d.fc_n = d.cand_n + 32;  // the Froude-cap list itself is allocated with FW_OPT_HOST_MATH
-  if ((rc = get(kRedBlocks * sizeof(R), (void **)&d.red)) != FW_OK) return rc;
+  d.EtaW = d.Eta;
+  const size_t nred = std::max<size_t>(kRedBlocks, red_blocks(c->g));
+  if ((rc = get(nred * sizeof(R), (void **)&d.red)) != FW_OK) return rc;
   if ((rc = get(kRedBlocks * 7 * sizeof(double), (void **)&d.red64)) != FW_OK) return rc;
   if ((rc = get(64 * sizeof(double), &c->scal)) != FW_OK) return rc;
   const fw_config &f = c->cfg;
@@ -214,7 +223,10 @@ int alloc_state(fw_ctx *c) {
   size_t stage_elems = (size_t)(N + 8) > (size_t)(2 * nfreq + 8) ? (size_t)(N + 8) : (size_t)(2 * nfreq + 8);
   if ((rc = get(stage_elems * sizeof(R), (void **)&d.wk_stage)) != FW_OK) return rc;
   c->slot_bytes = (stage_elems * sizeof(R) + 255) & ~(size_t)255;
-  HIPCHK(c, hipHostMalloc((void **)&c->pinned, c->slot_bytes * kStageSlots + 4096));
+  HIPCHK(c, hipHostMalloc((void **)&c->pinned, c->slot_bytes * (kStageSlots + 1) + 4096));
+  HIPCHK(c, hipHostMalloc((void **)&c->pub, 2 * sizeof(Pub), hipHostMallocMapped | hipHostMallocCoherent));
+  HIPCHK(c, hipHostGetDevicePointer((void **)&c->pub_dev, c->pub, 0));
+  memset(c->pub, 0, 2 * sizeof(Pub));
   for (int k = 0; k < kStageSlots; k++) HIPCHK(c, hipEventCreateWithFlags(&c->slot_ev[k], hipEventDisableTiming));
   // MASK_STRUC defaults to 1 (no structures); MASK9 / MASK to 1 until uploaded
   return FW_OK;
@@ -290,21 +302,34 @@ int stage_wavemaker(fw_ctx *c, R &AA) {
   return FW_OK;
 }
 
+// the factors of a whole step, formed once (TIME stays the same over its
+// stages); the pinned slot is free again when the step has ended
+template <class R>
+int step_wavemaker(fw_ctx *c, R &AA) {
+  AA = (R)0;
+  if (c->cfg.wavemaker == FW_WK_NONE) return FW_OK;
+  int rc = prepare_wavemaker<R>(c);
+  if (rc) return rc;
+  R *h = (R *)(c->pinned + (size_t)kStageSlots * c->slot_bytes + 4096);
+  size_t n = 0;
+  if ((rc = wavemaker_factors<R>(c, (R)c->time, AA, h, &n))) return rc;
+  if (n) HIPCHK(c, hipMemcpyAsync(c->dev<R>().wk_stage, h, n * sizeof(R), hipMemcpyHostToDevice, c->stream));
+  return FW_OK;
+}
+
 // ---- routines ---------------------------------------------------------------
 template <class R>
 void halo_exchange_list(fw_ctx *c, HaloList &L, HaloList &Lf) {
   const Geo &g = c->g;
-  int cnt = 6 * (g.M + 1) + 6 * (g.N + 1) + 64;
+  const int cnt = 6 * (g.M + 1) + 6 * (g.N + 1) + 64;
   // grid rows = arrays of the list
-  dim3 b(256);
-  auto grid = [&](const HaloList &l) { return dim3((cnt + 255) / 256, l.n); };
+  const dim3 b(256), gr((cnt + 255) / 256, L.n + Lf.n);
+  if (!gr.y) return;
   if (!c->cfg.PERIODIC) {
     for (int k = 0; k < Lf.n; k++) L.a[L.n++] = Lf.a[k];
-    if (L.n) launch(c, "halo", k_halo<R>, grid(L), b, L, g, 0);
+    launch(c, "halo", k_halo<R>, gr, b, L, g, 0);
   } else {
-    if (L.n) launch(c, "halo", k_halo<R>, grid(L), b, L, g, 1);
-    if (L.n) launch(c, "halo", k_halo<R>, grid(L), b, L, g, 2);
-    if (Lf.n) launch(c, "halo", k_halo<R>, grid(Lf), b, Lf, g, 0);
+    launch(c, "halo", k_halo_per<R>, gr, b, L, Lf, g);
   }
 }
 
@@ -383,9 +408,10 @@ bool disp_one_pass(fw_ctx *c) {
 }
 
 // in_step: called by fw_step, whose RK update forms the cross derivatives
-// (the per-routine ESTIMATE_HUV reads them from the arrays)
+// (the per-routine ESTIMATE_HUV reads them from the arrays); dtp: DT on the
+// device, where the host does not have it yet
 template <class R>
-int do_dispersion(fw_ctx *c, bool in_step = false) {
+int do_dispersion(fw_ctx *c, bool in_step = false, const R *dtp = nullptr) {
   Dev<R> &d = c->dev<R>();
   const Geo &g = c->g;
   if (disp_one_pass<R>(c)) {
@@ -394,15 +420,15 @@ int do_dispersion(fw_ctx *c, bool in_step = false) {
     Prm<R> p = c->prm<R>();
     p.xd_in_huv = in_step ? 1 : 0;
     if (spacing_pow2<R>(c))
-      launch(c, "disp", k_disp_fused<R, true>, gr, b, d, g, p, (R)c->dt);
+      launch(c, "disp", k_disp_fused<R, true>, gr, b, d, g, p, (R)c->dt, dtp);
     else
-      launch(c, "disp", k_disp_fused<R, false>, gr, b, d, g, p, (R)c->dt);
+      launch(c, "disp", k_disp_fused<R, false>, gr, b, d, g, p, (R)c->dt, dtp);
     return FW_OK;
   }
   if (spacing_pow2<R>(c))
-    launch(c, "disp_deriv", k_disp_deriv<R, true>, grid2(g.M, g.N, kBT), kBT, d, g, c->prm<R>(), (R)c->dt);
+    launch(c, "disp_deriv", k_disp_deriv<R, true>, grid2(g.M, g.N, kBT), kBT, d, g, c->prm<R>(), (R)c->dt, dtp);
   else
-    launch(c, "disp_deriv", k_disp_deriv<R, false>, grid2(g.M, g.N, kBT), kBT, d, g, c->prm<R>(), (R)c->dt);
+    launch(c, "disp_deriv", k_disp_deriv<R, false>, grid2(g.M, g.N, kBT), kBT, d, g, c->prm<R>(), (R)c->dt, dtp);
   HaloList L{}, Lf{};
   hadd(L, d.Uxx, 2); hadd(L, d.DUxx, 2); hadd(L, d.Vyy, 3); hadd(L, d.DVyy, 3);
   hadd(L, d.Uxy, 1); hadd(L, d.DUxy, 1); hadd(L, d.Vxy, 1); hadd(L, d.DVxy, 1);
@@ -418,9 +444,9 @@ int do_dispersion(fw_ctx *c, bool in_step = false) {
   }
   halo_exchange_list<R>(c, L, Lf);
   if (spacing_pow2<R>(c))
-    launch(c, "disp_terms", k_disp_terms<R, true>, grid2(g.M, g.N, kBT), kBT, d, g, c->prm<R>(), (R)c->dt);
+    launch(c, "disp_terms", k_disp_terms<R, true>, grid2(g.M, g.N, kBT), kBT, d, g, c->prm<R>(), (R)c->dt, dtp);
   else
-    launch(c, "disp_terms", k_disp_terms<R, false>, grid2(g.M, g.N, kBT), kBT, d, g, c->prm<R>(), (R)c->dt);
+    launch(c, "disp_terms", k_disp_terms<R, false>, grid2(g.M, g.N, kBT), kBT, d, g, c->prm<R>(), (R)c->dt, dtp);
   return FW_OK;
 }
 
@@ -532,37 +558,39 @@ int do_breaking(fw_ctx *c);
 template <class R>
 int do_roller(fw_ctx *c);
 
-// overlap: UPDATE_MASK and WAVE_BREAKING follow on two more streams,
-// concurrently with the line solves
+// the fused RK update of one stage with the wavemaker amplitude AA (its
+// factors are on the device)
 template <class R>
-int do_src_huv(fw_ctx *c, int istage, bool overlap) {
-  if (istage < 1 || istage > 3) return fail(c, FW_E_INVALID, "istage must be 1..3");
+void launch_src_huv(fw_ctx *c, int istage, R AA) {
   const R alpha[3] = {(R)0, (R)3 / (R)4, (R)1 / (R)3};
   const R beta[3] = {(R)1, (R)1 / (R)4, (R)2 / (R)3};
-  R AA;
-  int rc = stage_wavemaker<R>(c, AA);
-  if (rc) return rc;
-  Dev<R> &d = c->dev<R>();
   const Geo &g = c->g;
   // with the one-pass dispersion of fw_step the update forms the cross
   // derivatives itself
   const bool xd = c->cfg.DISPERSION && disp_one_pass<R>(c);
+  auto go = [&](auto k) {
+    launch(c, "src_huv", k, grid2(g.M, g.N, kBH), kBH, c->dev<R>(), g, c->prm<R>(), alpha[istage - 1],
+           beta[istage - 1], (R)c->dt, AA);
+  };
   if (spacing_pow2<R>(c)) {
-    if (xd)
-      launch(c, "src_huv", k_huv<R, true, true, true>, grid2(g.M, g.N, kBH), kBH, d, g, c->prm<R>(),
-             alpha[istage - 1], beta[istage - 1], (R)c->dt, AA);
-    else
-      launch(c, "src_huv", k_huv<R, true, true>, grid2(g.M, g.N, kBH), kBH, d, g, c->prm<R>(), alpha[istage - 1],
-             beta[istage - 1], (R)c->dt, AA);
+    if (xd) go(k_huv<R, true, true, true>);
+    else go(k_huv<R, true, true>);
   } else {
-    if (xd)
-      launch(c, "src_huv", k_huv<R, true, false, true>, grid2(g.M, g.N, kBH), kBH, d, g, c->prm<R>(),
-             alpha[istage - 1], beta[istage - 1], (R)c->dt, AA);
-    else
-      launch(c, "src_huv", k_huv<R, true, false>, grid2(g.M, g.N, kBH), kBH, d, g, c->prm<R>(), alpha[istage - 1],
-             beta[istage - 1], (R)c->dt, AA);
+    if (xd) go(k_huv<R, true, false, true>);
+    else go(k_huv<R, true, false>);
   }
-  if (!overlap) return do_solve<R>(c, true);
+}
+
+// A stage from SourceTerms to WAVE_BREAKING with its routines' own kernels
+// (every intermediate kept, or the Froude cap left to the host): UPDATE_MASK
+// and WAVE_BREAKING follow the RK update on two more streams, concurrently
+// with the line solves.
+template <class R>
+int do_src_huv(fw_ctx *c, int istage) {
+  R AA;
+  int rc = stage_wavemaker<R>(c, AA);
+  if (rc) return rc;
+  launch_src_huv<R>(c, istage, AA);
   // UPDATE_MASK reads Eta, Depth, H and the old MASK and writes MASKn,
   // MASK9, DepthX/Y; WAVE_BREAKING reads Eta, Depth, H, the dispersion
   // slopes and AGE and writes AGEn, nu_break; the line solves and the
@@ -599,10 +627,9 @@ int do_src_huv(fw_ctx *c, int istage, bool overlap) {
 template <class R>
 int froude_cap_on_host(fw_ctx *c);
 
-// line solves and the final velocities (GET_Eta_U_V_HU_HV after the
-// coefficient assembly); fac: c' has been formed by k_trid_fac (fw_step)
+// line solves; fac: c' has been formed by k_trid_fac (fw_step)
 template <class R>
-int do_solve(fw_ctx *c, bool fac) {
+int do_lines(fw_ctx *c, bool fac) {
   Dev<R> &d = c->dev<R>();
   const Geo &g = c->g;
   if (c->cfg.DISPERSION && !fac) {
@@ -626,9 +653,20 @@ int do_solve(fw_ctx *c, bool fac) {
     }
     HIPCHK(c, hipGetLastError());  // (the only launch with more than 64 KB of dynamic LDS)
   }
+  return FW_OK;
+}
+
+// line solves and the final velocities (GET_Eta_U_V_HU_HV after the
+// coefficient assembly)
+template <class R>
+int do_solve(fw_ctx *c, bool fac) {
+  int rc = do_lines<R>(c, fac);
+  if (rc) return rc;
+  Dev<R> &d = c->dev<R>();
+  const Geo &g = c->g;
   launch(c, "uv_final", k_uv_final<R>, grid2(g.M, g.N, kB2), kB2, d, g, c->prm<R>());
   if (c->prm<R>().host_math) {
-    int rc = froude_cap_on_host<R>(c);
+    rc = froude_cap_on_host<R>(c);
     if (rc) return rc;
   }
   if (!c->cfg.DISPERSION) {
@@ -715,8 +753,18 @@ int read_break_flag(fw_ctx *c, void *flags) {
   return fail(c, FW_E_BREAK_ITER, "breaking-age propagation did not settle");
 }
 
+// after a step: the breaking flag, then CHECK_BLOWUP
+int check_step(fw_ctx *c, double max_eta) {
+  if (!(max_eta > c->cfg.EtaBlowVal)) return FW_OK;
+  char buf[128];
+  snprintf(buf, sizeof buf, "blow-up: max|eta|=%g > EtaBlowVal=%g at time %g", max_eta, c->cfg.EtaBlowVal, c->time);
+  return fail(c, FW_E_BLOWUP, buf);
+}
+
+// whole steps with the routines' own kernels: every intermediate kept, or
+// the Froude cap left to the host
 template <class R>
-int do_step(fw_ctx *c, int nsteps) {
+int do_step_routines(fw_ctx *c, int nsteps) {
   Dev<R> &d = c->dev<R>();
   const fw_config &f = c->cfg;
   const size_t pe = plane_elems(c->g);
@@ -732,20 +780,128 @@ int do_step(fw_ctx *c, int nsteps) {
       if (f.DISPERSION && (rc = do_dispersion<R>(c, true))) return rc;
       if ((rc = do_fluxes<R>(c))) return rc;
       if (fac && (rc = join_factor<R>(c))) return rc;
-      if ((rc = do_src_huv<R>(c, st, true))) return rc;
+      if ((rc = do_src_huv<R>(c, st))) return rc;
       if ((rc = do_exchange<R>(c, f.DIRECT_SPONGE != 0))) return rc;
     }
     double m;
     if ((rc = do_max_eta<R>(c, &m))) return rc;
     if ((rc = read_break_flag(c, (void *)d.flags))) return rc;
-    if (m > f.EtaBlowVal) {
-      char buf[128];
-      snprintf(buf, sizeof buf, "blow-up: max|eta|=%g > EtaBlowVal=%g at time %g", m, f.EtaBlowVal, c->time);
-      return fail(c, FW_E_BLOWUP, buf);
+    if ((rc = check_step(c, m))) return rc;
+  }
+  return FW_OK;
+}
+
+// The host's side of publish(): spins until the kernel has stored seq.  A wait
+// longer than 20 ms goes to the stream, whose error it then reports.
+int wait_pub(fw_ctx *c, const Pub *p, unsigned seq) {
+  const auto t0 = std::chrono::steady_clock::now();
+  while (__atomic_load_n(&p->seq, __ATOMIC_ACQUIRE) != seq) {
+    for (int k = 0; k < 32; k++) __builtin_ia32_pause();
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20)) {
+      HIPCHK(c, hipStreamSynchronize(c->stream));
+      if (__atomic_load_n(&p->seq, __ATOMIC_ACQUIRE) != seq) return fail(c, FW_E_HIP, "a step kernel did not finish");
     }
   }
-  if (c->prof) return collect_profile(c);
   return FW_OK;
+}
+
+// Whole steps of the production path.  One stream: k_begin and k_dt_pub, then
+// per stage the dispersion, the fluxes, the RK update, the line solves and
+// k_tail.  The first stage's dispersion and fluxes are queued before the host
+// has the new DT (the dispersion reads it on the device); the wavemaker
+// factors, functions of TIME only, are formed once per step.
+template <class R>
+int do_step_prod(fw_ctx *c, int nsteps) {
+  Dev<R> &d = c->dev<R>();
+  const fw_config &f = c->cfg;
+  const Geo &g = c->g;
+  const Prm<R> &p = c->prm<R>();
+  const bool per = f.PERIODIC, sponge = f.DIRECT_SPONGE;
+  const dim3 gb = grid2(g.M, g.N, kB2), gt = grid2(g.M + 1, g.N + 1, kB2);
+  // the breaking ages' ghost cells by the one workgroup of k_brk2_fill, or, on
+  // a longer boundary, by a launch of their own (96 x 72: 5.6 us against 4 + 4;
+  // 777 x 601: 11.5 against 4 + 4; 2048 x 2048: 39 against 5 + 5)
+  const bool one_fill = 6 * (g.M + g.N) <= 4096;
+  struct EtaW {  // the RK update leaves Eta in a plane of its own
+    Dev<R> &d;
+    EtaW(Dev<R> &d_, bool own) : d(d_) { if (own) d.EtaW = d.eta2; }
+    ~EtaW() { d.EtaW = d.Eta; }
+  } guard(d, !per);
+  int rc = FW_OK;
+  for (int s = 0; s < nsteps; s++) {
+    const unsigned seq = ++c->pub_seq;
+    int nblk = (int)(gb.x * gb.y);
+    if (!per) {
+      launch(c, "begin", k_begin<R>, gb, kB2, d, g, p);
+    } else {
+      launch(c, "copy3", k_copy3<R>, dim3(2048), dim3(256), d.Eta0, (const R *)d.Eta, d.Ubar0, (const R *)d.Ubar,
+             d.Vbar0, (const R *)d.Vbar, plane_elems(g));
+      if ((rc = do_exchange<R>(c, false))) return rc;
+      nblk = (int)std::min<long>(kRedBlocks, ((long)g.M * g.N + 255) / 256);
+      launch(c, "dt_partial", k_dt_partial<R>, dim3(nblk), dim3(256), d, g, p, 1);
+    }
+    launch(c, "dt_final", k_dt_pub<R>, dim3(1), dim3(1024), d, p, nblk, (R *)c->scal, c->pub_dev, seq);
+    R AA = (R)0;
+    for (int st = 1; st <= 3; st++) {
+      const bool fac = f.DISPERSION && (3 * s + st <= 2 || !trid_fixed(p));
+      if (fac && (rc = fork_factor<R>(c))) return rc;
+      if (f.DISPERSION && (rc = do_dispersion<R>(c, true, st == 1 ? (const R *)c->scal : nullptr))) return rc;
+      if ((rc = do_fluxes<R>(c))) return rc;
+      if (st == 1) {
+        if ((rc = wait_pub(c, c->pub, seq))) return rc;
+        const R dt = (R)c->pub[0].val;
+        c->dt = (double)dt;
+        c->time = (double)((R)c->time + dt);
+        if ((rc = step_wavemaker<R>(c, AA))) return rc;
+      }
+      if (fac && (rc = join_factor<R>(c))) return rc;
+      launch_src_huv<R>(c, st, AA);
+      if ((rc = do_lines<R>(c, true))) return rc;
+      const bool last = st == 3;
+      Pub *pub = last ? c->pub_dev + 1 : nullptr;
+      if (!per) {
+        launch(c, "tail", k_tail<R, true>, gt, kB2, d, g, p, (R)c->dt, sponge ? 1 : 0, last ? 1 : 0);
+        if (one_fill) {
+          if (last || p.SHOW_BRK || p.VISC_BRK)
+            launch(c, "brk2", k_brk2_fill<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt, (int)(gt.x * gt.y), pub, seq);
+        } else {
+          if (p.SHOW_BRK) launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt);
+          HaloList L{}, Lf{};
+          if (p.VISC_BRK) {
+            hadd(L, p.SHOW_BRK ? d.AGEn : d.AGE_BREAKING, 1);
+            hadd(L, d.nu_break, 1);
+          }
+          halo_exchange_list<R>(c, L, Lf);
+          if (last) launch(c, "max_final", k_max_pub<R>, dim3(1), dim3(1024), d, (int)(gt.x * gt.y), pub, seq);
+        }
+      } else {
+        launch(c, "tail", k_tail<R, false>, gt, kB2, d, g, p, (R)c->dt, 0, 0);
+        if (!f.DISPERSION) launch(c, "ubar_hu", k_ubar_from_hu<R>, dim3(1024), dim3(256), d, plane_elems(g));
+        if (p.SHOW_BRK) launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt);
+      }
+      std::swap(d.MASK, d.MASKn);
+      if (p.SHOW_BRK) std::swap(d.AGE_BREAKING, d.AGEn);
+      if (per && (rc = do_exchange<R>(c, sponge))) return rc;
+    }
+    if (per) {
+      launch(c, "maxeta", k_maxeta_partial<R>, dim3(256), dim3(256), d, g);
+      launch(c, "max_final", k_max_pub<R>, dim3(1), dim3(1024), d, 256, c->pub_dev + 1, seq);
+    }
+    if ((rc = wait_pub(c, c->pub + 1, seq))) return rc;
+    if (c->pub[1].flag && (rc = read_break_flag(c, (void *)d.flags))) return rc;
+    if ((rc = check_step(c, c->pub[1].val))) break;
+  }
+  // (the last kernel has told the host its result, but may not have ended)
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  return rc;
+}
+
+template <class R>
+int do_step(fw_ctx *c, int nsteps) {
+  const Prm<R> &p = c->prm<R>();
+  const int rc = p.full_state || p.host_math ? do_step_routines<R>(c, nsteps) : do_step_prod<R>(c, nsteps);
+  if (rc) return rc;
+  return c->prof ? collect_profile(c) : FW_OK;
 }
 
 template <class R>
@@ -912,6 +1068,7 @@ int fw_destroy(fw_ctx *c) {
     if (c->slot_ev[k]) (void)hipEventDestroy(c->slot_ev[k]);
   for (void *p : c->allocs) (void)hipFree(p);
   if (c->pinned) (void)hipHostFree(c->pinned);
+  if (c->pub) (void)hipHostFree(c->pub);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
   if (c->ev_fac) (void)hipEventDestroy(c->ev_fac);
@@ -1084,7 +1241,7 @@ int fw_save_stage0(fw_ctx *c, int which) {
   }
   return FW_OK;
 }
-int fw_cal_dispersion(fw_ctx *c) { ENTRY(c, DISPATCH(c, do_dispersion)(c, false)); }
+int fw_cal_dispersion(fw_ctx *c) { ENTRY(c, c->rb == 8 ? do_dispersion<double>(c) : do_dispersion<float>(c)); }
 int fw_fluxes(fw_ctx *c) { ENTRY(c, DISPATCH(c, do_fluxes)(c)); }
 int fw_source_terms(fw_ctx *c) { ENTRY(c, DISPATCH(c, do_sources)(c)); }
 int fw_estimate_huv(fw_ctx *c, int istage) { ENTRY(c, DISPATCH(c, do_huv)(c, istage)); }
