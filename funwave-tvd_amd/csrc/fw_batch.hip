@@ -520,7 +520,7 @@ int build_queues(fw_batch *b) {
   if (b->rb == 4) {  // columns marched in strips of 4 faces, 64 x 4 threads
     if ((rc = make_tiles(b, "flux_y", dim3(64, 4), 64, 16, M_, [](const Geo &g) { return g.N + 1; }))) return rc;
   } else {  // the LDS tile
-    constexpr int FY = FluxYTile<FluxYK<double>::K>::faces;
+    constexpr int FY = FluxYTile<1>::faces;
     if ((rc = make_tiles(b, "flux_y", dim3(64, kFluxYThreadRows), 64, FY, M_, [](const Geo &g) { return g.N + 1; })))
       return rc;
   }
@@ -621,8 +621,8 @@ int rec_step(fw_batch *b, int p0, bool first) {
       if (b->disp) bl<R>(b, s, "flux_y", kb_flux_y_march<R, true, 4>, par, par);
       else bl<R>(b, s, "flux_y", kb_flux_y_march<R, false, 4>, par, par);
     } else {
-      if (b->disp) bl<R>(b, s, "flux_y", kb_flux_y<R, true, FluxYK<R>::K>, par, par);
-      else bl<R>(b, s, "flux_y", kb_flux_y<R, false, FluxYK<R>::K>, par, par);
+      if (b->disp) bl<R>(b, s, "flux_y", kb_flux_y<R, true, 1>, par, par);
+      else bl<R>(b, s, "flux_y", kb_flux_y<R, false, 1>, par, par);
     }
     if (fac) BCHK(b, hipStreamWaitEvent(s, b->ev_fac, 0));
     if (b->disp && !b->periodic) bl<R>(b, s, "huv", kb_huv<R, P2, true>, par, par, alpha[st], beta[st]);

@@ -1434,12 +1434,6 @@ struct FluxYTile {
   static constexpr int rows = kFluxYThreadRows * K;
   static constexpr int faces = rows - 2;
 };
-// rows per thread: 2 in FP32, 1 in FP64 (LDS holds 7 fields x rows x 64)
-template <class R>
-struct FluxYK {
-  static constexpr int K = sizeof(R) == 4 ? 2 : 1;
-};
-
 template <class R, bool DISP, int K, bool PROD = false>
 __device__ __forceinline__ void flux_y_body(Dev<R> d, Geo g, Prm<R> p, const Blk &B) {
   constexpr int NV = DISP ? 7 : 5;
@@ -1497,7 +1491,13 @@ __device__ __forceinline__ void flux_y_body(Dev<R> d, Geo g, Prm<R> p, const Blk
 #pragma unroll
     for (int q = 0; q < NV; q++) {
       R Lv, Rv;
-      pair_states(vc[k][q], D[k][q], Dn[k][q], Lv, Rv);
+      if constexpr (sizeof(R) == 4) {
+        bool mx = false;
+        pair_states_m(vc[k][q], D[k][q], Dn[k][q], Lv, Rv, mx);
+        if (mx) pair_states(vc[k][q], D[k][q], Dn[k][q], Lv, Rv);
+      } else {
+        pair_states(vc[k][q], D[k][q], Dn[k][q], Lv, Rv);
+      }
       Rf[k][q] = pok ? Rv : (R)0;
       sX[q][r][tx] = pok ? Lv : (R)0;
     }
@@ -1533,6 +1533,24 @@ __device__ __forceinline__ void flux_y_body(Dev<R> d, Geo g, Prm<R> p, const Blk
 template <class R, bool DISP, int K, bool PROD = false>
 __global__ void __launch_bounds__(64 * kFluxYThreadRows) k_flux_y(Dev<R> d, Geo g, Prm<R> p) {
   flux_y_body<R, DISP, K, PROD>(d, g, p, grid_blk());
+}
+
+// Both directions in one launch, for small grids: the first nbx workgroups
+// take 16 rows of x faces, the others a tile of y faces.  Such a grid leaves
+// most of the chip idle and its fluxes are a chain of latencies, so the two
+// run side by side, and y faces take the LDS tile (one slope and one pair per
+// thread) instead of the march's nine dependent passes.  The whole step at
+// 96 x 72 cells, FP32: 244 -> 162 us (x 9.5 + y 31 us per stage before).
+template <class R, bool DISP, bool PROD>
+__device__ __forceinline__ void flux_xy_body(const Dev<R> &d, const Geo &g, const Prm<R> &p, const Blk &B, int gxx,
+                                             int gyx) {
+  const int nbx = gxx * ((g.N + kFluxYThreadRows - 1) / kFluxYThreadRows);
+  if (B.x < nbx) flux_x_body<R, DISP, PROD>(d, g, p, Blk{B.x % gxx, B.x / gxx, gxx, 0, 0});
+  else flux_y_body<R, DISP, 1, PROD>(d, g, p, Blk{(B.x - nbx) % gyx, (B.x - nbx) / gyx, gyx, 0, 0});
+}
+template <class R, bool DISP, bool PROD>
+__global__ void __launch_bounds__(64 * kFluxYThreadRows) k_flux_xy(Dev<R> d, Geo g, Prm<R> p, int gxx, int gyx) {
+  flux_xy_body<R, DISP, PROD>(d, g, p, grid_blk(), gxx, gyx);
 }
 
 // y faces by marching: each thread walks one column through a strip of RS

@@ -450,14 +450,30 @@ int do_dispersion(fw_ctx *c, bool in_step = false, const R *dtp = nullptr) {
   return FW_OK;
 }
 
+// Cells up to which both directions' fluxes go in one launch (k_flux_xy).  The
+// step at 1400 x 1000 takes 798 us with it and 817 without, at 1600 x 1200 1050
+// and 1042 (FP32); at 800 x 600 698 and 712, at 1021 x 770 1048 and 1043 (FP64).
+template <class R>
+constexpr long kFluxOne = sizeof(R) == 4 ? 1500000 : 600000;
 // production launches (FW_OPT_FULL_STATE 0) take the flux kernels without
 // the full-state arrays' code
 template <class R, bool PROD>
 int do_fluxes_as(fw_ctx *c) {
   Dev<R> &d = c->dev<R>();
   const Geo &g = c->g;
-  const dim3 gx((g.M + 1 + kFluxXFaces - 1) / kFluxXFaces, (g.N + kB2.y - 1) / kB2.y);
   const bool disp = c->cfg.DISPERSION;
+  constexpr int FY = FluxYTile<1>::faces;
+  const int gxx = (g.M + 1 + kFluxXFaces - 1) / kFluxXFaces, gyx = (g.M + 63) / 64, gyy = (g.N + 1 + FY - 1) / FY;
+  const dim3 by(64, kFluxYThreadRows);
+  if ((long)g.M * g.N <= kFluxOne<R>) {
+    const dim3 gr(gxx * ((g.N + kFluxYThreadRows - 1) / kFluxYThreadRows) + gyx * gyy);
+    if (disp)
+      launch(c, "flux_xy", k_flux_xy<R, true, PROD>, gr, by, d, g, c->prm<R>(), gxx, gyx);
+    else
+      launch(c, "flux_xy", k_flux_xy<R, false, PROD>, gr, by, d, g, c->prm<R>(), gxx, gyx);
+    return FW_OK;
+  }
+  const dim3 gx(gxx, (g.N + kB2.y - 1) / kB2.y);
   if (disp)
     launch(c, "flux_x", k_flux_x<R, true, PROD>, gx, kB2, d, g, c->prm<R>());
   else
@@ -466,19 +482,18 @@ int do_fluxes_as(fw_ctx *c) {
     // FP32: columns marched in strips of 4 faces (independent waves)
     constexpr int RS = 4;
     const int nt = (g.N + 1 + RS - 1) / RS;
-    const dim3 by(64, 4), gy((g.M + 63) / 64, (nt + 3) / 4);
+    const dim3 bm(64, 4), gm(gyx, (nt + 3) / 4);
     if (disp)
-      launch(c, "flux_y", k_flux_y_march<R, true, RS, PROD>, gy, by, d, g, c->prm<R>());
+      launch(c, "flux_y", k_flux_y_march<R, true, RS, PROD>, gm, bm, d, g, c->prm<R>());
     else
-      launch(c, "flux_y", k_flux_y_march<R, false, RS, PROD>, gy, by, d, g, c->prm<R>());
+      launch(c, "flux_y", k_flux_y_march<R, false, RS, PROD>, gm, bm, d, g, c->prm<R>());
   } else {
     // FP64: the LDS tile (the marching window would need 216 VGPRs)
-    constexpr int KY = FluxYK<R>::K, FY = FluxYTile<KY>::faces;
-    const dim3 gy((g.M + 63) / 64, (g.N + 1 + FY - 1) / FY), by(64, kFluxYThreadRows);
+    const dim3 gy(gyx, gyy);
     if (disp)
-      launch(c, "flux_y", k_flux_y<R, true, KY, PROD>, gy, by, d, g, c->prm<R>());
+      launch(c, "flux_y", k_flux_y<R, true, 1, PROD>, gy, by, d, g, c->prm<R>());
     else
-      launch(c, "flux_y", k_flux_y<R, false, KY, PROD>, gy, by, d, g, c->prm<R>());
+      launch(c, "flux_y", k_flux_y<R, false, 1, PROD>, gy, by, d, g, c->prm<R>());
   }
   return FW_OK;
 }
