@@ -13,6 +13,8 @@
 // arranges within one domain).  The kernels are the per-domain kernels' own
 // bodies (fw_kernels.h), so every member's arithmetic is exactly that of
 // fw_step on the member alone.
+// As in fw_step, a non-periodic member's step starts with one pass (kb_begin)
+// and what follows the line solves is another (kb_tail).
 //
 // Nothing goes back to the host during a run: each member's DT, TIME and
 // status live on the device (ESTIMATE_DT, misc.F:216-296, with FIXED_DT;
@@ -56,16 +58,16 @@ struct Member {
   Dev<R> d;
   Geo g;
   Prm<R> p;
-  HaloList hx[2];   // EXCHANGE arrays at buffer parity 0 / 1 (non-periodic: with P, Q)
-  HaloList hxf[2];  // periodic: the face arrays P, Q, filled after the cell arrays
-  HaloList hd;      // CAL_DISPERSION second derivatives (+ ETAx, ETAy)
+  HaloList hx[2];   // periodic: EXCHANGE cell arrays at buffer parity 0 / 1
+  HaloList hxf[2];  // periodic: the face arrays P, Q
+  HaloList hd;      // periodic: CAL_DISPERSION second derivatives (+ ETAx, ETAy)
   R *clk;           // [0] DT, [1] TIME, [2] max |eta|
   int *st;          // [0] status, [1] steps taken since the wavemaker table
                     // was filled, [2] steps taken in this run
   const R *wk;      // per step: AA, then the band's row / frequency factors
   int wks;          // stride of wk (0: no per-step wavemaker source)
   int show_brk;
-  int ndt, nmax;    // workgroups of the ESTIMATE_DT / CHECK_BLOWUP reductions
+  int ndt, nmax;    // block extremes that ESTIMATE_DT / CHECK_BLOWUP reduce
   size_t pe;        // elements of one plane
 };
 
@@ -109,14 +111,32 @@ __global__ void kb_copy3(FWB_ARGS) {
   }
 }
 
-// list 0: EXCHANGE cell arrays (non-periodic: with P, Q), 1: periodic P, Q,
-// 2: CAL_DISPERSION's arrays; queue y = array of the list
+// Periodic fills; list 0: EXCHANGE (queue y = array, then face array), 1:
+// CAL_DISPERSION's arrays
 template <class R>
-__global__ void kb_halo(FWB_ARGS, int list, int mode, int pm) {
+__global__ void kb_halo_per(FWB_ARGS, int list, int pm) {
   FWB_HEAD
-  const HaloList &L = list == 0 ? M.hx[pm] : (list == 1 ? M.hxf[pm] : M.hd);
-  if (e.y >= L.n) return;
-  halo_body<R>(L.a[e.y], M.g, mode, tile_blk(e));
+  const HaloList &L = list == 0 ? M.hx[pm] : M.hd;
+  if (e.y < L.n) halo_per_body<R>(L.a[e.y], M.g, tile_blk(e));
+  else halo_body<R>(M.hxf[pm].a[e.y - L.n], M.g, 0, tile_blk(e));
+}
+
+template <class R>
+__global__ void __launch_bounds__(256) kb_begin(FWB_ARGS, int pm, int pa) {
+  FWB_HEAD
+  begin_body<R>(mdev(M, pm, pa), M.g, M.p, tile_blk(e, e.aux));
+}
+
+template <class R, bool FILL>
+__global__ void __launch_bounds__(256) kb_tail(FWB_ARGS, int pm, int pa, int last) {
+  FWB_HEAD
+  tail_body<R, FILL>(mdev(M, pm, pa), M.g, M.p, M.clk[0], FILL && M.p.DIRECT_SPONGE, last, tile_blk(e, e.aux));
+}
+
+template <class R>
+__global__ void __launch_bounds__(1024) kb_brk2_fill(FWB_ARGS, int pm, int pa) {
+  FWB_HEAD
+  brk2_fill_body<R>(mdev(M, pm, pa), M.g, M.p, M.clk[0], tile_blk(e));
 }
 
 // sponge < 0: the member's own DIRECT_SPONGE
@@ -136,11 +156,12 @@ __global__ void kb_dt_partial(FWB_ARGS, int pm, int pa) {
 // DT_fixed (no halving), else the member stops here with ST_DT; then
 // TIME = TIME + DT
 template <class R>
-__global__ void kb_dt_final(FWB_ARGS) {
+__global__ void __launch_bounds__(1024) kb_dt_final(FWB_ARGS) {
   FWB_HEAD
-  dt_final_body<R>(M.d, M.p, M.ndt, M.clk, tile_blk(e));
+  const R least = extreme1024<R, false>(M.d.red, M.ndt, Lit<R>::large());
   if (threadIdx.x == 0) {
-    const R dt = M.clk[0];
+    const R dt = dt_of(M.p, least);
+    M.clk[0] = dt;
     if (dt != M.p.DTF) {
       M.st[0] = ST_DT;
     } else {
@@ -217,28 +238,9 @@ __global__ void __launch_bounds__(kTridThreads) kb_trid_solve(FWB_ARGS, int pm, 
 }
 
 template <class R>
-__global__ void kb_uv_final(FWB_ARGS, int pm, int pa) {
-  FWB_HEAD
-  uv_final_body<R>(mdev(M, pm, pa), M.g, M.p, tile_blk(e));
-}
-
-template <class R>
 __global__ void kb_ubar_from_hu(FWB_ARGS) {
   FWB_HEAD
   ubar_from_hu_body<R>(M.d, M.pe, tile_blk(e, e.aux));
-}
-
-template <class R>
-__global__ void kb_mask(FWB_ARGS, int pm, int pa) {
-  FWB_HEAD
-  mask_body<R>(mdev(M, pm, pa), M.g, M.p, tile_blk(e));
-}
-
-template <class R>
-__global__ void kb_brk1(FWB_ARGS, int pm, int pa) {
-  FWB_HEAD
-  if (!M.show_brk) return;
-  brk1_body<R>(mdev(M, pm, pa), M.g, M.p, M.clk[0], tile_blk(e));
 }
 
 template <class R>
@@ -256,10 +258,13 @@ __global__ void kb_maxeta_partial(FWB_ARGS) {
 
 // CHECK_BLOWUP (misc.F:394-433): a member over EtaBlowVal stops here
 template <class R>
-__global__ void kb_max_final(FWB_ARGS) {
+__global__ void __launch_bounds__(1024) kb_max_final(FWB_ARGS) {
   FWB_HEAD
-  max_final_body<R>(M.d, M.nmax, M.clk + 2, tile_blk(e));
-  if (threadIdx.x == 0 && M.clk[2] > M.p.BLOW) M.st[0] = ST_BLOWUP;
+  const R m = extreme1024<R, true>(M.d.red, M.nmax, (R)0);
+  if (threadIdx.x == 0) {
+    M.clk[2] = m;
+    if (m > M.p.BLOW) M.st[0] = ST_BLOWUP;
+  }
 }
 
 // start of a run: steps counter to zero (a kernel, not a memset, so that
@@ -276,8 +281,7 @@ __global__ void kb_reset_steps(int *const *st, int n) {
 // launch bounds); names as reported by fw_batch_autotune
 enum Group { G_DISP = 0, G_HUV, G_CELL, G_BRK, G_COUNT };
 const char *kGroupName[G_COUNT] = {"disp (disp_deriv, disp_terms; periodic members)", "src_huv",
-                                   "cell (uv_final, mask_mul)",
-                                   "mask/brk (mask, brk1)"};
+                                   "cell (mask_mul; periodic members)", "mask/brk (part of the fixed-shape tail)"};
 
 // The shapes a batch starts with: the single-domain step's (64 x 8 for the
 // neighbour-reading kernels, 64 x 4 elsewhere).  They are set explicitly: a
@@ -303,7 +307,7 @@ struct fw_batch {
   bool periodic = false, disp = false, pow2 = false;
   std::string err;
   hipStream_t stream = nullptr, side = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_fac = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_fac = nullptr;
   void *members = nullptr;     // Member<R>[n] on the device
   std::vector<char> members_h;  // host image
   void *clk = nullptr;         // n x 4 R
@@ -375,7 +379,8 @@ int upload_queue(fw_batch *b, Queue &Q) {
   return FW_OK;
 }
 
-// 2-D tile queue: member m covers ceil(nx(m)/bx) x ceil(ny(m)/by) tiles
+// 2-D tile queue: member m covers ceil(nx(m)/bx) x ceil(ny(m)/by) tiles; aux:
+// the tiles of a row
 template <class FX, class FY>
 int make_tiles(fw_batch *b, const std::string &name, dim3 block, int bx, int by, FX nx, FY ny) {
   Queue &Q = b->q[name];
@@ -385,7 +390,7 @@ int make_tiles(fw_batch *b, const std::string &name, dim3 block, int bx, int by,
     const Geo &g = b->mem[m]->g;
     const int tx = (nx(g) + bx - 1) / bx, ty = (ny(g) + by - 1) / by;
     for (int y = 0; y < ty; y++)
-      for (int x = 0; x < tx; x++) Q.h.push_back(QEnt{m, x, y, 0});
+      for (int x = 0; x < tx; x++) Q.h.push_back(QEnt{m, x, y, tx});
   }
   xcd_order(Q.h);
   return upload_queue(b, Q);
@@ -410,19 +415,19 @@ Member<R> &mem_h(fw_batch *b, int m) {
   return ((Member<R> *)b->members_h.data())[m];
 }
 
-// halo queue of one list: ghost chunks x arrays
+// halo queue of the periodic fills: ghost chunks x arrays
 template <class R>
-int make_halo_queue(fw_batch *b, const std::string &name, int which) {
+int make_halo_queue(fw_batch *b, const std::string &name, int list) {
   Queue &Q = b->q[name];
   Q.h.clear();
   Q.block = dim3(256);
   for (int m = 0; m < b->n; m++) {
     const Member<R> &M = mem_h<R>(b, m);
-    const HaloList &L = which == 0 ? M.hx[0] : (which == 1 ? M.hxf[0] : M.hd);
+    const int arrays = list == 0 ? M.hx[0].n + M.hxf[0].n : M.hd.n;
     const Geo &g = M.g;
     const int cnt = 6 * (g.M + 1) + 6 * (g.N + 1) + 64;
     const int nx = (cnt + 255) / 256;
-    for (int y = 0; y < L.n; y++)
+    for (int y = 0; y < arrays; y++)
       for (int x = 0; x < nx; x++) Q.h.push_back(QEnt{m, x, y, 0});
   }
   return upload_queue(b, Q);
@@ -446,10 +451,6 @@ void exchange_lists(fw_ctx *c, const Dev<R> &d, HaloList &L, HaloList &Lf) {
   hadd(L, d.HU, 2);
   hadd(L, d.V, 3);
   hadd(L, d.HV, 3);
-  if (!f.PERIODIC) {
-    for (int k = 0; k < Lf.n; k++) L.a[L.n++] = Lf.a[k];
-    Lf.n = 0;
-  }
 }
 
 template <class R>
@@ -458,6 +459,8 @@ void swapped(const Dev<R> &in, Dev<R> &out, bool brk) {
   std::swap(out.MASK, out.MASKn);
   if (brk) std::swap(out.AGE_BREAKING, out.AGEn);
 }
+
+inline int tiles(int n) { return (n + 63) / 64; }
 
 // the member table from the contexts' current arrays (parity 0 = as the
 // contexts hold them now)
@@ -468,6 +471,7 @@ int fill_members(fw_batch *b) {
     fw_ctx *c = b->mem[m];
     Member<R> &M = mem_h<R>(b, m);
     M.d = c->dev<R>();
+    if (!c->cfg.PERIODIC) M.d.EtaW = M.d.eta2;  // as in fw_step
     M.g = c->g;
     M.p = c->prm<R>();
     // the one-pass dispersion leaves the cross derivatives and U1p, V1p to
@@ -491,8 +495,13 @@ int fill_members(fw_batch *b) {
     M.wks = b->wk_stride[m];
     M.wk = M.wks ? (const R *)((char *)b->wk + b->wk_off[m]) : nullptr;
     const long ncell = (long)c->g.M * c->g.N;
-    M.ndt = (int)std::min<long>(kRedBlocks, (ncell + 255) / 256);
-    M.nmax = std::min(256, c->g.Je - c->g.Jb + 1);
+    if (c->cfg.PERIODIC) {
+      M.ndt = (int)std::min<long>(kRedBlocks, (ncell + 255) / 256);
+      M.nmax = std::min(256, c->g.Je - c->g.Jb + 1);
+    } else {  // the workgroups of kb_begin and kb_tail
+      M.ndt = tiles(c->g.M) * ((c->g.N + 3) / 4);
+      M.nmax = tiles(c->g.M + 1) * ((c->g.N + 4) / 4);
+    }
     M.pe = plane_elems(c->g);
   }
   BCHK(b, hipMemcpy(b->members, b->members_h.data(), b->members_h.size(), hipMemcpyHostToDevice));
@@ -506,15 +515,16 @@ int build_queues(fw_batch *b) {
   int rc;
   auto M_ = [](const Geo &g) { return g.M; };
   auto N_ = [](const Geo &g) { return g.N; };
-  const dim3 sd = b->shape[G_DISP], sh = b->shape[G_HUV], sc = b->shape[G_CELL], sb = b->shape[G_BRK];
+  const dim3 sd = b->shape[G_DISP], sh = b->shape[G_HUV], sc = b->shape[G_CELL];
   if ((rc = make_tiles(b, "disp", sd, sd.x, sd.y, M_, N_))) return rc;
   if ((rc = make_tiles(b, "dispf", dim3(kDispTX, kDispTY), kDispTX, kDispTY, M_, N_))) return rc;
   if ((rc = make_tiles(b, "huv", sh, sh.x, sh.y, M_, N_))) return rc;
   if ((rc = make_tiles(b, "cell", sc, sc.x, sc.y, M_, N_))) return rc;
-  if ((rc = make_tiles(b, "brk1", sb, sb.x, sb.y, M_, N_))) return rc;
-  if ((rc = make_tiles(b, "mask", sb, sb.x, sb.y, [](const Geo &g) { return g.M + 1; },
-                       [](const Geo &g) { return g.N + 1; })))
-    return rc;
+  auto M1 = [](const Geo &g) { return g.M + 1; };
+  auto N1 = [](const Geo &g) { return g.N + 1; };
+  // (one partial per workgroup: 64 x 4 threads, the tile row length in aux)
+  if ((rc = make_tiles(b, "begin", dim3(64, 4), 64, 4, M_, N_))) return rc;
+  if ((rc = make_tiles(b, "tail", dim3(64, 4), 64, 4, M1, N1))) return rc;
   if ((rc = make_tiles(b, "flux_x", dim3(64, 4), kFluxXFaces, 4, [](const Geo &g) { return g.M + 1; }, N_)))
     return rc;
   if (b->rb == 4) {  // columns marched in strips of 4 faces, 64 x 4 threads
@@ -527,7 +537,6 @@ int build_queues(fw_batch *b) {
   auto mem = [b](int m) -> const Member<R> & { return mem_h<R>(b, m); };
   if ((rc = make_line(b, "dt", dim3(256), [&](int m) { return mem(m).ndt; }, [](int) { return 0; }))) return rc;
   if ((rc = make_line(b, "max", dim3(256), [&](int m) { return mem(m).nmax; }, [](int) { return 0; }))) return rc;
-  if ((rc = make_line(b, "one", dim3(256), [](int) { return 1; }, [](int) { return 0; }))) return rc;
   if ((rc = make_line(b, "one1024", dim3(1024), [](int) { return 1; }, [](int) { return 0; }))) return rc;
   auto chunks = [&](int m) { return (int)std::min<size_t>(2048, (mem(m).pe + 2047) / 2048); };
   if ((rc = make_line(b, "copy", dim3(256), chunks, chunks))) return rc;
@@ -547,9 +556,10 @@ int build_queues(fw_batch *b) {
   b->trid = trid_lds<R>(rows);
   b->trid_fixed = true;
   for (int m = 0; m < b->n; m++) b->trid_fixed = b->trid_fixed && trid_fixed(mem(m).p);
-  if ((rc = make_halo_queue<R>(b, "halo_x", 0))) return rc;
-  if ((rc = make_halo_queue<R>(b, "halo_xf", 1))) return rc;
-  if ((rc = make_halo_queue<R>(b, "halo_d", 2))) return rc;
+  if (b->periodic) {
+    if ((rc = make_halo_queue<R>(b, "halo_x", 0))) return rc;
+    if ((rc = make_halo_queue<R>(b, "halo_d", 1))) return rc;
+  }
   return FW_OK;
 }
 
@@ -569,32 +579,32 @@ void bl(fw_batch *b, hipStream_t s, const char *qname, K k, A... args) {
   bl_lds<R>(b, s, qname, 0, k, args...);
 }
 
-// EXCHANGE (+ SPONGE_DAMPING when sponge) at buffer parity par
+// periodic EXCHANGE (+ SPONGE_DAMPING when sponge) at buffer parity par
 template <class R>
 void rec_exchange(fw_batch *b, int par, int sponge) {
   hipStream_t s = b->stream;
-  if (!b->periodic) {
-    bl<R>(b, s, "halo_x", kb_halo<R>, 0, 0, par);
-  } else {
-    bl<R>(b, s, "halo_x", kb_halo<R>, 0, 1, par);
-    bl<R>(b, s, "halo_x", kb_halo<R>, 0, 2, par);
-    bl<R>(b, s, "halo_xf", kb_halo<R>, 1, 0, par);
-  }
+  bl<R>(b, s, "halo_x", kb_halo_per<R>, 0, par);
   bl<R>(b, s, "cell", kb_mask_mul<R>, par, par, sponge, 1);
 }
 
-// one whole step, starting at buffer parity p0 (do_step's sequence); first:
-// the first step of a call, whose first two stages form the line solves' c'
+// one whole step, starting at buffer parity p0 (do_step_prod's sequence);
+// first: the first step of a call, whose first two stages form the line
+// solves' c'
 template <class R, bool P2>
 int rec_step(fw_batch *b, int p0, bool first) {
   hipStream_t s = b->stream, sd = b->side;
   const R alpha[3] = {(R)0, (R)3 / (R)4, (R)1 / (R)3};
   const R beta[3] = {(R)1, (R)1 / (R)4, (R)2 / (R)3};
+  const bool per = b->periodic;
   int par = p0;
-  bl<R>(b, s, "copy", kb_copy3<R>);
-  rec_exchange<R>(b, par, 0);
-  bl<R>(b, s, "dt", kb_dt_partial<R>, par, par);
-  bl<R>(b, s, "one", kb_dt_final<R>);
+  if (!per) {
+    bl<R>(b, s, "begin", kb_begin<R>, par, par);
+  } else {
+    bl<R>(b, s, "copy", kb_copy3<R>);
+    rec_exchange<R>(b, par, 0);
+    bl<R>(b, s, "dt", kb_dt_partial<R>, par, par);
+  }
+  bl<R>(b, s, "one1024", kb_dt_final<R>);
   for (int st = 0; st < 3; st++) {
     const bool fac = b->disp && ((first && st < 2) || !b->trid_fixed);
     if (fac) {  // beside the dispersion and the fluxes
@@ -603,16 +613,11 @@ int rec_step(fw_batch *b, int p0, bool first) {
       bl<R>(b, sd, "trid_fac", kb_trid_fac<R>, par, par);
       BCHK(b, hipEventRecord(b->ev_fac, sd));
     }
-    if (b->disp && !b->periodic) {
+    if (b->disp && !per) {
       bl<R>(b, s, "dispf", kb_disp_fused<R, P2>, par, par);
     } else if (b->disp) {
       bl<R>(b, s, "disp", kb_disp_deriv<R, P2>, par, par);
-      if (!b->periodic) {
-        bl<R>(b, s, "halo_d", kb_halo<R>, 2, 0, par);
-      } else {
-        bl<R>(b, s, "halo_d", kb_halo<R>, 2, 1, par);
-        bl<R>(b, s, "halo_d", kb_halo<R>, 2, 2, par);
-      }
+      bl<R>(b, s, "halo_d", kb_halo_per<R>, 1, par);
       bl<R>(b, s, "disp", kb_disp_terms<R, P2>, par, par);
     }
     if (b->disp) bl<R>(b, s, "flux_x", kb_flux_x<R, true>, par, par);
@@ -625,31 +630,29 @@ int rec_step(fw_batch *b, int p0, bool first) {
       else bl<R>(b, s, "flux_y", kb_flux_y<R, false, 1>, par, par);
     }
     if (fac) BCHK(b, hipStreamWaitEvent(s, b->ev_fac, 0));
-    if (b->disp && !b->periodic) bl<R>(b, s, "huv", kb_huv<R, P2, true>, par, par, alpha[st], beta[st]);
+    if (b->disp && !per) bl<R>(b, s, "huv", kb_huv<R, P2, true>, par, par, alpha[st], beta[st]);
     else bl<R>(b, s, "huv", kb_huv<R, P2>, par, par, alpha[st], beta[st]);
-    // line solves and the velocity tail beside UPDATE_MASK + WAVE_BREAKING
-    BCHK(b, hipEventRecord(b->ev_fork, s));
-    BCHK(b, hipStreamWaitEvent(sd, b->ev_fork, 0));
     if (b->disp) {
       auto solve = [&](auto kres, auto kstream) {
         if (b->trid.res) bl_lds<R>(b, s, "trid", b->trid.lds, kres, par, par);
         else bl_lds<R>(b, s, "trid", b->trid.lds, kstream, par, par);
       };
-      if (b->periodic) solve(kb_trid_solve<R, true, true>, kb_trid_solve<R, false, true>);
+      if (per) solve(kb_trid_solve<R, true, true>, kb_trid_solve<R, false, true>);
       else solve(kb_trid_solve<R, true, false>, kb_trid_solve<R, false, false>);
     }
-    bl<R>(b, s, "cell", kb_uv_final<R>, par, par);
-    if (!b->disp) bl<R>(b, s, "copy", kb_ubar_from_hu<R>);
-    bl<R>(b, sd, "mask", kb_mask<R>, par, par);
-    bl<R>(b, sd, "brk1", kb_brk1<R>, par ^ 1, par);
-    bl<R>(b, sd, "one1024", kb_brk2<R>, par ^ 1, par);
-    BCHK(b, hipEventRecord(b->ev_join, sd));
-    BCHK(b, hipStreamWaitEvent(s, b->ev_join, 0));
+    if (!per) {
+      bl<R>(b, s, "tail", kb_tail<R, true>, par, par, st == 2 ? 1 : 0);
+      bl<R>(b, s, "one1024", kb_brk2_fill<R>, par, par);
+    } else {
+      bl<R>(b, s, "tail", kb_tail<R, false>, par, par, 0);
+      if (!b->disp) bl<R>(b, s, "copy", kb_ubar_from_hu<R>);
+      bl<R>(b, s, "one1024", kb_brk2<R>, par, par);
+    }
     par ^= 1;
-    rec_exchange<R>(b, par, -1);
+    if (per) rec_exchange<R>(b, par, -1);
   }
-  bl<R>(b, s, "max", kb_maxeta_partial<R>);
-  bl<R>(b, s, "one", kb_max_final<R>);
+  if (per) bl<R>(b, s, "max", kb_maxeta_partial<R>);
+  bl<R>(b, s, "one1024", kb_max_final<R>);
   return FW_OK;
 }
 
@@ -906,6 +909,7 @@ int autotune(fw_batch *b, int trial, std::string &rep) {
     // the two-pass dispersion kernels run only for periodic members (the
     // others take the fused kernel, whose tile is fixed)
     if (gi == G_DISP && !(b->disp && b->periodic)) continue;
+    if ((gi == G_CELL && !b->periodic) || gi == G_BRK) continue;  // UPDATE_MASK and breaking are in kb_tail
     dim3 best = cand[gi][0];
     double best_ms = 1e30;
     for (const dim3 &s : cand[gi]) {
@@ -1007,7 +1011,6 @@ int fw_batch_create(fw_ctx *const *members, int n, fw_batch **out) {
     if (hipSetDevice(c0->device) != hipSuccess || hipStreamCreate(&b->stream) != hipSuccess ||
         hipStreamCreate(&b->side) != hipSuccess ||
         hipEventCreateWithFlags(&b->ev_fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&b->ev_join, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&b->ev_fac, hipEventDisableTiming) != hipSuccess)
       rc = bfail(b, FW_E_HIP, "stream/event creation failed");
   }
@@ -1033,7 +1036,6 @@ int fw_batch_destroy(fw_batch *b) {
   for (void *p : b->allocs) (void)hipFree(p);
   if (b->pinned) (void)hipHostFree(b->pinned);
   if (b->ev_fork) (void)hipEventDestroy(b->ev_fork);
-  if (b->ev_join) (void)hipEventDestroy(b->ev_join);
   if (b->ev_fac) (void)hipEventDestroy(b->ev_fac);
   if (b->side) (void)hipStreamDestroy(b->side);
   if (b->stream) (void)hipStreamDestroy(b->stream);
