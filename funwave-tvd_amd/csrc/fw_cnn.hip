@@ -253,81 +253,137 @@ __global__ void k_loss(const float *__restrict__ out, const float *__restrict__ 
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-// Weight and bias gradients of one layer over a tile of 4 rows x 64
-// pixels: thread (tap, ci) accumulates dW[tap][ci][0..COUT) in fp32;
-// partial sums per workgroup, reduced by k_reduce_grad.
-//   in: layer input, CIN channels stored (CREAL used); g: gradient of the
-//   layer's pre-activation output, GC channels stored (COUT used).
+// Weight and bias gradients on the matrix cores.  dW[tap][ci][co] is a sum of
+// in[pixel + tap][ci] * g[pixel][co] over pixels: M = 16 (tap, ci) rows, N = 16
+// output channels, K = 32 pixels of a row, bf16 operands, fp32 accumulation.
+// A lane's fragment is 8 consecutive pixels of one channel, so a tile (4 rows
+// x 64 pixels) is staged into LDS channel by channel: thread (row, 8 channels,
+// 8 pixels) loads its pixels as they lie, transposes them in registers and
+// writes 16 B per channel.  A tap's column offset would misalign the
+// fragments, so the input is staged three times, shifted by -1, 0, +1 pixel.
+// Channel rows are 72 pixels apart: the 16 channels of a fragment read cover
+// all 64 banks.  A workgroup walks tiles and keeps its sums in registers;
+// partials go to part[workgroup] in the parameters' own layout and
+// k_reduce_adam adds them.  All four layers are one launch (blockIdx.y).
+// 16 samples of 64 x 64: fp32 loops on one LDS element at a time took 286 us
+// and their serial reductions, Adam and repacking 248; now 23 and 5.
+constexpr int kWgPx = 72;    // LDS pixels per channel row
+constexpr int kWgMax = 128;  // workgroups per layer (partial sums)
+template <int CIN, int GC>
+struct WgTile {
+  static constexpr int in = 3 * 6 * CIN * kWgPx, g = 4 * GC * kWgPx;  // bf16 elements
+  static constexpr size_t bytes = (size_t)(in + g) * sizeof(bf16);
+};
+// 16 bits of channel ch of a pixel's 8 channels
+__device__ __forceinline__ uint32_t ch16(const uint4 &v, int ch) {
+  const uint32_t w = ch < 2 ? v.x : (ch < 4 ? v.y : (ch < 6 ? v.z : v.w));
+  return ch & 1 ? w >> 16 : w & 0xffffu;
+}
 template <int CIN, int CREAL, int GC, int COUT>
-__global__ void __launch_bounds__(9 * CIN) k_wgrad(const bf16 *__restrict__ in, const bf16 *__restrict__ gin,
-                                                   float *__restrict__ part, Grid g) {
-  __shared__ __attribute__((aligned(16))) bf16 sin_[6][66][CIN];
-  __shared__ float sg[4][64][COUT];
-  const int t = threadIdx.x;
-  const int b = blockIdx.z, y0 = blockIdx.y * 4, x0 = blockIdx.x * 64;
-  // stage the input tile with a one-pixel halo (rows y0-1..y0+4), and g
-  for (int e = t; e < 6 * 66 * CIN / 8; e += blockDim.x) {
-    const int c8 = e % (CIN / 8), px = (e / (CIN / 8)) % 66, ry = e / (CIN / 8) / 66;
-    const int yy = y0 - 1 + ry, xx = x0 - 1 + px;
-    uint4 v{0u, 0u, 0u, 0u};
-    if (yy >= -1 && yy <= g.H && xx >= -1 && xx <= g.W)
-      v = *(const uint4 *)(in + ((size_t)b * g.PS + (size_t)(yy + 1) * (g.W + 2) + (xx + 1)) * CIN + 8 * c8);
-    *(uint4 *)&sin_[ry][px][8 * c8] = v;
+__device__ __forceinline__ void wgrad_layer(const bf16 *__restrict__ in, const bf16 *__restrict__ gin,
+                                            float *__restrict__ dst, const Grid &g, int ntx, int nty, int ntiles,
+                                            bf16 *smem) {
+  // M-tiles: 32 channels: tap x two halves; 8 channels: two taps each
+  constexpr int MT = CIN == 32 ? 18 : 5, NT = GC == 32 ? 2 : 1, JOBS = MT * NT, PERW = (JOBS + 3) / 4;
+  bf16 *const si = smem, *const sg = smem + WgTile<CIN, GC>::in;
+  const int t = threadIdx.x, wave = t >> 6, l = t & 63, row = l & 15, grp = l >> 4;
+  // job j of wave w: w + 4 j; its N-tile is the same for every j
+  const int nt = wave % NT;
+  f32x4 acc[PERW], accb = f32x4{0.f, 0.f, 0.f, 0.f};
+  int abase[PERW];
+#pragma unroll
+  for (int j = 0; j < PERW; j++) {
+    acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int mt = min(wave + 4 * j, JOBS - 1) / NT;
+    const int tap = CIN == 32 ? mt / 2 : min(2 * mt + row / 8, 8);
+    const int ci = CIN == 32 ? 16 * (mt % 2) + row : row % 8;
+    abase[j] = (((tap % 3) * 6 + tap / 3) * CIN + ci) * kWgPx + 8 * grp;
   }
-  for (int e = t; e < 4 * 64 * COUT; e += blockDim.x) {
-    const int co = e % COUT, px = (e / COUT) % 64, ry = e / COUT / 64;
-    const int yy = y0 + ry, xx = x0 + px;
-    float v = 0.f;
-    if (yy < g.H && xx < g.W) v = bf2f(gin[g.pix(b, yy, xx) * GC + co]);
-    sg[ry][px][co] = v;
-  }
-  __syncthreads();
-  const int tap = t / CIN, ci = t % CIN;
-  const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-  float acc[COUT], accb[COUT];
+  const int bbase = (GC == 32 ? 16 * nt + row : row % 8) * kWgPx + 8 * grp;
+  bf16x8 ones;
 #pragma unroll
-  for (int co = 0; co < COUT; co++) acc[co] = accb[co] = 0.f;
-  const bool doBias = (t == 0);
-  for (int ry = 0; ry < 4; ry++)
-    for (int px = 0; px < 64; px++) {
-      const float a = bf2f(sin_[ry + 1 + dy][px + 1 + dx][ci]);
+  for (int e = 0; e < 8; e++) ones[e] = (__bf16)1.f;
+  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const int b = tile / (ntx * nty), ty = tile / ntx % nty, tx = tile % ntx;
+    const int y0 = 4 * ty, x0 = 64 * tx;
+    __syncthreads();  // the last tile's fragments have been read
+    for (int e = t; e < 6 * CIN; e += 256) {  // (row, 8 pixels, 8 channels)
+      const int c8 = e % (CIN / 8), pb = e / (CIN / 8) % 8, r = e / CIN;
+      const int yy = y0 - 1 + r;
+      uint4 v[10];
 #pragma unroll
-      for (int co = 0; co < COUT; co++) acc[co] += a * sg[ry][px][co];
-      if (doBias) {
+      for (int q = 0; q < 10; q++) {
+        const int xx = x0 + 8 * pb - 1 + q;
+        v[q] = uint4{0u, 0u, 0u, 0u};
+        if (yy <= g.H && xx <= g.W) v[q] = *(const uint4 *)(in + g.pix(b, yy, xx) * CIN + 8 * c8);
+      }
 #pragma unroll
-        for (int co = 0; co < COUT; co++) accb[co] += sg[ry][px][co];
+      for (int ch = 0; ch < 8; ch++)
+#pragma unroll
+        for (int s = 0; s < 3; s++) {
+          uint32_t w[4];
+#pragma unroll
+          for (int k = 0; k < 4; k++) w[k] = ch16(v[s + 2 * k], ch) | (ch16(v[s + 2 * k + 1], ch) << 16);
+          *(uint4 *)&si[((s * 6 + r) * CIN + 8 * c8 + ch) * kWgPx + 8 * pb] = uint4{w[0], w[1], w[2], w[3]};
+        }
+    }
+    for (int e = t; e < 4 * GC; e += 256) {
+      const int c8 = e % (GC / 8), pb = e / (GC / 8) % 8, r = e / GC;
+      const int yy = y0 + r;
+      uint4 v[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const int xx = x0 + 8 * pb + q;
+        v[q] = uint4{0u, 0u, 0u, 0u};
+        if (yy < g.H && xx < g.W) v[q] = *(const uint4 *)(gin + g.pix(b, yy, xx) * GC + 8 * c8);
+      }
+#pragma unroll
+      for (int ch = 0; ch < 8; ch++) {
+        uint32_t w[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) w[k] = ch16(v[2 * k], ch) | (ch16(v[2 * k + 1], ch) << 16);
+        *(uint4 *)&sg[(r * GC + 8 * c8 + ch) * kWgPx + 8 * pb] = uint4{w[0], w[1], w[2], w[3]};
       }
     }
-  const size_t nblk = (size_t)blockIdx.x + (size_t)gridDim.x * (blockIdx.y + (size_t)gridDim.y * blockIdx.z);
-  float *dst = part + nblk * (9 * CREAL * COUT + COUT);
-  if (ci < CREAL) {
+    __syncthreads();
+#pragma unroll 2
+    for (int kk = 0; kk < 8; kk++) {  // 32 pixels: row kk/2, half kk%2
+      const int ro = kk >> 1, po = 32 * (kk & 1);
+      const bf16x8 fb = *(const bf16x8 *)&sg[ro * GC * kWgPx + bbase + po];
 #pragma unroll
-    for (int co = 0; co < COUT; co++) dst[(tap * CREAL + ci) * COUT + co] = acc[co];
+      for (int j = 0; j < PERW; j++) {
+        const bf16x8 fa = *(const bf16x8 *)&si[ro * CIN * kWgPx + abase[j] + po];
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb, acc[j], 0, 0, 0);
+      }
+      if (wave < NT) accb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, fb, accb, 0, 0, 0);
+    }
   }
-  if (doBias) {
+  const int co = 16 * nt + row;  // (8-channel gradients: columns past COUT are dropped)
 #pragma unroll
-    for (int co = 0; co < COUT; co++) dst[9 * CREAL * COUT + co] = accb[co];
+  for (int j = 0; j < PERW; j++) {
+    if (wave + 4 * j >= JOBS) continue;
+    const int mt = (wave + 4 * j) / NT;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int m = 4 * grp + r;
+      const int tap = CIN == 32 ? mt / 2 : 2 * mt + m / 8, ci = CIN == 32 ? 16 * (mt % 2) + m : m % 8;
+      if (tap < 9 && ci < CREAL && co < COUT) dst[(tap * CREAL + ci) * COUT + co] = acc[j][r];
+    }
   }
+  if (wave < NT && grp == 0 && co < COUT) dst[9 * CREAL * COUT + co] = accb[0];
 }
-
-// grad[off + k] = sum over blocks of part[blk][k]
-__global__ void k_reduce_grad(const float *__restrict__ part, int nblk, int len, float *__restrict__ grad) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= len) return;
-  float s = 0.f;
-  for (int q = 0; q < nblk; q++) s += part[(size_t)q * len + k];
-  grad[k] = s;
-}
-
-__global__ void k_adam(float *p, float *m, float *v, const float *gr, int n, float lr, float c1, float c2) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  const float gk = gr[k];
-  const float mk = 0.9f * m[k] + 0.1f * gk;
-  const float vk = 0.999f * v[k] + 0.001f * gk * gk;
-  m[k] = mk;
-  v[k] = vk;
-  p[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + 1e-8f);
+struct WgArgs {
+  const bf16 *a[4], *g[4];  // input and output gradient of layers 1..4
+};
+__global__ void __launch_bounds__(256) k_wgrad(WgArgs w, float *__restrict__ part, Grid g, int ntx, int nty, int ntiles) {
+  extern __shared__ __attribute__((aligned(16))) bf16 wg_smem[];
+  float *dst = part + (size_t)blockIdx.x * kNP;
+  switch (blockIdx.y) {
+    case 0: wgrad_layer<32, kC, 32, kC>(w.a[1], w.g[1], dst + oW2, g, ntx, nty, ntiles, wg_smem); break;
+    case 1: wgrad_layer<32, kC, 32, kC>(w.a[2], w.g[2], dst + oW3, g, ntx, nty, ntiles, wg_smem); break;
+    case 2: wgrad_layer<8, kCin, 32, kC>(w.a[0], w.g[0], dst + oW1, g, ntx, nty, ntiles, wg_smem); break;
+    default: wgrad_layer<32, kC, 8, kCout>(w.a[3], w.g[3], dst + oW4, g, ntx, nty, ntiles, wg_smem); break;
+  }
 }
 
 // forward and data-gradient weight packs from the fp32 parameters
@@ -376,6 +432,57 @@ __global__ void k_pack(const float *__restrict__ p, Packs k) {
     k.bias3[t] = p[oB3 + t];
   }
   if (t < 16) k.bias4[t] = t < kCout ? p[oB4 + t] : 0.f;
+}
+
+// The gradient (the sum of nblk partials, in a fixed order), Adam, and the
+// parameter's places in the weight packs (as k_pack lays them out; their
+// padding stays zero).  Workgroup: 32 parameters x 8 groups of partials.
+__global__ void __launch_bounds__(256) k_reduce_adam(const float *__restrict__ part, int nblk, float *__restrict__ grad,
+                                                     float *__restrict__ p, float *__restrict__ m, float *__restrict__ v,
+                                                     float lr, float c1, float c2, Packs pk) {
+  __shared__ float sm[8][32];
+  const int c = threadIdx.x & 31, q = threadIdx.x >> 5, k = blockIdx.x * 32 + c;
+  float s = 0.f;
+  if (k < kNP) {
+#pragma unroll 4
+    for (int b = q; b < nblk; b += 8) s += part[(size_t)b * kNP + k];
+  }
+  sm[q][c] = s;
+  __syncthreads();
+  if (q || k >= kNP) return;
+  float gk = sm[0][c];
+#pragma unroll
+  for (int r = 1; r < 8; r++) gk += sm[r][c];
+  grad[k] = gk;
+  const float mk = 0.9f * m[k] + 0.1f * gk;
+  const float vk = 0.999f * v[k] + 0.001f * gk * gk;
+  m[k] = mk;
+  v[k] = vk;
+  const float pn = p[k] - lr * (mk / c1) / (sqrtf(vk / c2) + 1e-8f);
+  p[k] = pn;
+  const bf16 h = f2bf(pn);
+  if (k < oB1) {
+    const int tap = k / (kCin * kC), ci = k / kC % kCin, co = k % kC;
+    pk.f1[((tap / 4 * 2 + co / 16) * 64 + tap % 4 * 16 + co % 16) * 8 + ci] = h;
+  } else if (k < oW2) {
+    pk.bias1[k - oB1] = pn;
+  } else if (k < oW4) {
+    const bool two = k < oW3;
+    const int i = k - (two ? oW2 : oW3);
+    if (i >= 9 * kC * kC) {
+      (two ? pk.bias2 : pk.bias3)[i - 9 * kC * kC] = pn;
+    } else {
+      const int tap = i / (kC * kC), ci = i / kC % kC, co = i % kC;
+      (two ? pk.f2 : pk.f3)[((tap * 2 + co / 16) * 64 + ci / 8 * 16 + co % 16) * 8 + ci % 8] = h;
+      (two ? pk.b2 : pk.b3)[(((8 - tap) * 2 + ci / 16) * 64 + co / 8 * 16 + ci % 16) * 8 + co % 8] = h;
+    }
+  } else if (k < oB4) {
+    const int i = k - oW4, tap = i / (kC * kCout), ci = i / kCout % kC, co = i % kCout, tp = 8 - tap;
+    pk.f4[(tap * 64 + ci / 8 * 16 + co) * 8 + ci % 8] = h;
+    pk.b4[((tp / 4 * 2 + ci / 16) * 64 + tp % 4 * 16 + ci % 16) * 8 + co] = h;
+  } else {
+    pk.bias4[k - oB4] = pn;
+  }
 }
 
 // wet-cell mean of the eta correction (R)(o0*s0), accumulated in FP64 by
@@ -475,10 +582,7 @@ int cget(fw_cnn *n, size_t count, T **out) {
   return FW_OK;
 }
 
-constexpr int kWgBlockRows = 4;
-
 dim3 conv_grid(const fw_cnn *n, int B) { return dim3((n->W + 63) / 64, (n->H + 3) / 4, B); }
-dim3 wgrad_grid(const fw_cnn *n, int B) { return dim3((n->W + 63) / 64, (n->H + kWgBlockRows - 1) / kWgBlockRows, B); }
 
 void forward(fw_cnn *n, int B) {
   const dim3 gr = conv_grid(n, B), bl(256);
@@ -514,9 +618,7 @@ int fw_cnn_create(int H, int W, int max_batch, fw_cnn **out) {
   if (hipStreamCreate(&n->stream) != hipSuccess) { delete n; return FW_E_HIP; }
   const size_t px = (size_t)max_batch * n->g.PS;
   const size_t plane = (size_t)max_batch * H * W;
-  const dim3 wg = wgrad_grid(n, max_batch);
-  const size_t nblk = (size_t)wg.x * wg.y * wg.z;
-  n->part_len = nblk * (9 * kC * kC + kC);
+  n->part_len = (size_t)kWgMax * kNP;
   int rc;
   if ((rc = cget(n, kNP, &n->params)) || (rc = cget(n, kNP, &n->am)) || (rc = cget(n, kNP, &n->av)) ||
       (rc = cget(n, kNP, &n->grad)) || (rc = cget(n, n->part_len, &n->part)) || (rc = cget(n, 4096, &n->lpart)) ||
@@ -602,30 +704,21 @@ int fw_cnn_train_step(fw_cnn *n, const float *in, const float *target, int B, fl
   hipLaunchKernelGGL((k_conv<8, 2, MODE_MASK>), gr, bl, 0, n->stream, n->g4, n->pk.b4, nullptr, n->g3, n->a3, n->g);
   hipLaunchKernelGGL((k_conv<32, 2, MODE_MASK>), gr, bl, 0, n->stream, n->g3, n->pk.b3, nullptr, n->g2, n->a2, n->g);
   hipLaunchKernelGGL((k_conv<32, 2, MODE_MASK>), gr, bl, 0, n->stream, n->g2, n->pk.b2, nullptr, n->g1, n->a1, n->g);
-  // weight gradients, reduced into the parameter layout
-  const dim3 wg = wgrad_grid(n, B);
-  const int nblk = (int)(wg.x * wg.y * wg.z);
-  auto reduce = [&](int len, int off) {
-    hipLaunchKernelGGL(k_reduce_grad, dim3((len + 255) / 256), dim3(256), 0, n->stream, n->part, nblk, len,
-                       n->grad + off);
-  };
-  hipLaunchKernelGGL((k_wgrad<8, kCin, 32, kC>), wg, dim3(9 * 8), 0, n->stream, n->a0, n->g1, n->part, n->g);
-  reduce(9 * kCin * kC + kC, oW1);
-  hipLaunchKernelGGL((k_wgrad<32, kC, 32, kC>), wg, dim3(9 * 32), 0, n->stream, n->a1, n->g2, n->part, n->g);
-  reduce(9 * kC * kC + kC, oW2);
-  hipLaunchKernelGGL((k_wgrad<32, kC, 32, kC>), wg, dim3(9 * 32), 0, n->stream, n->a2, n->g3, n->part, n->g);
-  reduce(9 * kC * kC + kC, oW3);
-  hipLaunchKernelGGL((k_wgrad<32, kC, 8, kCout>), wg, dim3(9 * 32), 0, n->stream, n->a3, n->g4, n->part, n->g);
-  reduce(9 * kC * kCout + kCout, oW4);
+  // weight gradients, then their sum, Adam and the new weight packs
+  n->adam_t += 1;
+  const float c1 = 1.f - powf(0.9f, (float)n->adam_t), c2 = 1.f - powf(0.999f, (float)n->adam_t);
+  const dim3 wt = conv_grid(n, B);  // tiles of 4 rows x 64 pixels
+  const int ntiles = (int)(wt.x * wt.y * wt.z), nwg = ntiles < kWgMax ? ntiles : kWgMax;
+  const WgArgs wa{{n->a0, n->a1, n->a2, n->a3}, {n->g1, n->g2, n->g3, n->g4}};
+  hipLaunchKernelGGL(k_wgrad, dim3(nwg, 4), dim3(256), (WgTile<32, 32>::bytes), n->stream, wa, n->part, n->g, (int)wt.x,
+                     (int)wt.y, ntiles);
+  CHK(n, hipGetLastError());
+  hipLaunchKernelGGL(k_reduce_adam, dim3((kNP + 31) / 32), dim3(256), 0, n->stream, n->part, nwg, n->grad, n->params,
+                     n->am, n->av, lr, c1, c2, n->pk);
   CHK(n, hipGetLastError());
   if (grad) CHK(n, hipMemcpyAsync(grad, n->grad, kNP * sizeof(float), hipMemcpyDeviceToHost, n->stream));
   std::vector<float> lp(nlb);
   CHK(n, hipMemcpyAsync(lp.data(), n->lpart, nlb * sizeof(float), hipMemcpyDeviceToHost, n->stream));
-  n->adam_t += 1;
-  const float c1 = 1.f - powf(0.9f, (float)n->adam_t), c2 = 1.f - powf(0.999f, (float)n->adam_t);
-  hipLaunchKernelGGL(k_adam, dim3((kNP + 255) / 256), dim3(256), 0, n->stream, n->params, n->am, n->av, n->grad,
-                     kNP, lr, c1, c2);
-  if ((rc = pack(n))) return rc;
   CHK(n, hipStreamSynchronize(n->stream));
   if (loss) {
     double s = 0;
