@@ -485,29 +485,51 @@ __global__ void __launch_bounds__(256) k_reduce_adam(const float *__restrict__ p
   }
 }
 
-// wet-cell mean of the eta correction (R)(o0*s0), accumulated in FP64 by
-// one workgroup in a fixed order (deterministic); 0 without wet cells
-template <class R>
-__global__ void __launch_bounds__(1024) k_wet_mean(const float *__restrict__ o, const int *mask, int P, int Ib, int Jb,
-                                                   int H, int W, float s0, double *mean) {
-  __shared__ double ss[1024], sc[1024];
+// wet-cell mean of the eta correction (R)(o0*s0), accumulated in FP64 in a
+// fixed order (deterministic); 0 without wet cells.  Rows go to the
+// workgroups in turn; the last launch (one workgroup) adds their sums.  (One
+// workgroup over all cells took 193 us at 700 x 468, the two launches 10.)
+constexpr int kWetBlocks = 256;
+__device__ __forceinline__ void sum2_256(double &s, double &c) {
+  __shared__ double ss[256], sc[256];
   const int t = threadIdx.x;
-  double s = 0, c = 0;
-  for (int k = t; k < H * W; k += 1024) {
-    const int y = k / W, x = k - y * W;
-    if (mask[(size_t)(Jb - 1 + y) * P + (Ib - 1 + x)] >= 1) {
-      s += (double)(R)(o[k] * s0);
-      c += 1;
-    }
-  }
   ss[t] = s;
   sc[t] = c;
   __syncthreads();
-  for (int w = 512; w > 0; w >>= 1) {
+  for (int w = 128; w > 0; w >>= 1) {
     if (t < w) { ss[t] += ss[t + w]; sc[t] += sc[t + w]; }
     __syncthreads();
   }
-  if (t == 0) mean[0] = sc[0] > 0 ? ss[0] / sc[0] : 0.0;
+  s = ss[0];
+  c = sc[0];
+}
+template <class R>
+__global__ void __launch_bounds__(256) k_wet_sum(const float *__restrict__ o, const int *__restrict__ mask, int P,
+                                                 int Ib, int Jb, int H, int W, float s0, double *part) {
+  double s = 0, c = 0;
+  for (int y = blockIdx.x; y < H; y += gridDim.x) {
+    const int *mrow = mask + (size_t)(Jb - 1 + y) * P + (Ib - 1);
+    const float *orow = o + (size_t)y * W;
+    for (int x = threadIdx.x; x < W; x += 256)
+      if (mrow[x] >= 1) {
+        s += (double)(R)(orow[x] * s0);
+        c += 1;
+      }
+  }
+  sum2_256(s, c);
+  if (threadIdx.x == 0) {
+    part[2 * blockIdx.x] = s;
+    part[2 * blockIdx.x + 1] = c;
+  }
+}
+__global__ void __launch_bounds__(256) k_wet_mean(const double *__restrict__ part, int n, double *mean) {
+  double s = 0, c = 0;
+  if ((int)threadIdx.x < n) {
+    s = part[2 * threadIdx.x];
+    c = part[2 * threadIdx.x + 1];
+  }
+  sum2_256(s, c);
+  if (threadIdx.x == 0) mean[0] = c > 0 ? s / c : 0.0;
 }
 
 // correction of the coarse state from the network output (planar [3][H][W]);
@@ -552,7 +574,7 @@ struct fw_cnn {
   bf16 *a0 = nullptr, *a1 = nullptr, *a2 = nullptr, *a3 = nullptr;
   bf16 *g4 = nullptr, *g3 = nullptr, *g2 = nullptr, *g1 = nullptr;
   float *in = nullptr, *out = nullptr, *tgt = nullptr;
-  double *mean = nullptr;  // wet-cell mean of the eta correction
+  double *mean = nullptr;  // wet-cell mean of the eta correction, then its partial sums
   int conserve = 0;
   int adam_t = 0;
   std::string err;
@@ -627,7 +649,7 @@ int fw_cnn_create(int H, int W, int max_batch, fw_cnn **out) {
       (rc = cget(n, 9 * 512 * 2, &n->pk.b2)) || (rc = cget(n, 9 * 512 * 2, &n->pk.b3)) ||
       (rc = cget(n, 3 * 512 * 2, &n->pk.b4)) || (rc = cget(n, 32, &n->pk.bias1)) ||
       (rc = cget(n, 32, &n->pk.bias2)) || (rc = cget(n, 32, &n->pk.bias3)) || (rc = cget(n, 16, &n->pk.bias4)) ||
-      (rc = cget(n, 1, &n->mean)) ||
+      (rc = cget(n, 1 + 2 * kWetBlocks, &n->mean)) ||
       (rc = cget(n, px * 8, &n->a0)) || (rc = cget(n, px * kC, &n->a1)) || (rc = cget(n, px * kC, &n->a2)) ||
       (rc = cget(n, px * kC, &n->a3)) || (rc = cget(n, px * 8, &n->g4)) || (rc = cget(n, px * kC, &n->g3)) ||
       (rc = cget(n, px * kC, &n->g2)) || (rc = cget(n, px * kC, &n->g1)) ||
@@ -789,17 +811,19 @@ int fw_cnn_correct(fw_cnn *n, fw_ctx *solver, const float fs[4], const float os[
   forward(n, 1);
   n->stream = keep;
   const double *mean = n->conserve ? n->mean : nullptr;
+  auto wet_mean = [&](auto k) {
+    const int nb = Hs < kWetBlocks ? Hs : kWetBlocks;
+    hipLaunchKernelGGL(k, dim3(nb), dim3(256), 0, s, n->out, (const int *)mask, P, cfg.Ibeg, cfg.Jbeg, Hs, Ws, os[0],
+                       n->mean + 1);
+    hipLaunchKernelGGL(k_wet_mean, dim3(1), dim3(256), 0, s, (const double *)(n->mean + 1), nb, n->mean);
+  };
   if (cfg.real_bytes == 8) {
-    if (mean)
-      hipLaunchKernelGGL(k_wet_mean<double>, dim3(1), dim3(1024), 0, s, n->out, (const int *)mask, P, cfg.Ibeg,
-                         cfg.Jbeg, Hs, Ws, os[0], n->mean);
+    if (mean) wet_mean(k_wet_sum<double>);
     hipLaunchKernelGGL(k_correct<double>, g2, b2, 0, s, n->out, (double *)eta, (double *)u, (double *)v, (double *)h,
                        (double *)hu, (double *)hv, (double *)ub, (double *)vb, (const double *)dep, (const int *)mask,
                        P, cfg.Ibeg, cfg.Jbeg, Hs, Ws, os[0], os[1], os[2], cfg.Gamma3, cfg.MinDepthFrc, mean);
   } else {
-    if (mean)
-      hipLaunchKernelGGL(k_wet_mean<float>, dim3(1), dim3(1024), 0, s, n->out, (const int *)mask, P, cfg.Ibeg,
-                         cfg.Jbeg, Hs, Ws, os[0], n->mean);
+    if (mean) wet_mean(k_wet_sum<float>);
     hipLaunchKernelGGL(k_correct<float>, g2, b2, 0, s, n->out, (float *)eta, (float *)u, (float *)v, (float *)h,
                        (float *)hu, (float *)hv, (float *)ub, (float *)vb, (const float *)dep, (const int *)mask, P,
                        cfg.Ibeg, cfg.Jbeg, Hs, Ws, os[0], os[1], os[2], (float)cfg.Gamma3, (float)cfg.MinDepthFrc,
