@@ -185,8 +185,12 @@ __global__ void __launch_bounds__(WideLB<R>::wg512) kb_disp_terms(FWB_ARGS, int 
 }
 
 template <class R, bool P2>
-__global__ void __launch_bounds__(kDispTX * kDispTY) kb_disp_fused(FWB_ARGS, int pm, int pa) {
+__global__ void __launch_bounds__(kDispTX * kDispTY) kb_disp_fused(FWB_ARGS, int pm, int pa, int brk) {
   FWB_HEAD
+  if (e.x < 0) {  // the previous stage's brk2_fill, as in k_disp_fused
+    if (brk) brk2_fill_body<R>(mdev(M, pm ^ 1, pa ^ 1), M.g, M.p, M.clk[0], tile_blk(e));
+    return;
+  }
   disp_fused_body<R, P2>(mdev(M, pm, pa), M.g, M.p, M.clk[0], tile_blk(e));
 }
 
@@ -226,9 +230,9 @@ __global__ void __launch_bounds__(WideLB<R>::wg256) kb_huv(FWB_ARGS, int pm, int
 }
 
 template <class R>
-__global__ void __launch_bounds__(kTridThreads) kb_trid_fac(FWB_ARGS, int pm, int pa) {
+__global__ void __launch_bounds__(kTridThreads) kb_trid_fac(FWB_ARGS, int pm, int pa, int again) {
   FWB_HEAD
-  trid_fac_body<R>(mdev(M, pm, pa), M.g, M.p, e.aux, tile_blk(e));
+  trid_fac_body<R>(mdev(M, pm, pa), M.g, M.p, e.aux, again, tile_blk(e));
 }
 
 template <class R, bool RES, bool PER>
@@ -380,9 +384,9 @@ int upload_queue(fw_batch *b, Queue &Q) {
 }
 
 // 2-D tile queue: member m covers ceil(nx(m)/bx) x ceil(ny(m)/by) tiles; aux:
-// the tiles of a row
+// the tiles of a row; extra: one more entry per member, x = -1, ahead of them
 template <class FX, class FY>
-int make_tiles(fw_batch *b, const std::string &name, dim3 block, int bx, int by, FX nx, FY ny) {
+int make_tiles(fw_batch *b, const std::string &name, dim3 block, int bx, int by, FX nx, FY ny, bool extra = false) {
   Queue &Q = b->q[name];
   Q.h.clear();
   Q.block = block;
@@ -393,6 +397,8 @@ int make_tiles(fw_batch *b, const std::string &name, dim3 block, int bx, int by,
       for (int x = 0; x < tx; x++) Q.h.push_back(QEnt{m, x, y, tx});
   }
   xcd_order(Q.h);
+  if (extra)
+    for (int m = 0; m < b->n; m++) Q.h.insert(Q.h.begin(), QEnt{m, -1, 0, 0});
   return upload_queue(b, Q);
 }
 
@@ -517,7 +523,8 @@ int build_queues(fw_batch *b) {
   auto N_ = [](const Geo &g) { return g.N; };
   const dim3 sd = b->shape[G_DISP], sh = b->shape[G_HUV], sc = b->shape[G_CELL];
   if ((rc = make_tiles(b, "disp", sd, sd.x, sd.y, M_, N_))) return rc;
-  if ((rc = make_tiles(b, "dispf", dim3(kDispTX, kDispTY), kDispTX, kDispTY, M_, N_))) return rc;
+  // (and one workgroup per member for the previous stage's brk2_fill, first)
+  if ((rc = make_tiles(b, "dispf", dim3(kDispTX, kDispTY), kDispTX, kDispTY, M_, N_, true))) return rc;
   if ((rc = make_tiles(b, "huv", sh, sh.x, sh.y, M_, N_))) return rc;
   if ((rc = make_tiles(b, "cell", sc, sc.x, sc.y, M_, N_))) return rc;
   auto M1 = [](const Geo &g) { return g.M + 1; };
@@ -610,11 +617,11 @@ int rec_step(fw_batch *b, int p0, bool first) {
     if (fac) {  // beside the dispersion and the fluxes
       BCHK(b, hipEventRecord(b->ev_fork, s));
       BCHK(b, hipStreamWaitEvent(sd, b->ev_fork, 0));
-      bl<R>(b, sd, "trid_fac", kb_trid_fac<R>, par, par);
+      bl<R>(b, sd, "trid_fac", kb_trid_fac<R>, par, par, first && st == 1 && b->trid_fixed ? 1 : 0);
       BCHK(b, hipEventRecord(b->ev_fac, sd));
     }
     if (b->disp && !per) {
-      bl<R>(b, s, "dispf", kb_disp_fused<R, P2>, par, par);
+      bl<R>(b, s, "dispf", kb_disp_fused<R, P2>, par, par, st > 0 ? 1 : 0);
     } else if (b->disp) {
       bl<R>(b, s, "disp", kb_disp_deriv<R, P2>, par, par);
       bl<R>(b, s, "halo_d", kb_halo_per<R>, 1, par);
@@ -642,7 +649,7 @@ int rec_step(fw_batch *b, int p0, bool first) {
     }
     if (!per) {
       bl<R>(b, s, "tail", kb_tail<R, true>, par, par, st == 2 ? 1 : 0);
-      bl<R>(b, s, "one1024", kb_brk2_fill<R>, par, par);
+      if (st == 2 || !b->disp) bl<R>(b, s, "one1024", kb_brk2_fill<R>, par, par);
     } else {
       bl<R>(b, s, "tail", kb_tail<R, false>, par, par, 0);
       if (!b->disp) bl<R>(b, s, "copy", kb_ubar_from_hu<R>);

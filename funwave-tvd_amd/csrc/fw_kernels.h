@@ -936,10 +936,6 @@ __device__ __forceinline__ void disp_fused_body(Dev<R> d, Geo g, Prm<R> p, R DT,
     d.ETAy[o] = etay;
   }
 }
-template <class R, bool P2>
-__global__ void __launch_bounds__(kDispTX * kDispTY) k_disp_fused(Dev<R> d, Geo g, Prm<R> p, R DT, const R *dtp) {
-  disp_fused_body<R, P2>(d, g, p, dtp ? *dtp : DT, grid_blk());
-}
 
 // --------------------------------------------------------------------------
 // FLUXES (fluxes.F:52-117).  CONSTRUCT_HO_X/Y (:1531-1754): 4th-order
@@ -2129,8 +2125,13 @@ struct alignas(2 * sizeof(R)) FacOut {
   R c, den;
 };
 
+// again: the second stage of a call, which has nothing to do unless k_tail
+// changed MASK9 in the interior (flags[1]); the first one clears the mark
 template <class R>
-__device__ __forceinline__ void trid_fac_body(const Dev<R> &d, const Geo &g, const Prm<R> &p, int nxblk, const Blk &B) {
+__device__ __forceinline__ void trid_fac_body(const Dev<R> &d, const Geo &g, const Prm<R> &p, int nxblk, int again,
+                                              const Blk &B) {
+  if (again && !d.flags[1]) return;
+  if (!again && B.x == 0 && threadIdx.x == 0) d.flags[1] = 0;
   constexpr int L = kTridL, CH = kFacCH, PER = L * CH / kTridNS;
   __shared__ FacRow<R> in[2][L][CH + 1];
   __shared__ FacOut<R> out[2][L][CH + 1];
@@ -2211,8 +2212,8 @@ __device__ __forceinline__ void trid_fac_body(const Dev<R> &d, const Geo &g, con
   }
 }
 template <class R>
-__global__ void __launch_bounds__(kTridThreads) k_trid_fac(Dev<R> d, Geo g, Prm<R> p, int nxblk) {
-  trid_fac_body<R>(d, g, p, nxblk, grid_blk());
+__global__ void __launch_bounds__(kTridThreads) k_trid_fac(Dev<R> d, Geo g, Prm<R> p, int nxblk, int again) {
+  trid_fac_body<R>(d, g, p, nxblk, again, grid_blk());
 }
 
 // ---- d' and back substitution.
@@ -3156,6 +3157,7 @@ __global__ void k_brk1(Dev<R> d, Geo g, Prm<R> p, R DT) {
 template <class R>
 __device__ __forceinline__ void brk2_body(const Dev<R> &d, const Geo &g, const Prm<R> &p, R DT, const Blk &B) {
   __shared__ int changed;
+  const int tid = threadIdx.x + threadIdx.y * blockDim.x, nt = blockDim.x * blockDim.y;
   const int n = *d.cand_n;
   if (n == 0) return;
   // the dependency chains are at most n long, so n+1 sweeps reach the fixed point
@@ -3163,9 +3165,9 @@ __device__ __forceinline__ void brk2_body(const Dev<R> &d, const Geo &g, const P
   int it = 0;
   for (;;) {
     __syncthreads();
-    if (threadIdx.x == 0) changed = 0;
+    if (tid == 0) changed = 0;
     __syncthreads();
-    for (int k = threadIdx.x; k < n; k += blockDim.x) {
+    for (int k = tid; k < n; k += nt) {
       size_t o = (size_t)d.cand[k];
       int i = 1 + (int)(o % g.P), j = 1 + (int)(o / g.P);
       const R *ci = d.cinf + 8 * (size_t)k;
@@ -3180,12 +3182,12 @@ __device__ __forceinline__ void brk2_body(const Dev<R> &d, const Geo &g, const P
     __syncthreads();
     if (!changed) break;
     if (++it >= maxit) {
-      if (threadIdx.x == 0) d.flags[0] = 1;
+      if (tid == 0) d.flags[0] = 1;
       break;
     }
   }
   __syncthreads();
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
+  for (int k = tid; k < n; k += nt) {
     size_t o = (size_t)d.cand[k];
     int i = 1 + (int)(o % g.P), j = 1 + (int)(o / g.P);
     const R *ci = d.cinf + 8 * (size_t)k;
@@ -3194,7 +3196,7 @@ __device__ __forceinline__ void brk2_body(const Dev<R> &d, const Geo &g, const P
     d.nu_break[o] = brk_nu(p, g, b, i, j, d.AGEn[o], d.Depth[o], d.EtaW[o]);
   }
   __syncthreads();
-  if (threadIdx.x == 0) *d.cand_n = 0;
+  if (tid == 0) *d.cand_n = 0;
 }
 template <class R>
 __global__ void __launch_bounds__(1024) k_brk2(Dev<R> d, Geo g, Prm<R> p, R DT) {
@@ -3458,7 +3460,10 @@ __device__ __forceinline__ void tail_body(const Dev<R> &d, const Geo &g, const P
           if (ddiv(dabs(e0), rmax(h0, p.MDF)) > p.SWE) m9 = 0;
         }
       }
-      if (m9 != m9_old) d.MASK9[o] = m9;
+      if (m9 != m9_old) {
+        d.MASK9[o] = m9;
+        if (inner) d.flags[1] = 1;  // the line solves' c' are of the old one
+      }
       if (!FILL) d.MASKn[o] = m;
       if (brk) brk1_cell(d, g, p, DT, i, j, o, ring, age, et, h, h0, e0);
       if (inner) {
@@ -3549,17 +3554,18 @@ __device__ __forceinline__ void brk2_fill_body(const Dev<R> &d, const Geo &g, co
   if (p.SHOW_BRK) brk2_body<R>(d, g, p, DT, B);
   if (!p.VISC_BRK) return;
   __syncthreads();
+  const int tid = threadIdx.x + threadIdx.y * blockDim.x, nt = blockDim.x * blockDim.y;
   const HaloSpec s = halo_spec(g, 0);
   const int cnt = 6 * g.M + 6 * (g.Je - g.Jb + 1);
   R *arr[2] = {p.SHOW_BRK ? d.AGEn : d.AGE_BREAKING, d.nu_break};
   constexpr int K = 4;  // ghost cells of a thread in flight together
-  for (int t0 = threadIdx.x; t0 < cnt; t0 += K * blockDim.x) {
+  for (int t0 = tid; t0 < cnt; t0 += K * nt) {
     size_t dst[K];
     R va[K], vn[K];
 #pragma unroll
     for (int k = 0; k < K; k++) {
       int i, j;
-      const int t = min(t0 + k * (int)blockDim.x, cnt - 1);
+      const int t = min(t0 + k * nt, cnt - 1);
       halo_pos(s, t, 0, i, j);
       const int si = i < g.Ib ? 2 * g.Ib - 1 - i : (i > g.Ie ? 2 * g.Ie + 1 - i : i);
       const int sj = j < g.Jb ? 2 * g.Jb - 1 - j : (j > g.Je ? 2 * g.Je + 1 - j : j);
@@ -3569,7 +3575,7 @@ __device__ __forceinline__ void brk2_fill_body(const Dev<R> &d, const Geo &g, co
     }
 #pragma unroll
     for (int k = 0; k < K; k++) {
-      if (t0 + k * (int)blockDim.x >= cnt) continue;
+      if (t0 + k * nt >= cnt) continue;
       arr[0][dst[k]] = va[k];
       arr[1][dst[k]] = vn[k];
     }
@@ -3583,6 +3589,29 @@ __global__ void __launch_bounds__(1024) k_brk2_fill(Dev<R> d, Geo g, Prm<R> p, R
   __syncthreads();
   const R m = extreme1024<R, true>(d.red, nblk, (R)0);
   if (threadIdx.x == 0) publish(pub, (double)m, d.flags[0], seq);
+}
+
+// CAL_DISPERSION in one pass, and, with brk, the previous stage's
+// brk2_fill_body by one more workgroup, the first of the launch: the
+// dispersion reads neither ages nor viscosities, so the single workgroup that
+// would hold up the stream for 5 us (96 x 72) to 39 (2048 x 2048) runs beside it
+// (as the last workgroup it would end 30 us after the others at 2048 x 2048).
+// age, agen: the age buffers as that stage had them (they swap after it).
+template <class R, bool P2>
+__global__ void __launch_bounds__(kDispTX * kDispTY) k_disp_fused(Dev<R> d, Geo g, Prm<R> p, R DT, const R *dtp,
+                                                                  int brk, R *age, R *agen) {
+  const R dt = dtp ? *dtp : DT;
+  Blk B = grid_blk();
+  B.gy -= brk;
+  B.y -= brk;
+  if (B.y < 0) {
+    if (B.x != 0) return;
+    d.AGE_BREAKING = age;
+    d.AGEn = agen;
+    brk2_fill_body<R>(d, g, p, dt, B);
+    return;
+  }
+  disp_fused_body<R, P2>(d, g, p, dt, B);
 }
 
 // FP64 budget (mass, energy, extrema) over the interior.

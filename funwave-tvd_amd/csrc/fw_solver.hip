@@ -409,20 +409,22 @@ bool disp_one_pass(fw_ctx *c) {
 
 // in_step: called by fw_step, whose RK update forms the cross derivatives
 // (the per-routine ESTIMATE_HUV reads them from the arrays); dtp: DT on the
-// device, where the host does not have it yet
+// device, where the host does not have it yet; brk2: the last stage's
+// brk2_fill_body is still due
 template <class R>
-int do_dispersion(fw_ctx *c, bool in_step = false, const R *dtp = nullptr) {
+int do_dispersion(fw_ctx *c, bool in_step = false, const R *dtp = nullptr, bool brk2 = false) {
   Dev<R> &d = c->dev<R>();
   const Geo &g = c->g;
   if (disp_one_pass<R>(c)) {
     // one pass: the second derivatives stay in LDS (k_disp_fused)
-    const dim3 b(kDispTX, kDispTY), gr((g.M + kDispTX - 1) / kDispTX, (g.N + kDispTY - 1) / kDispTY);
+    const dim3 b(kDispTX, kDispTY), gr((g.M + kDispTX - 1) / kDispTX, (g.N + kDispTY - 1) / kDispTY + (brk2 ? 1 : 0));
     Prm<R> p = c->prm<R>();
     p.xd_in_huv = in_step ? 1 : 0;
-    if (spacing_pow2<R>(c))
-      launch(c, "disp", k_disp_fused<R, true>, gr, b, d, g, p, (R)c->dt, dtp);
-    else
-      launch(c, "disp", k_disp_fused<R, false>, gr, b, d, g, p, (R)c->dt, dtp);
+    // (the host has swapped the age buffers since that stage)
+    R *age = p.SHOW_BRK ? d.AGEn : d.AGE_BREAKING, *agen = p.SHOW_BRK ? d.AGE_BREAKING : d.AGEn;
+    auto go = [&](auto k) { launch(c, "disp", k, gr, b, d, g, p, (R)c->dt, dtp, brk2 ? 1 : 0, age, agen); };
+    if (spacing_pow2<R>(c)) go(k_disp_fused<R, true>);
+    else go(k_disp_fused<R, false>);
     return FW_OK;
   }
   if (spacing_pow2<R>(c))
@@ -530,8 +532,9 @@ bool factor_forks(fw_ctx *c) {
   const Geo &g = c->g;
   return std::max(g.Ie - g.Ib, c->cfg.PERIODIC ? 0 : g.Je - g.Jb) + 1 > kFacFork;
 }
+// again: the second stage of a call (k_trid_fac)
 template <class R>
-int fork_factor(fw_ctx *c) {
+int fork_factor(fw_ctx *c, bool again) {
   const TridGrid tg = trid_grid<R>(c->g, c->cfg.PERIODIC);
   const dim3 gr(tg.nx + (c->cfg.PERIODIC ? 0 : tg.ny));
   const bool fork = factor_forks<R>(c);
@@ -540,7 +543,8 @@ int fork_factor(fw_ctx *c) {
     HIPCHK(c, hipStreamWaitEvent(c->side, c->ev_fork, 0));
     c->cur = c->side;
   }
-  launch(c, "trid_fac", k_trid_fac<R>, gr, dim3(kTridThreads), c->dev<R>(), c->g, c->prm<R>(), tg.nx);
+  launch(c, "trid_fac", k_trid_fac<R>, gr, dim3(kTridThreads), c->dev<R>(), c->g, c->prm<R>(), tg.nx,
+         again ? 1 : 0);
   c->cur = c->stream;
   if (fork) HIPCHK(c, hipEventRecord(c->ev_fac, c->side));
   return FW_OK;
@@ -791,7 +795,7 @@ int do_step_routines(fw_ctx *c, int nsteps) {
     if ((rc = do_estimate_dt<R>(c, true))) return rc;
     for (int st = 1; st <= 3; st++) {
       const bool fac = f.DISPERSION && (3 * s + st <= 2 || !trid_fixed(c->prm<R>()));
-      if (fac && (rc = fork_factor<R>(c))) return rc;
+      if (fac && (rc = fork_factor<R>(c, false))) return rc;
       if (f.DISPERSION && (rc = do_dispersion<R>(c, true))) return rc;
       if ((rc = do_fluxes<R>(c))) return rc;
       if (fac && (rc = join_factor<R>(c))) return rc;
@@ -833,8 +837,8 @@ int do_step_prod(fw_ctx *c, int nsteps) {
   const Prm<R> &p = c->prm<R>();
   const bool per = f.PERIODIC, sponge = f.DIRECT_SPONGE;
   const dim3 gb = grid2(g.M, g.N, kB2), gt = grid2(g.M + 1, g.N + 1, kB2);
-  // the breaking ages' ghost cells by the one workgroup of k_brk2_fill, or, on
-  // a longer boundary, by a launch of their own (96 x 72: 5.6 us against 4 + 4;
+  // the last stage's breaking ages' ghost cells by the one workgroup of
+  // k_brk2_fill, or, on a longer boundary, by a launch of their own (96 x 72: 5.6 us against 4 + 4;
   // 777 x 601: 11.5 against 4 + 4; 2048 x 2048: 39 against 5 + 5)
   const bool one_fill = 6 * (g.M + g.N) <= 4096;
   struct EtaW {  // the RK update leaves Eta in a plane of its own
@@ -857,10 +861,12 @@ int do_step_prod(fw_ctx *c, int nsteps) {
     }
     launch(c, "dt_final", k_dt_pub<R>, dim3(1), dim3(1024), d, p, nblk, (R *)c->scal, c->pub_dev, seq);
     R AA = (R)0;
+    bool brk2_due = false;
     for (int st = 1; st <= 3; st++) {
       const bool fac = f.DISPERSION && (3 * s + st <= 2 || !trid_fixed(p));
-      if (fac && (rc = fork_factor<R>(c))) return rc;
-      if (f.DISPERSION && (rc = do_dispersion<R>(c, true, st == 1 ? (const R *)c->scal : nullptr))) return rc;
+      if (fac && (rc = fork_factor<R>(c, 3 * s + st == 2 && trid_fixed(p)))) return rc;
+      if (f.DISPERSION && (rc = do_dispersion<R>(c, true, st == 1 ? (const R *)c->scal : nullptr, brk2_due))) return rc;
+      brk2_due = false;
       if ((rc = do_fluxes<R>(c))) return rc;
       if (st == 1) {
         if ((rc = wait_pub(c, c->pub, seq))) return rc;
@@ -876,7 +882,9 @@ int do_step_prod(fw_ctx *c, int nsteps) {
       Pub *pub = last ? c->pub_dev + 1 : nullptr;
       if (!per) {
         launch(c, "tail", k_tail<R, true>, gt, kB2, d, g, p, (R)c->dt, sponge ? 1 : 0, last ? 1 : 0);
-        if (one_fill) {
+        if (!last && f.DISPERSION) {
+          brk2_due = p.SHOW_BRK || p.VISC_BRK;  // beside the next stage's dispersion
+        } else if (one_fill) {
           if (last || p.SHOW_BRK || p.VISC_BRK)
             launch(c, "brk2", k_brk2_fill<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt, (int)(gt.x * gt.y), pub, seq);
         } else {
