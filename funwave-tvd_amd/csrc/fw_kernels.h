@@ -235,7 +235,7 @@ __global__ void k_halo_per(HaloList L, HaloList Lf, Geo g) {
 
 // --------------------------------------------------------------------------
 // ESTIMATE_DT (misc.F:216-296) over all cells including ghosts; the block
-// minima are reduced by k_dt_final.  Also U0 := U, V0 := V (main.F:331-332)
+// minima are reduced by k_dt_pub.  Also U0 := U, V0 := V (main.F:331-332)
 // when copy_uv is set.
 template <class R>
 __device__ __forceinline__ void dt_partial_body(Dev<R> d, Geo g, Prm<R> p, int copy_uv, const Blk &B) {
@@ -290,23 +290,6 @@ __device__ __forceinline__ R dt_of(const Prm<R> &p, R least) {
   R dt = p.DTF;
   while (dt > dtt) dt = ddiv(dt, (R)2);
   return dt;
-}
-template <class R>
-__device__ __forceinline__ void dt_final_body(Dev<R> d, Prm<R> p, int nblk, R *out, const Blk &B) {
-  __shared__ R sm[256];
-  R m = Lit<R>::large();
-  for (int q = threadIdx.x; q < nblk; q += blockDim.x) m = rmin(m, d.red[q]);
-  sm[threadIdx.x] = m;
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sm[threadIdx.x] = rmin(sm[threadIdx.x], sm[threadIdx.x + s]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[0] = dt_of(p, sm[0]);
-}
-template <class R>
-__global__ void k_dt_final(Dev<R> d, Prm<R> p, int nblk, R *out) {
-  dt_final_body<R>(d, p, nblk, out, grid_blk());
 }
 // A value handed to the host through pinned memory: the host spins on seq
 // (a few us) instead of a copy and a stream synchronisation (12 us).
@@ -384,23 +367,6 @@ __global__ void k_maxeta_partial(Dev<R> d, Geo g) {
   maxeta_partial_body<R>(d, g, grid_blk());
 }
 template <class R>
-__device__ __forceinline__ void max_final_body(Dev<R> d, int nblk, R *out, const Blk &B) {
-  __shared__ R sm[256];
-  R m = (R)0;
-  for (int q = threadIdx.x; q < nblk; q += blockDim.x) m = rmax(m, d.red[q]);
-  sm[threadIdx.x] = m;
-  __syncthreads();
-  for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sm[threadIdx.x] = rmax(sm[threadIdx.x], sm[threadIdx.x + s]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[0] = sm[0];
-}
-template <class R>
-__global__ void k_max_final(Dev<R> d, int nblk, R *out) {
-  max_final_body<R>(d, nblk, out, grid_blk());
-}
-template <class R>
 __global__ void __launch_bounds__(1024) k_max_pub(Dev<R> d, int nblk, Pub *pub, unsigned seq) {
   const R m = extreme1024<R, true>(d.red, nblk, (R)0);
   if (threadIdx.x == 0) publish(pub, (double)m, d.flags[0], seq);
@@ -427,6 +393,26 @@ __global__ void k_copy3(R *d0, const R *s0, R *d1, const R *s1, R *d2, const R *
     d1[q] = s1[q];
     d2[q] = s2[q];
   }
+}
+
+template <class R>
+__global__ void k_copy2(R *d0, const R *s0, R *d1, const R *s1, size_t n) {
+  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x) {
+    d0[q] = s0[q];
+    d1[q] = s1[q];
+  }
+}
+
+// The wavemaker factors of a stage, up to 2 KB of them, handed over as a kernel
+// argument: a launch (3.5 us) instead of a copy, an event and its wait (13).
+template <class R>
+struct WkArg {
+  static constexpr int cap = 2048 / sizeof(R);
+  R v[cap];
+};
+template <class R>
+__global__ void __launch_bounds__(512) k_wk_stage(WkArg<R> a, int n, R *dst) {
+  for (int k = threadIdx.x; k < n; k += blockDim.x) dst[k] = a.v[k];
 }
 
 // --------------------------------------------------------------------------
@@ -3199,8 +3185,11 @@ __device__ __forceinline__ void brk2_body(const Dev<R> &d, const Geo &g, const P
   if (tid == 0) *d.cand_n = 0;
 }
 template <class R>
-__global__ void __launch_bounds__(1024) k_brk2(Dev<R> d, Geo g, Prm<R> p, R DT) {
+__global__ void __launch_bounds__(1024) k_brk2(Dev<R> d, Geo g, Prm<R> p, R DT, Pub *pub, unsigned seq) {
   brk2_body<R>(d, g, p, DT, grid_blk());
+  if (!pub) return;
+  __syncthreads();
+  if (threadIdx.x == 0) publish(pub, 0.0, d.flags[0], seq);
 }
 
 // --------------------------------------------------------------------------

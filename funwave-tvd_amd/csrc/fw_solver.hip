@@ -223,10 +223,10 @@ int alloc_state(fw_ctx *c) {
   size_t stage_elems = (size_t)(N + 8) > (size_t)(2 * nfreq + 8) ? (size_t)(N + 8) : (size_t)(2 * nfreq + 8);
   if ((rc = get(stage_elems * sizeof(R), (void **)&d.wk_stage)) != FW_OK) return rc;
   c->slot_bytes = (stage_elems * sizeof(R) + 255) & ~(size_t)255;
-  HIPCHK(c, hipHostMalloc((void **)&c->pinned, c->slot_bytes * (kStageSlots + 1) + 4096));
-  HIPCHK(c, hipHostMalloc((void **)&c->pub, 2 * sizeof(Pub), hipHostMallocMapped | hipHostMallocCoherent));
+  HIPCHK(c, hipHostMalloc((void **)&c->pinned, c->slot_bytes * kStageSlots));
+  HIPCHK(c, hipHostMalloc((void **)&c->pub, 3 * sizeof(Pub), hipHostMallocMapped | hipHostMallocCoherent));
   HIPCHK(c, hipHostGetDevicePointer((void **)&c->pub_dev, c->pub, 0));
-  memset(c->pub, 0, 2 * sizeof(Pub));
+  memset(c->pub, 0, 3 * sizeof(Pub));
   for (int k = 0; k < kStageSlots; k++) HIPCHK(c, hipEventCreateWithFlags(&c->slot_ev[k], hipEventDisableTiming));
   // MASK_STRUC defaults to 1 (no structures); MASK9 / MASK to 1 until uploaded
   return FW_OK;
@@ -283,7 +283,8 @@ template int wavemaker_factors<double>(fw_ctx *, double, double &, double *, siz
 
 namespace {
 
-// per-stage factors: returns AA; queues the copy of the row/frequency table
+// The wavemaker factors at the current TIME: returns AA and queues the row or
+// frequency table's way to the device.
 template <class R>
 int stage_wavemaker(fw_ctx *c, R &AA) {
   AA = (R)0;
@@ -291,29 +292,37 @@ int stage_wavemaker(fw_ctx *c, R &AA) {
   int rc = prepare_wavemaker<R>(c);
   if (rc) return rc;
   const R T = (R)c->time;
+  const fw_config &f = c->cfg;
+  size_t n = 0;
+  // (as many factors as wavemaker_factors forms)
+  const int cnt = f.wavemaker == FW_WK_REG ? std::max(0, f.jhi - f.jlo + 1) : 2 * f.NumFreq;
+  if (cnt <= WkArg<R>::cap) {
+    WkArg<R> a;
+    if ((rc = wavemaker_factors<R>(c, T, AA, a.v, &n))) return rc;
+    if (n) launch(c, "wk_stage", k_wk_stage<R>, dim3(1), dim3(512), a, (int)n, c->dev<R>().wk_stage);
+    return FW_OK;
+  }
   int slot = c->slot_next;
   c->slot_next = (c->slot_next + 1) % kStageSlots;
   HIPCHK(c, hipEventSynchronize(c->slot_ev[slot]));
   R *h = (R *)(c->pinned + (size_t)slot * c->slot_bytes);
-  size_t n = 0;
   if ((rc = wavemaker_factors<R>(c, T, AA, h, &n))) return rc;
   HIPCHK(c, hipMemcpyAsync(c->dev<R>().wk_stage, h, n * sizeof(R), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipEventRecord(c->slot_ev[slot], c->stream));
   return FW_OK;
 }
 
-// the factors of a whole step, formed once (TIME stays the same over its
-// stages); the pinned slot is free again when the step has ended
-template <class R>
-int step_wavemaker(fw_ctx *c, R &AA) {
-  AA = (R)0;
-  if (c->cfg.wavemaker == FW_WK_NONE) return FW_OK;
-  int rc = prepare_wavemaker<R>(c);
-  if (rc) return rc;
-  R *h = (R *)(c->pinned + (size_t)kStageSlots * c->slot_bytes + 4096);
-  size_t n = 0;
-  if ((rc = wavemaker_factors<R>(c, (R)c->time, AA, h, &n))) return rc;
-  if (n) HIPCHK(c, hipMemcpyAsync(c->dev<R>().wk_stage, h, n * sizeof(R), hipMemcpyHostToDevice, c->stream));
+// The host's side of publish(): spins until the kernel has stored seq.  A wait
+// longer than 20 ms goes to the stream, whose error it then reports.
+int wait_pub(fw_ctx *c, const Pub *p, unsigned seq) {
+  const auto t0 = std::chrono::steady_clock::now();
+  while (__atomic_load_n(&p->seq, __ATOMIC_ACQUIRE) != seq) {
+    for (int k = 0; k < 32; k++) __builtin_ia32_pause();
+    if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20)) {
+      HIPCHK(c, hipStreamSynchronize(c->stream));
+      if (__atomic_load_n(&p->seq, __ATOMIC_ACQUIRE) != seq) return fail(c, FW_E_HIP, "a step kernel did not finish");
+    }
+  }
   return FW_OK;
 }
 
@@ -377,11 +386,12 @@ int do_estimate_dt(fw_ctx *c, bool copy_uv) {
   long ncell = (long)c->g.M * c->g.N;
   if ((ncell + 255) / 256 < nblk) nblk = (int)((ncell + 255) / 256);
   launch(c, "dt_partial", k_dt_partial<R>, dim3(nblk), dim3(256), d, c->g, c->prm<R>(), copy_uv ? 1 : 0);
-  launch(c, "dt_final", k_dt_final<R>, dim3(1), dim3(256), d, c->prm<R>(), nblk, (R *)c->scal);
-  R *h = (R *)(c->pinned + (size_t)kStageSlots * c->slot_bytes);
-  HIPCHK(c, hipMemcpyAsync(h, c->scal, sizeof(R), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  R dt = h[0];
+  const unsigned seq = ++c->pub_seq;
+  launch(c, "dt_final", k_dt_pub<R>, dim3(1), dim3(1024), d, c->prm<R>(), nblk, (R *)c->scal, c->pub_dev, seq);
+  HIPCHK(c, hipGetLastError());
+  int rc = wait_pub(c, c->pub, seq);
+  if (rc) return rc;
+  const R dt = (R)c->pub[0].val;
   c->dt = (double)dt;
   c->time = (double)((R)c->time + dt);
   return FW_OK;
@@ -392,11 +402,12 @@ int do_max_eta(fw_ctx *c, double *out) {
   Dev<R> &d = c->dev<R>();
   int nblk = 256;
   launch(c, "maxeta", k_maxeta_partial<R>, dim3(nblk), dim3(256), d, c->g);
-  launch(c, "max_final", k_max_final<R>, dim3(1), dim3(256), d, nblk, (R *)c->scal + 1);
-  R *h = (R *)(c->pinned + (size_t)kStageSlots * c->slot_bytes) + 2;
-  HIPCHK(c, hipMemcpyAsync(h, (R *)c->scal + 1, sizeof(R), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  *out = (double)h[0];
+  const unsigned seq = ++c->pub_seq;
+  launch(c, "max_final", k_max_pub<R>, dim3(1), dim3(1024), d, nblk, c->pub_dev + 1, seq);
+  HIPCHK(c, hipGetLastError());
+  int rc = wait_pub(c, c->pub + 1, seq);
+  if (rc) return rc;
+  *out = c->pub[1].val;
   return FW_OK;
 }
 
@@ -573,7 +584,7 @@ int do_huv(fw_ctx *c, int istage) {
 template <class R>
 int do_mask(fw_ctx *c);
 template <class R>
-int do_breaking(fw_ctx *c);
+int do_breaking(fw_ctx *c, Pub *pub = nullptr, unsigned seq = 0);
 template <class R>
 int do_roller(fw_ctx *c);
 
@@ -739,13 +750,14 @@ int do_mask(fw_ctx *c) {
   return FW_OK;
 }
 
+// pub: the breaking flag goes to the host as pub[2] under seq
 template <class R>
-int do_breaking(fw_ctx *c) {
+int do_breaking(fw_ctx *c, Pub *pub, unsigned seq) {
   if (!c->cfg.SHOW_BREAKING) return FW_OK;
   Dev<R> &d = c->dev<R>();
   const Geo &g = c->g;
   launch(c, "brk1", k_brk1<R>, grid2(g.M, g.N, kBT), kBT, d, g, c->prm<R>(), (R)c->dt);
-  launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, c->prm<R>(), (R)c->dt);
+  launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, c->prm<R>(), (R)c->dt, pub, seq);
   std::swap(d.AGE_BREAKING, d.AGEn);
   return FW_OK;
 }
@@ -810,20 +822,6 @@ int do_step_routines(fw_ctx *c, int nsteps) {
   return FW_OK;
 }
 
-// The host's side of publish(): spins until the kernel has stored seq.  A wait
-// longer than 20 ms goes to the stream, whose error it then reports.
-int wait_pub(fw_ctx *c, const Pub *p, unsigned seq) {
-  const auto t0 = std::chrono::steady_clock::now();
-  while (__atomic_load_n(&p->seq, __ATOMIC_ACQUIRE) != seq) {
-    for (int k = 0; k < 32; k++) __builtin_ia32_pause();
-    if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20)) {
-      HIPCHK(c, hipStreamSynchronize(c->stream));
-      if (__atomic_load_n(&p->seq, __ATOMIC_ACQUIRE) != seq) return fail(c, FW_E_HIP, "a step kernel did not finish");
-    }
-  }
-  return FW_OK;
-}
-
 // Whole steps of the production path.  One stream: k_begin and k_dt_pub, then
 // per stage the dispersion, the fluxes, the RK update, the line solves and
 // k_tail.  The first stage's dispersion and fluxes are queued before the host
@@ -873,7 +871,7 @@ int do_step_prod(fw_ctx *c, int nsteps) {
         const R dt = (R)c->pub[0].val;
         c->dt = (double)dt;
         c->time = (double)((R)c->time + dt);
-        if ((rc = step_wavemaker<R>(c, AA))) return rc;
+        if ((rc = stage_wavemaker<R>(c, AA))) return rc;
       }
       if (fac && (rc = join_factor<R>(c))) return rc;
       launch_src_huv<R>(c, st, AA);
@@ -888,7 +886,7 @@ int do_step_prod(fw_ctx *c, int nsteps) {
           if (last || p.SHOW_BRK || p.VISC_BRK)
             launch(c, "brk2", k_brk2_fill<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt, (int)(gt.x * gt.y), pub, seq);
         } else {
-          if (p.SHOW_BRK) launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt);
+          if (p.SHOW_BRK) launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt, (Pub *)nullptr, 0u);
           HaloList L{}, Lf{};
           if (p.VISC_BRK) {
             hadd(L, p.SHOW_BRK ? d.AGEn : d.AGE_BREAKING, 1);
@@ -900,7 +898,7 @@ int do_step_prod(fw_ctx *c, int nsteps) {
       } else {
         launch(c, "tail", k_tail<R, false>, gt, kB2, d, g, p, (R)c->dt, 0, 0);
         if (!f.DISPERSION) launch(c, "ubar_hu", k_ubar_from_hu<R>, dim3(1024), dim3(256), d, plane_elems(g));
-        if (p.SHOW_BRK) launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt);
+        if (p.SHOW_BRK) launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt, (Pub *)nullptr, 0u);
       }
       std::swap(d.MASK, d.MASKn);
       if (p.SHOW_BRK) std::swap(d.AGE_BREAKING, d.AGEn);
@@ -1262,25 +1260,27 @@ int fw_estimate_dt(fw_ctx *c, double *dt, double *time) {
   if (time) *time = c->time;
   return c->prof ? collect_profile(c) : FW_OK;
 }
-int fw_save_stage0(fw_ctx *c, int which) {
-  if (!c) return FW_E_INVALID;
+}  // extern "C"
+
+namespace {
+template <class R>
+int do_save_stage0(fw_ctx *c, int which) {
+  Dev<R> &d = c->dev<R>();
   const size_t pe = plane_elems(c->g);
-  size_t bytes = pe * c->rb;
-  if (which == 1) {
-    void *e0 = field_ptr(c, F_Eta0), *e = field_ptr(c, F_Eta);
-    void *u0 = field_ptr(c, F_Ubar0), *u = field_ptr(c, F_Ubar);
-    void *v0 = field_ptr(c, F_Vbar0), *v = field_ptr(c, F_Vbar);
-    HIPCHK(c, hipMemcpyAsync(e0, e, bytes, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(u0, u, bytes, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(v0, v, bytes, hipMemcpyDeviceToDevice, c->stream));
-  } else if (which == 2) {
-    HIPCHK(c, hipMemcpyAsync(field_ptr(c, F_U0), field_ptr(c, F_U), bytes, hipMemcpyDeviceToDevice, c->stream));
-    HIPCHK(c, hipMemcpyAsync(field_ptr(c, F_V0), field_ptr(c, F_V), bytes, hipMemcpyDeviceToDevice, c->stream));
-  } else {
+  const dim3 gr((unsigned)std::min<size_t>(2048, (pe + 255) / 256)), b(256);
+  if (which == 1)
+    launch(c, "copy3", k_copy3<R>, gr, b, d.Eta0, (const R *)d.Eta, d.Ubar0, (const R *)d.Ubar, d.Vbar0,
+           (const R *)d.Vbar, pe);
+  else if (which == 2)
+    launch(c, "copy2", k_copy2<R>, gr, b, d.U0, (const R *)d.U, d.V0, (const R *)d.V, pe);
+  else
     return fail(c, FW_E_INVALID, "which must be 1 or 2");
-  }
   return FW_OK;
 }
+}  // namespace
+
+extern "C" {
+int fw_save_stage0(fw_ctx *c, int which) { ENTRY(c, DISPATCH(c, do_save_stage0)(c, which)); }
 int fw_cal_dispersion(fw_ctx *c) { ENTRY(c, c->rb == 8 ? do_dispersion<double>(c) : do_dispersion<float>(c)); }
 int fw_fluxes(fw_ctx *c) { ENTRY(c, DISPATCH(c, do_fluxes)(c)); }
 int fw_source_terms(fw_ctx *c) { ENTRY(c, DISPATCH(c, do_sources)(c)); }
@@ -1288,10 +1288,15 @@ int fw_estimate_huv(fw_ctx *c, int istage) { ENTRY(c, DISPATCH(c, do_huv)(c, ist
 int fw_update_mask(fw_ctx *c) { ENTRY(c, DISPATCH(c, do_mask)(c)); }
 int fw_wave_breaking(fw_ctx *c) {
   if (!c) return FW_E_INVALID;
-  int rc = DISPATCH(c, do_breaking)(c);
+  const unsigned seq = ++c->pub_seq;
+  int rc = c->rb == 8 ? do_breaking<double>(c, c->pub_dev + 2, seq) : do_breaking<float>(c, c->pub_dev + 2, seq);
   if (rc == FW_OK) rc = DISPATCH(c, do_roller)(c);
   if (rc) return rc;
-  if ((rc = read_break_flag(c, c->rb == 8 ? (void *)c->dd.flags : (void *)c->df.flags))) return rc;
+  if (c->cfg.SHOW_BREAKING) {
+    HIPCHK(c, hipGetLastError());
+    if ((rc = wait_pub(c, c->pub + 2, seq))) return rc;
+    if (c->pub[2].flag && (rc = read_break_flag(c, c->rb == 8 ? (void *)c->dd.flags : (void *)c->df.flags))) return rc;
+  }
   return c->prof ? collect_profile(c) : FW_OK;
 }
 int fw_sponge_damping(fw_ctx *c) { ENTRY(c, DISPATCH(c, do_sponge_only)(c)); }
