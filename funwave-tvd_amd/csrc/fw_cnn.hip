@@ -26,6 +26,7 @@
 #include <string>
 #include <vector>
 
+#include "fw_staging.h"
 #include "fwcnn.h"
 
 namespace fwl {
@@ -267,6 +268,7 @@ __global__ void k_loss(const float *__restrict__ out, const float *__restrict__ 
 // k_reduce_adam adds them.  All four layers are one launch (blockIdx.y).
 // 16 samples of 64 x 64: fp32 loops on one LDS element at a time took 286 us
 // and their serial reductions, Adam and repacking 248; now 23 and 5.
+constexpr int kGradPitch = (kNP + 63) / 64 * 64;  // the loss partials follow the gradient
 constexpr int kWgPx = 72;    // LDS pixels per channel row
 constexpr int kWgMax = 128;  // workgroups per layer (partial sums)
 template <int CIN, int GC>
@@ -568,7 +570,7 @@ struct fw_cnn {
   Grid g{};
   hipStream_t stream = nullptr;
   std::vector<void *> allocs;
-  float *params = nullptr, *am = nullptr, *av = nullptr, *grad = nullptr, *part = nullptr, *lpart = nullptr;
+  float *params = nullptr, *am = nullptr, *av = nullptr, *grad = nullptr, *part = nullptr;
   size_t part_len = 0;
   Packs pk{};
   bf16 *a0 = nullptr, *a1 = nullptr, *a2 = nullptr, *a3 = nullptr;
@@ -577,6 +579,7 @@ struct fw_cnn {
   double *mean = nullptr;  // wet-cell mean of the eta correction, then its partial sums
   int conserve = 0;
   int adam_t = 0;
+  fws::Staging stg;  // host arrays
   std::string err;
 };
 
@@ -643,7 +646,7 @@ int fw_cnn_create(int H, int W, int max_batch, fw_cnn **out) {
   n->part_len = (size_t)kWgMax * kNP;
   int rc;
   if ((rc = cget(n, kNP, &n->params)) || (rc = cget(n, kNP, &n->am)) || (rc = cget(n, kNP, &n->av)) ||
-      (rc = cget(n, kNP, &n->grad)) || (rc = cget(n, n->part_len, &n->part)) || (rc = cget(n, 4096, &n->lpart)) ||
+      (rc = cget(n, kGradPitch + 4096, &n->grad)) || (rc = cget(n, n->part_len, &n->part)) ||
       (rc = cget(n, 3 * 512 * 2, &n->pk.f1)) || (rc = cget(n, 9 * 512 * 2, &n->pk.f2)) ||
       (rc = cget(n, 9 * 512 * 2, &n->pk.f3)) || (rc = cget(n, 9 * 512 * 1, &n->pk.f4)) ||
       (rc = cget(n, 9 * 512 * 2, &n->pk.b2)) || (rc = cget(n, 9 * 512 * 2, &n->pk.b3)) ||
@@ -667,6 +670,7 @@ int fw_cnn_destroy(fw_cnn *n) {
   if (!n) return FW_E_INVALID;
   if (n->stream) (void)hipStreamSynchronize(n->stream);
   for (void *p : n->allocs) (void)hipFree(p);
+  n->stg.release();
   if (n->stream) (void)hipStreamDestroy(n->stream);
   delete n;
   return FW_OK;
@@ -695,17 +699,23 @@ int fw_cnn_get_params(fw_cnn *n, float *p, int count) {
   return FW_OK;
 }
 
+// host arrays (fw_staging.h)
+static hipError_t upload(fw_cnn *n, float *dst, const float *src, size_t planes) {
+  return n->stg.up((uint32_t *)dst, n->W, (const uint32_t *)src, n->W, planes * n->H, n->stream);
+}
+static hipError_t download(fw_cnn *n, float *dst, const float *src, uint32_t w, size_t h) {
+  return n->stg.down((uint32_t *)dst, (const uint32_t *)src, w, w, h, n->stream);
+}
+
 int fw_cnn_forward(fw_cnn *n, const float *in, float *out, int B) {
   int rc = check_batch(n, B);
   if (rc) return rc;
   if (!in || !out) return cfail(n, FW_E_INVALID, "null buffer");
-  const size_t plane = (size_t)B * n->H * n->W;
-  CHK(n, hipMemcpyAsync(n->in, in, plane * kCin * sizeof(float), hipMemcpyHostToDevice, n->stream));
+  CHK(n, upload(n, n->in, in, (size_t)kCin * B));
   hipLaunchKernelGGL(k_pack_input, dim3(1024), dim3(256), 0, n->stream, n->in, n->a0, n->g, B);
   forward(n, B);
   CHK(n, hipGetLastError());
-  CHK(n, hipMemcpyAsync(out, n->out, plane * kCout * sizeof(float), hipMemcpyDeviceToHost, n->stream));
-  CHK(n, hipStreamSynchronize(n->stream));
+  CHK(n, download(n, out, n->out, n->W, (size_t)kCout * B * n->H));
   return FW_OK;
 }
 
@@ -714,12 +724,12 @@ int fw_cnn_train_step(fw_cnn *n, const float *in, const float *target, int B, fl
   if (rc) return rc;
   if (!in || !target) return cfail(n, FW_E_INVALID, "null buffer");
   const size_t plane = (size_t)B * n->H * n->W;
-  CHK(n, hipMemcpyAsync(n->in, in, plane * kCin * sizeof(float), hipMemcpyHostToDevice, n->stream));
-  CHK(n, hipMemcpyAsync(n->tgt, target, plane * kCout * sizeof(float), hipMemcpyHostToDevice, n->stream));
+  CHK(n, upload(n, n->in, in, (size_t)kCin * B));
+  CHK(n, upload(n, n->tgt, target, (size_t)kCout * B));
   hipLaunchKernelGGL(k_pack_input, dim3(1024), dim3(256), 0, n->stream, n->in, n->a0, n->g, B);
   forward(n, B);
   const int nlb = 1024;
-  hipLaunchKernelGGL(k_loss, dim3(nlb), dim3(256), 0, n->stream, n->out, n->tgt, n->g4, n->lpart, n->g, B,
+  hipLaunchKernelGGL(k_loss, dim3(nlb), dim3(256), 0, n->stream, n->out, n->tgt, n->g4, n->grad + kGradPitch, n->g, B,
                      1.f / (float)(plane * kCout));
   // data gradients through layers 4, 3, 2 (ReLU masks from the activations)
   const dim3 gr = conv_grid(n, B), bl(256);
@@ -738,13 +748,14 @@ int fw_cnn_train_step(fw_cnn *n, const float *in, const float *target, int B, fl
   hipLaunchKernelGGL(k_reduce_adam, dim3((kNP + 31) / 32), dim3(256), 0, n->stream, n->part, nwg, n->grad, n->params,
                      n->am, n->av, lr, c1, c2, n->pk);
   CHK(n, hipGetLastError());
-  if (grad) CHK(n, hipMemcpyAsync(grad, n->grad, kNP * sizeof(float), hipMemcpyDeviceToHost, n->stream));
-  std::vector<float> lp(nlb);
-  CHK(n, hipMemcpyAsync(lp.data(), n->lpart, nlb * sizeof(float), hipMemcpyDeviceToHost, n->stream));
-  CHK(n, hipStreamSynchronize(n->stream));
+  // the loss partials and, in front of them, the gradient, in one copy
+  std::vector<float> res(kGradPitch + nlb);
+  const size_t off = grad ? 0 : kGradPitch;
+  CHK(n, download(n, res.data() + off, n->grad + off, (uint32_t)(res.size() - off), 1));
+  if (grad) memcpy(grad, res.data(), kNP * sizeof(float));
   if (loss) {
     double s = 0;
-    for (float v : lp) s += v;
+    for (int k = 0; k < nlb; k++) s += res[kGradPitch + k];
     *loss = (float)(s / (double)(plane * kCout));
   }
   return FW_OK;

@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "fw_kernels.h"
+#include "fw_staging.h"
 #include "fwgpu.h"
 
 namespace fwi {
@@ -75,6 +76,7 @@ struct fw_ctx {
   size_t slot_bytes = 0;
   hipEvent_t slot_ev[kStageSlots]{};
   int slot_next = 0;
+  fws::Staging stg;      // fw_upload, fw_download
   void *scal = nullptr;  // device scalars
   // values the step kernels hand to the host: [0] DT, [1] max |eta| and the
   // breaking flag (pinned memory, as the host and as the device see it)

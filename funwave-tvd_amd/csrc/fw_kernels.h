@@ -372,19 +372,6 @@ __global__ void __launch_bounds__(1024) k_max_pub(Dev<R> d, int nblk, Pub *pub, 
   if (threadIdx.x == 0) publish(pub, (double)m, d.flags[0], seq);
 }
 
-// w x h elements between arrays of different pitch (fw_upload, fw_download).
-// The runtime's own pitched copy to or from pageable host memory goes row by
-// row (0.6 GB/s at 1024 x 768); a dense one runs at about 20 GB/s, so fields
-// are made dense on the device first (four fields and the budget of 1024 x 768
-// cells: 21.7 -> 1.07 ms).
-template <class T>
-__global__ void __launch_bounds__(256) k_rows(T *__restrict__ dst, size_t dp, const T *__restrict__ src, size_t sp,
-                                              int w, int h) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= w) return;
-  for (int j = blockIdx.y; j < h; j += gridDim.y) dst[j * dp + i] = src[j * sp + i];
-}
-
 // plain copies of whole pitched arrays (Eta0 := Eta etc.)
 template <class R>
 __global__ void k_copy3(R *d0, const R *s0, R *d1, const R *s1, R *d2, const R *s2, size_t n) {

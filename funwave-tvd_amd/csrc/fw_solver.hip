@@ -1090,6 +1090,7 @@ int fw_destroy(fw_ctx *c) {
   for (void *p : c->allocs) (void)hipFree(p);
   if (c->pinned) (void)hipHostFree(c->pinned);
   if (c->pub) (void)hipHostFree(c->pub);
+  c->stg.release();
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
   if (c->ev_fac) (void)hipEventDestroy(c->ev_fac);
@@ -1152,28 +1153,13 @@ static int transfer(fw_ctx *c, int id, void *host, bool up) {
     if (k == K_XFACE) w += 1;
     if (k == K_YFACE) h += 1;
     void *dp = field_ptr(c, id);
-    // through a dense plane of the solver's scratch (the periodic line solves'
-    // y1, which holds nothing between calls)
-    void *dense = c->rb == 8 ? (void *)c->dd.y1 : (void *)c->df.y1;
-    const size_t bytes = (size_t)w * h * es;
-    const dim3 gr((w + 255) / 256, std::min(h, 32768)), b(256);
-    auto rows = [&](void *dst, size_t dpitch, const void *src, size_t spitch) {
-      if (es == 8)
-        hipLaunchKernelGGL(k_rows<uint64_t>, gr, b, 0, c->stream, (uint64_t *)dst, dpitch, (const uint64_t *)src,
-                           spitch, w, h);
-      else
-        hipLaunchKernelGGL(k_rows<uint32_t>, gr, b, 0, c->stream, (uint32_t *)dst, dpitch, (const uint32_t *)src,
-                           spitch, w, h);
-    };
-    if (up) {
-      HIPCHK(c, hipMemcpyAsync(dense, host, bytes, hipMemcpyHostToDevice, c->stream));
-      rows(dp, g.P, dense, w);
-    } else {
-      rows(dense, w, dp, g.P);
-      HIPCHK(c, hipMemcpyAsync(host, dense, bytes, hipMemcpyDeviceToHost, c->stream));
-    }
-    HIPCHK(c, hipGetLastError());
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (es == 8)
+      HIPCHK(c, up ? c->stg.up((uint64_t *)dp, g.P, (const uint64_t *)host, w, h, c->stream)
+                   : c->stg.down((uint64_t *)host, (const uint64_t *)dp, g.P, w, h, c->stream));
+    else
+      HIPCHK(c, up ? c->stg.up((uint32_t *)dp, g.P, (const uint32_t *)host, w, h, c->stream)
+                   : c->stg.down((uint32_t *)host, (const uint32_t *)dp, g.P, w, h, c->stream));
+    if (up) HIPCHK(c, c->stg.drain(c->stream));
     return FW_OK;
   }
   // band tables

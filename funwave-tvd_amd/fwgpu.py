@@ -217,7 +217,7 @@ class Solver:
         if fid < 0:
             raise KeyError(name)
         dt = np.int32 if name in INTF else self.rdt
-        a = np.zeros(self.shape_of(name), dt)
+        a = np.empty(self.shape_of(name), dt)
         self._check(self.lib.fw_download(self.ctx, fid, a.ctypes.data))
         return a
 
