@@ -1337,9 +1337,37 @@ __device__ __forceinline__ void flux_x_body(Dev<R> d, Geo g, Prm<R> p, const Blk
   if (!comp || !DISP) { u4L = d.U4xL[o]; u4R = d.U4xR[o]; v4L = d.V4xL[o]; v4R = d.V4xR[o]; }
   xface_finish<R, PROD>(d, g, p, c, j, comp, uL, uR, vL, vR, huL, huR, hvL, hvR, eL, eR, u4L, u4R, v4L, v4R);
 }
+// The previous stage's brk2_fill_body that is still due (on: 1), to be run by
+// one more workgroup of the next launch that neither reads nor writes ages and
+// viscosities: the dispersion, or without it the fluxes.  age, agen: the age
+// buffers as that stage had them (they swap after it).
+template <class R>
+struct BrkDue {
+  int on;
+  R DT, *age, *agen;
+};
+template <class R>
+__device__ __forceinline__ void brk2_fill_body(const Dev<R> &d, const Geo &g, const Prm<R> &p, R DT, const Blk &B);
+template <class R>
+__device__ __forceinline__ void brk2_due(Dev<R> d, const Geo &g, const Prm<R> &p, R DT, const BrkDue<R> &due,
+                                         const Blk &B) {
+  d.AGE_BREAKING = due.age;
+  d.AGEn = due.agen;
+  brk2_fill_body<R>(d, g, p, DT, B);
+}
+// (the first row of workgroups, where the previous stage's breaking is due)
 template <class R, bool DISP, bool PROD = false>
-__global__ void __launch_bounds__(256) k_flux_x(Dev<R> d, Geo g, Prm<R> p) {
-  flux_x_body<R, DISP, PROD>(d, g, p, grid_blk());
+__global__ void __launch_bounds__(256) k_flux_x(Dev<R> d, Geo g, Prm<R> p, BrkDue<R> due) {
+  Blk B = grid_blk();
+  if constexpr (!DISP) {
+    B.gy -= due.on;
+    B.y -= due.on;
+    if (B.y < 0) {
+      if (B.x == 0) brk2_due<R>(d, g, p, due.DT, due, B);
+      return;
+    }
+  }
+  flux_x_body<R, DISP, PROD>(d, g, p, B);
 }
 
 // y faces (CONSTRUCT_HO_Y fluxes.F:1642-1754, bc.F:147-210 and :221-293).
@@ -1530,9 +1558,22 @@ __device__ __forceinline__ void flux_xy_body(const Dev<R> &d, const Geo &g, cons
   if (B.x < nbx) flux_x_body<R, DISP, PROD>(d, g, p, Blk{B.x % gxx, B.x / gxx, gxx, 0, 0});
   else flux_y_body<R, DISP, 1, PROD>(d, g, p, Blk{(B.x - nbx) % gyx, (B.x - nbx) / gyx, gyx, 0, 0});
 }
+// Without dispersion the launch's first workgroup does the previous stage's
+// breaking where that is due: two launches fewer per stage (777 x 601, FP32: 242
+// -> 231 us per step).
 template <class R, bool DISP, bool PROD>
-__global__ void __launch_bounds__(64 * kFluxYThreadRows) k_flux_xy(Dev<R> d, Geo g, Prm<R> p, int gxx, int gyx) {
-  flux_xy_body<R, DISP, PROD>(d, g, p, grid_blk(), gxx, gyx);
+__global__ void __launch_bounds__(64 * kFluxYThreadRows) k_flux_xy(Dev<R> d, Geo g, Prm<R> p, int gxx, int gyx,
+                                                                   BrkDue<R> due) {
+  Blk B = grid_blk();
+  if constexpr (!DISP) {
+    B.gx -= due.on;
+    B.x -= due.on;
+    if (B.x < 0) {
+      brk2_due<R>(d, g, p, due.DT, due, B);
+      return;
+    }
+  }
+  flux_xy_body<R, DISP, PROD>(d, g, p, B, gxx, gyx);
 }
 
 // y faces by marching: each thread walks one column through a strip of RS
@@ -3171,12 +3212,16 @@ __device__ __forceinline__ void brk2_body(const Dev<R> &d, const Geo &g, const P
   __syncthreads();
   if (tid == 0) *d.cand_n = 0;
 }
+// With pub, the maximum of nblk block maxima (0: none) and the breaking flag go
+// to the host.
 template <class R>
-__global__ void __launch_bounds__(1024) k_brk2(Dev<R> d, Geo g, Prm<R> p, R DT, Pub *pub, unsigned seq) {
-  brk2_body<R>(d, g, p, DT, grid_blk());
+__global__ void __launch_bounds__(1024) k_brk2(Dev<R> d, Geo g, Prm<R> p, R DT, int nblk, Pub *pub, unsigned seq) {
+  if (p.SHOW_BRK) brk2_body<R>(d, g, p, DT, grid_blk());
   if (!pub) return;
   __syncthreads();
-  if (threadIdx.x == 0) publish(pub, 0.0, d.flags[0], seq);
+  R m = (R)0;
+  if (nblk) m = extreme1024<R, true>(d.red, nblk, (R)0);
+  if (threadIdx.x == 0) publish(pub, (double)m, d.flags[0], seq);
 }
 
 // --------------------------------------------------------------------------
@@ -3567,24 +3612,20 @@ __global__ void __launch_bounds__(1024) k_brk2_fill(Dev<R> d, Geo g, Prm<R> p, R
   if (threadIdx.x == 0) publish(pub, (double)m, d.flags[0], seq);
 }
 
-// CAL_DISPERSION in one pass, and, with brk, the previous stage's
-// brk2_fill_body by one more workgroup, the first of the launch: the
+// CAL_DISPERSION in one pass, and the previous stage's brk2_fill_body, where it
+// is due, by one more workgroup, the first of the launch: the
 // dispersion reads neither ages nor viscosities, so the single workgroup that
 // would hold up the stream for 5 us (96 x 72) to 39 (2048 x 2048) runs beside it
 // (as the last workgroup it would end 30 us after the others at 2048 x 2048).
-// age, agen: the age buffers as that stage had them (they swap after it).
 template <class R, bool P2>
 __global__ void __launch_bounds__(kDispTX * kDispTY) k_disp_fused(Dev<R> d, Geo g, Prm<R> p, R DT, const R *dtp,
-                                                                  int brk, R *age, R *agen) {
+                                                                  BrkDue<R> due) {
   const R dt = dtp ? *dtp : DT;
   Blk B = grid_blk();
-  B.gy -= brk;
-  B.y -= brk;
+  B.gy -= due.on;
+  B.y -= due.on;
   if (B.y < 0) {
-    if (B.x != 0) return;
-    d.AGE_BREAKING = age;
-    d.AGEn = agen;
-    brk2_fill_body<R>(d, g, p, dt, B);
+    if (B.x == 0) brk2_due<R>(d, g, p, dt, due, B);
     return;
   }
   disp_fused_body<R, P2>(d, g, p, dt, B);

@@ -418,6 +418,15 @@ bool disp_one_pass(fw_ctx *c) {
   return !c->prm<R>().full_state && !c->cfg.PERIODIC;
 }
 
+// the last stage's brk2_fill_body, if it is still due (on)
+template <class R>
+BrkDue<R> brk_due(fw_ctx *c, bool on) {
+  const Dev<R> &d = c->dev<R>();
+  // (the host has swapped the age buffers since that stage)
+  const bool sw = c->prm<R>().SHOW_BRK;
+  return BrkDue<R>{on ? 1 : 0, (R)c->dt, sw ? d.AGEn : d.AGE_BREAKING, sw ? d.AGE_BREAKING : d.AGEn};
+}
+
 // in_step: called by fw_step, whose RK update forms the cross derivatives
 // (the per-routine ESTIMATE_HUV reads them from the arrays); dtp: DT on the
 // device, where the host does not have it yet; brk2: the last stage's
@@ -431,9 +440,8 @@ int do_dispersion(fw_ctx *c, bool in_step = false, const R *dtp = nullptr, bool 
     const dim3 b(kDispTX, kDispTY), gr((g.M + kDispTX - 1) / kDispTX, (g.N + kDispTY - 1) / kDispTY + (brk2 ? 1 : 0));
     Prm<R> p = c->prm<R>();
     p.xd_in_huv = in_step ? 1 : 0;
-    // (the host has swapped the age buffers since that stage)
-    R *age = p.SHOW_BRK ? d.AGEn : d.AGE_BREAKING, *agen = p.SHOW_BRK ? d.AGE_BREAKING : d.AGEn;
-    auto go = [&](auto k) { launch(c, "disp", k, gr, b, d, g, p, (R)c->dt, dtp, brk2 ? 1 : 0, age, agen); };
+    const BrkDue<R> due = brk_due<R>(c, brk2);
+    auto go = [&](auto k) { launch(c, "disp", k, gr, b, d, g, p, (R)c->dt, dtp, due); };
     if (spacing_pow2<R>(c)) go(k_disp_fused<R, true>);
     else go(k_disp_fused<R, false>);
     return FW_OK;
@@ -469,28 +477,30 @@ int do_dispersion(fw_ctx *c, bool in_step = false, const R *dtp = nullptr, bool 
 template <class R>
 constexpr long kFluxOne = sizeof(R) == 4 ? 1500000 : 600000;
 // production launches (FW_OPT_FULL_STATE 0) take the flux kernels without
-// the full-state arrays' code
+// the full-state arrays' code.  brk2: the last stage's brk2_fill_body is still due
+// (without dispersion)
 template <class R, bool PROD>
-int do_fluxes_as(fw_ctx *c) {
+int do_fluxes_as(fw_ctx *c, bool brk2) {
   Dev<R> &d = c->dev<R>();
   const Geo &g = c->g;
   const bool disp = c->cfg.DISPERSION;
   constexpr int FY = FluxYTile<1>::faces;
   const int gxx = (g.M + 1 + kFluxXFaces - 1) / kFluxXFaces, gyx = (g.M + 63) / 64, gyy = (g.N + 1 + FY - 1) / FY;
   const dim3 by(64, kFluxYThreadRows);
+  const BrkDue<R> due = brk_due<R>(c, brk2);
   if ((long)g.M * g.N <= kFluxOne<R>) {
-    const dim3 gr(gxx * ((g.N + kFluxYThreadRows - 1) / kFluxYThreadRows) + gyx * gyy);
+    const dim3 gr(gxx * ((g.N + kFluxYThreadRows - 1) / kFluxYThreadRows) + gyx * gyy + due.on);
     if (disp)
-      launch(c, "flux_xy", k_flux_xy<R, true, PROD>, gr, by, d, g, c->prm<R>(), gxx, gyx);
+      launch(c, "flux_xy", k_flux_xy<R, true, PROD>, gr, by, d, g, c->prm<R>(), gxx, gyx, due);
     else
-      launch(c, "flux_xy", k_flux_xy<R, false, PROD>, gr, by, d, g, c->prm<R>(), gxx, gyx);
+      launch(c, "flux_xy", k_flux_xy<R, false, PROD>, gr, by, d, g, c->prm<R>(), gxx, gyx, due);
     return FW_OK;
   }
-  const dim3 gx(gxx, (g.N + kB2.y - 1) / kB2.y);
+  const dim3 gx(gxx, (g.N + kB2.y - 1) / kB2.y + due.on);
   if (disp)
-    launch(c, "flux_x", k_flux_x<R, true, PROD>, gx, kB2, d, g, c->prm<R>());
+    launch(c, "flux_x", k_flux_x<R, true, PROD>, gx, kB2, d, g, c->prm<R>(), due);
   else
-    launch(c, "flux_x", k_flux_x<R, false, PROD>, gx, kB2, d, g, c->prm<R>());
+    launch(c, "flux_x", k_flux_x<R, false, PROD>, gx, kB2, d, g, c->prm<R>(), due);
   if constexpr (sizeof(R) == 4) {
     // FP32: columns marched in strips of 4 faces (independent waves)
     constexpr int RS = 4;
@@ -512,7 +522,7 @@ int do_fluxes_as(fw_ctx *c) {
 }
 template <class R>
 int do_fluxes(fw_ctx *c) {
-  return c->prm<R>().full_state ? do_fluxes_as<R, false>(c) : do_fluxes_as<R, true>(c);
+  return c->prm<R>().full_state ? do_fluxes_as<R, false>(c, false) : do_fluxes_as<R, true>(c, false);
 }
 
 template <class R>
@@ -757,7 +767,7 @@ int do_breaking(fw_ctx *c, Pub *pub, unsigned seq) {
   Dev<R> &d = c->dev<R>();
   const Geo &g = c->g;
   launch(c, "brk1", k_brk1<R>, grid2(g.M, g.N, kBT), kBT, d, g, c->prm<R>(), (R)c->dt);
-  launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, c->prm<R>(), (R)c->dt, pub, seq);
+  launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, c->prm<R>(), (R)c->dt, 0, pub, seq);
   std::swap(d.AGE_BREAKING, d.AGEn);
   return FW_OK;
 }
@@ -836,8 +846,10 @@ int do_step_prod(fw_ctx *c, int nsteps) {
   const bool per = f.PERIODIC, sponge = f.DIRECT_SPONGE;
   const dim3 gb = grid2(g.M, g.N, kB2), gt = grid2(g.M + 1, g.N + 1, kB2);
   // the last stage's breaking ages' ghost cells by the one workgroup of
-  // k_brk2_fill, or, on a longer boundary, by a launch of their own (96 x 72: 5.6 us against 4 + 4;
-  // 777 x 601: 11.5 against 4 + 4; 2048 x 2048: 39 against 5 + 5)
+  // k_brk2_fill, or, on a longer boundary, by a launch after k_brk2's (96 x 72: 5.6 us against 4 + 4;
+  // 777 x 601: 11.5 against 4 + 4; 2048 x 2048: 39 against 5 + 5).  Either first
+  // launch hands the step's maximum to the host: a third one for that cost
+  // 517 x 389 cells 5 us per step
   const bool one_fill = 6 * (g.M + g.N) <= 4096;
   struct EtaW {  // the RK update leaves Eta in a plane of its own
     Dev<R> &d;
@@ -864,8 +876,8 @@ int do_step_prod(fw_ctx *c, int nsteps) {
       const bool fac = f.DISPERSION && (3 * s + st <= 2 || !trid_fixed(p));
       if (fac && (rc = fork_factor<R>(c, 3 * s + st == 2 && trid_fixed(p)))) return rc;
       if (f.DISPERSION && (rc = do_dispersion<R>(c, true, st == 1 ? (const R *)c->scal : nullptr, brk2_due))) return rc;
+      if ((rc = do_fluxes_as<R, true>(c, brk2_due && !f.DISPERSION))) return rc;
       brk2_due = false;
-      if ((rc = do_fluxes<R>(c))) return rc;
       if (st == 1) {
         if ((rc = wait_pub(c, c->pub, seq))) return rc;
         const R dt = (R)c->pub[0].val;
@@ -880,25 +892,23 @@ int do_step_prod(fw_ctx *c, int nsteps) {
       Pub *pub = last ? c->pub_dev + 1 : nullptr;
       if (!per) {
         launch(c, "tail", k_tail<R, true>, gt, kB2, d, g, p, (R)c->dt, sponge ? 1 : 0, last ? 1 : 0);
-        if (!last && f.DISPERSION) {
-          brk2_due = p.SHOW_BRK || p.VISC_BRK;  // beside the next stage's dispersion
+        if (!last) {
+          brk2_due = p.SHOW_BRK || p.VISC_BRK;  // beside the next stage's dispersion or fluxes
         } else if (one_fill) {
-          if (last || p.SHOW_BRK || p.VISC_BRK)
-            launch(c, "brk2", k_brk2_fill<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt, (int)(gt.x * gt.y), pub, seq);
+          launch(c, "brk2", k_brk2_fill<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt, (int)(gt.x * gt.y), pub, seq);
         } else {
-          if (p.SHOW_BRK) launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt, (Pub *)nullptr, 0u);
+          launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt, (int)(gt.x * gt.y), pub, seq);
           HaloList L{}, Lf{};
           if (p.VISC_BRK) {
             hadd(L, p.SHOW_BRK ? d.AGEn : d.AGE_BREAKING, 1);
             hadd(L, d.nu_break, 1);
           }
           halo_exchange_list<R>(c, L, Lf);
-          if (last) launch(c, "max_final", k_max_pub<R>, dim3(1), dim3(1024), d, (int)(gt.x * gt.y), pub, seq);
         }
       } else {
         launch(c, "tail", k_tail<R, false>, gt, kB2, d, g, p, (R)c->dt, 0, 0);
         if (!f.DISPERSION) launch(c, "ubar_hu", k_ubar_from_hu<R>, dim3(1024), dim3(256), d, plane_elems(g));
-        if (p.SHOW_BRK) launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt, (Pub *)nullptr, 0u);
+        if (p.SHOW_BRK) launch(c, "brk2", k_brk2<R>, dim3(1), dim3(1024), d, g, p, (R)c->dt, 0, (Pub *)nullptr, 0u);
       }
       std::swap(d.MASK, d.MASKn);
       if (p.SHOW_BRK) std::swap(d.AGE_BREAKING, d.AGEn);
