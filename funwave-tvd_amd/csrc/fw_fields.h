@@ -105,6 +105,8 @@ struct Prm {
   R cxa, cxb, cxc, cxd, cya, cyb, cyc, cyd, b1h;
   R h5x, h5y;       // 0.5/DX, 0.5/DY (sources.F:441-449)
   R rDXg, rDYg;     // 1/DXg, 1/DYg (etauv_solver.F:124)
+  // 1/DX, 1/DY as sums of two doubles (FP32 quotients, Dv)
+  double hDX, lDX, hDY, lDY;
 };
 
 }  // namespace fw

@@ -150,6 +150,18 @@ void fill_prm(fw_ctx *c) {
   };
   p.rDX = (R)1 / p.DX;
   p.rDY = (R)1 / p.DY;
+  // h of 29 bits, below 1/x whatever the last bits of r (its product with a
+  // 24-bit number is exact); l > 0 the rest
+  auto recip = [](R x, double &h, double &l) {
+    const double r = 1.0 / (double)x;
+    int64_t b;
+    memcpy(&b, &r, 8);
+    b = (b - 4) & ~(int64_t)0xffffff;
+    memcpy(&h, &b, 8);
+    l = std::fma(-h, (double)x, 1.0) * r;
+  };
+  recip(p.DX, p.hDX, p.lDX);
+  recip(p.DY, p.hDY, p.lDY);
   p.dx_pow2 = pow2(p.DX);
   p.dy_pow2 = pow2(p.DY);
   p.rDXg = (R)1 / p.DXg;
