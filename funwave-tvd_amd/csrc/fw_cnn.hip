@@ -661,7 +661,10 @@ int fw_cnn_create(int H, int W, int max_batch, fw_cnn **out) {
     fw_cnn_destroy(n);
     return rc;
   }
-  if (hipStreamSynchronize(n->stream) != hipSuccess) { fw_cnn_destroy(n); return FW_E_HIP; }
+  if (n->stg.init() != hipSuccess || hipStreamSynchronize(n->stream) != hipSuccess) {
+    fw_cnn_destroy(n);
+    return FW_E_HIP;
+  }
   *out = n;
   return FW_OK;
 }

@@ -1164,6 +1164,18 @@ int fw_field_id(const char *name) {
   return FW_E_NOTFOUND;
 }
 
+// The context's device for a call made with another one current (the copies
+// are launches, and the ring is allocated there).
+struct OnDevice {
+  int was = -1;
+  explicit OnDevice(int dev) {
+    if (hipGetDevice(&was) != hipSuccess || was == dev || hipSetDevice(dev) != hipSuccess) was = -1;
+  }
+  ~OnDevice() {
+    if (was >= 0) (void)hipSetDevice(was);
+  }
+};
+
 static int transfer(fw_ctx *c, int id, void *host, bool up) {
   if (!c || !host || id < 0 || id >= F_COUNT) return fail(c, FW_E_INVALID, "bad field or pointer");
   const fw_config &f = c->cfg;
@@ -1175,6 +1187,7 @@ static int transfer(fw_ctx *c, int id, void *host, bool up) {
     if (k == K_XFACE) w += 1;
     if (k == K_YFACE) h += 1;
     void *dp = field_ptr(c, id);
+    const OnDevice on(c->device);
     if (es == 8)
       HIPCHK(c, up ? c->stg.up((uint64_t *)dp, g.P, (const uint64_t *)host, w, h, c->stream)
                    : c->stg.down((uint64_t *)host, (const uint64_t *)dp, g.P, w, h, c->stream));

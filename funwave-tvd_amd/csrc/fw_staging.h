@@ -79,14 +79,36 @@ __global__ void __launch_bounds__(256) k_slot_down(uint64_t *slot, const T *__re
   slot_done(count, flag, seq);
 }
 
-// A ring of one context or network, made at its first copy and freed with it.
+// A ring of one context or network, freed with it.
 class Staging {
  public:
+  // the ring, unless it is there: 0.1 ms, which a network spends when it is
+  // made and a context at its first copy
+  hipError_t init() {
+    if (ring) return hipSuccess;
+    char *r = nullptr;
+    unsigned *c = nullptr;
+    const unsigned zero[kSlots] = {};
+    hipError_t e = hipHostMalloc((void **)&r, kSlots * kSlot + 64, hipHostMallocMapped | hipHostMallocCoherent);
+    if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&ring_dev, r, 0);
+    if (e == hipSuccess) e = hipMalloc((void **)&c, sizeof zero);
+    if (e == hipSuccess) e = hipMemcpy(c, zero, sizeof zero, hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+      if (r) (void)hipHostFree(r);
+      if (c) (void)hipFree(c);
+      return e;
+    }
+    memset(r + kSlots * kSlot, 0, 64);
+    flag_dev = (uint64_t *)(ring_dev + kSlots * kSlot);
+    ring = r;
+    count = c;
+    return hipSuccess;
+  }
   // h rows of w elements: dst (device, pitch dp) := src (host, dense), queued
   // on s; src may be changed on return
   template <class T>
   hipError_t up(T *dst, size_t dp, const T *src, uint32_t w, size_t h, hipStream_t s) {
-    hipError_t e = make();
+    hipError_t e = init();
     const size_t n = (size_t)w * h, per = kSlot / sizeof(T);
     for (size_t k = 0; e == hipSuccess && k < n; k += per) {
       const size_t c = std::min(per, n - k);
@@ -104,7 +126,7 @@ class Staging {
   // it everything queued on s before
   template <class T>
   hipError_t down(T *dst, const T *src, size_t sp, uint32_t w, size_t h, hipStream_t s) {
-    hipError_t e = make();
+    hipError_t e = init();
     const size_t n = (size_t)w * h, per = kSlot / sizeof(T), nc = (n + per - 1) / per;
     const uint64_t first = next;
     size_t issued = 0;
@@ -150,26 +172,6 @@ class Staging {
   uint64_t busy[kSlots] = {};   // number of the slot's copy in flight, 0: none
 
   uint64_t *slot(int q) { return (uint64_t *)(ring_dev + q * kSlot); }
-  hipError_t make() {
-    if (ring) return hipSuccess;
-    char *r = nullptr;
-    unsigned *c = nullptr;
-    const unsigned zero[kSlots] = {};
-    hipError_t e = hipHostMalloc((void **)&r, kSlots * kSlot + 64, hipHostMallocMapped | hipHostMallocCoherent);
-    if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&ring_dev, r, 0);
-    if (e == hipSuccess) e = hipMalloc((void **)&c, sizeof zero);
-    if (e == hipSuccess) e = hipMemcpy(c, zero, sizeof zero, hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-      if (r) (void)hipHostFree(r);
-      if (c) (void)hipFree(c);
-      return e;
-    }
-    memset(r + kSlots * kSlot, 0, 64);
-    flag_dev = (uint64_t *)(ring_dev + kSlots * kSlot);
-    ring = r;
-    count = c;
-    return hipSuccess;
-  }
   // until the slot is free.  A wait longer than 20 ms goes to the stream,
   // whose error it then reports.
   hipError_t wait(int q, hipStream_t s) {
