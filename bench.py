@@ -49,9 +49,10 @@ KERNEL_TRAFFIC = {
     # SourceTerms fused into ESTIMATE_HUV: U V U4 V4 Cd H P Q Eta DepthX DepthY,
     # the two dispersive sums, nu_break HU HV Eta0 Ubar0 Vbar0 Ubar Vbar Fx Fy
     # Gx Gy Depth, MASK MASK9 (the cross derivatives and U1p, V1p formed from
-    # U, V, Depth) -> Eta Ubar Vbar H and the six line-solve coefficient arrays
-    "src_huv": (26, 2, 10, "cell"),
-    "trid": (6, 0, 2, "inner"),
+    # U, V, Depth) -> Eta Ubar Vbar H and d/a of the x and y rows
+    "src_huv": (26, 2, 6, "cell"),
+    "trid": (6, 0, 2, "inner"),          # d/a, den, c' -> U; the same -> V
+    "trid_fac": (1, 2, 4, "inner"),      # Depth, MASK MASK9 -> den, c' of the x and y rows
     "uv_final": (3, 1, 4, "cell"),
     "mask": (4, 2, 2, "cell"),
     "brk1": (8, 0, 2, "cell"),
@@ -59,9 +60,11 @@ KERNEL_TRAFFIC = {
 }
 # limiter of the kernels whose time is not set by HBM traffic (measured:
 # VALU busy and achieved bytes in the committed counter profiles)
-LIMITER = {"flux_x": "valu", "flux_y": "valu", "trid": "latency (serial recurrences)",
+LIMITER = {"flux_x": "valu", "flux_y": "valu", "flux_xy": "valu", "disp": "valu",
+           "trid": "latency (serial recurrences)", "trid_fac": "latency (serial recurrences)",
            "brk2": "latency (one workgroup)", "dt_final": "latency (one workgroup)",
-           "max_final": "latency (one workgroup)"}
+           "max_final": "latency (one workgroup)", "halo": "latency (ghost cells)",
+           "wk_stage": "latency (one workgroup)"}
 
 
 def parse():
@@ -287,7 +290,8 @@ def sync():
 
 
 # rocprofv3 names of the kernels behind each profiling name
-ROCPROF_NAME = {"trid": "k_trid_lds<", "src_huv": "k_huv<{r}, true,", "huv": "k_huv<{r}, false,",
+ROCPROF_NAME = {"trid": "k_trid_solve<", "trid_fac": "k_trid_fac<", "tail": "k_tail<", "begin": "k_begin<",
+                "halo": "k_halo<", "src_huv": "k_huv<{r}, true,", "huv": "k_huv<{r}, false,",
                 "flux_x": "k_flux_x<", "flux_y": "k_flux_y", "disp_deriv": "k_disp_deriv<",
                 "disp_terms": "k_disp_terms<", "disp": "k_disp_fused<", "sources": "k_sources<", "uv_final": "k_uv_final<",
                 "mask": "k_mask<", "brk1": "k_brk1<", "mask_mul": "k_mask_mul<"}
@@ -486,8 +490,8 @@ def main():
                                f"waves, {n}x{n} cells dx=2 m, sponges W/S/N, wetting-drying, "
                                f"dispersion + breaking, whole RK3 steps",
                    "Mglob": n, "Nglob": n, "precision": "FP64" if rb == 8 else "FP32",
-                   "line_solver": "thomas sweep, c' and d' recurrences on two waves of one workgroup "
-                                  "(LDS-staged; bitwise the reference's recurrence)",
+                   "line_solver": "thomas sweep, c' and denominators formed ahead, d' by Markstein quotients "
+                                  "(whole lines in LDS; bitwise the reference's recurrence)",
                    "froude_cap_math": "host C library" if args.host_math else "device math library",
                    "parallelism": "one domain on one GPU"},
         # The whole step against its canonical algorithmic traffic:
