@@ -38,6 +38,7 @@ B_ALG_WORDS = 93            # algorithmic words per interior cell-step (whole st
 KERNEL_TRAFFIC = {
     "flux_x": (8, 2, 3, "xface"),        # U V HU HV Eta U4 V4 DepthX, MASK MASK9 -> P Fx Gx
     "flux_y": (8, 2, 3, "yface"),
+    "flux_xy": (9, 2, 6, "cell"),        # both in one launch
     "disp_deriv": (6, 1, 11, "cell"),    # U V Depth Eta P Q, MASK9 -> 8 second derivatives, ETAT ETAx ETAy
     "disp_terms": (17, 1, 6, "cell"),    # 8 second derivatives, ETAT ETAx ETAy, U V U0 V0 Depth Eta
                                          #   -> U4 V4 U1p V1p and the sums U1pp+U2+U3, V1pp+V2+V3
@@ -292,7 +293,8 @@ def sync():
 # rocprofv3 names of the kernels behind each profiling name
 ROCPROF_NAME = {"trid": "k_trid_solve<", "trid_fac": "k_trid_fac<", "tail": "k_tail<", "begin": "k_begin<",
                 "halo": "k_halo<", "src_huv": "k_huv<{r}, true,", "huv": "k_huv<{r}, false,",
-                "flux_x": "k_flux_x<", "flux_y": "k_flux_y", "disp_deriv": "k_disp_deriv<",
+                "flux_x": "k_flux_x<", "flux_y": "k_flux_y",
+                "flux_xy": "k_flux_xy<", "disp_deriv": "k_disp_deriv<",
                 "disp_terms": "k_disp_terms<", "disp": "k_disp_fused<", "sources": "k_sources<", "uv_final": "k_uv_final<",
                 "mask": "k_mask<", "brk1": "k_brk1<", "mask_mul": "k_mask_mul<"}
 

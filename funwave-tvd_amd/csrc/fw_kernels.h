@@ -1452,12 +1452,18 @@ __device__ __forceinline__ void yface_finish(const Dev<R> &d, const Geo &g, cons
 }
 
 // y faces: the same cell-wise reconstruction as along x, with the
-// neighbours exchanged through LDS.  A workgroup of 64 x 16 threads covers 64
-// columns and 16*K consecutive faces j of each (thread row t handles tile
-// rows t, t+16, ...); tile row r forms D(j) and the pair of cell j, takes
+// neighbours exchanged through LDS.  A workgroup of 64 x 8 threads covers 64
+// columns and 8*K consecutive faces j of each (thread row t handles tile
+// rows t, t+8, ...); tile row r forms D(j) and the pair of cell j, takes
 // D(j+1) from row r+1 and the left state of face j from row r-1.  Rows
-// 1..16K-2 own their face, so consecutive workgroups overlap by two rows.
-constexpr int kFluxYThreadRows = 16;
+// 1..8K-2 own their face, so consecutive workgroups overlap by two rows.
+// Eight rows: with 16 fewer are formed twice (2 in 16 against 2 in 8), but one
+// workgroup of 16 waves fills a CU (100 registers and, in FP64, 57 KB of LDS)
+// and its loads, slopes and pairs then wait for one another at the
+// barriers; two of 8 waves overlap.  Step at 1200 x 900 FP32 644 -> 615 us, at
+// 200 x 150 FP64 228 -> 204, 1021 x 770 1027 -> 1020 (6 rows: 639, 209, 1063; 10: 635,
+// 211, 1062; 12: 615, 213, 1043).
+constexpr int kFluxYThreadRows = 8;
 template <int K>
 struct FluxYTile {
   static constexpr int rows = kFluxYThreadRows * K;
@@ -1559,17 +1565,13 @@ __device__ __forceinline__ void flux_y_body(Dev<R> d, Geo g, Prm<R> p, const Blk
     yface_finish<R, PROD>(d, g, p, i, j, comp, uL, uR, vL, vR, huL, huR, hvL, hvR, eL, eR, u4L, u4R, v4L, v4R);
   }
 }
-template <class R, bool DISP, int K, bool PROD = false>
-__global__ void __launch_bounds__(64 * kFluxYThreadRows) k_flux_y(Dev<R> d, Geo g, Prm<R> p) {
-  flux_y_body<R, DISP, K, PROD>(d, g, p, grid_blk());
-}
-
-// Both directions in one launch, for small grids: the first nbx workgroups
-// take 16 rows of x faces, the others a tile of y faces.  Such a grid leaves
-// most of the chip idle and its fluxes are a chain of latencies, so the two
-// run side by side, and y faces take the LDS tile (one slope and one pair per
-// thread) instead of the march's nine dependent passes.  The whole step at
-// 96 x 72 cells, FP32: 244 -> 162 us (x 9.5 + y 31 us per stage before).
+// Both directions in one launch, in FP64 and for FP32 grids up to kFluxOne: the
+// first nbx workgroups take 8 rows of x faces, the others a tile of y faces.
+// A small grid leaves most of the chip idle and its fluxes are a chain of
+// latencies, so the two run side by side, and y faces take the LDS tile (one
+// slope and one pair per thread) instead of the march's nine dependent passes;
+// a larger one keeps the cells that both read in the caches.  The whole step at
+// 96 x 72 cells, FP32: 244 -> 149 us (x 9.5 + y 31 us per stage before).
 template <class R, bool DISP, bool PROD>
 __device__ __forceinline__ void flux_xy_body(const Dev<R> &d, const Geo &g, const Prm<R> &p, const Blk &B, int gxx,
                                              int gyx) {

@@ -483,11 +483,12 @@ int do_dispersion(fw_ctx *c, bool in_step = false, const R *dtp = nullptr, bool 
   return FW_OK;
 }
 
-// Cells up to which both directions' fluxes go in one launch (k_flux_xy).  The
-// step at 1400 x 1000 takes 798 us with it and 817 without, at 1600 x 1200 1050
-// and 1042 (FP32); at 800 x 600 698 and 712, at 1021 x 770 1048 and 1043 (FP64).
-template <class R>
-constexpr long kFluxOne = sizeof(R) == 4 ? 1500000 : 600000;
+// FP32 cells up to which both directions' fluxes go in one launch (k_flux_xy); on
+// larger grids the y fluxes march.  The step at 1600 x 1200 takes 996 us with it
+// and 1032 without, at 1800 x 1500 1333 and 1345, 1900 x 1700 1574 and 1574, 2048 x
+// 2048 2008 and 1985.  FP64, whose marching window would need 216 VGPRs, takes it
+// at every size (1021 x 770 994 and 1022, 2048 x 2048 4245 and 4243).
+constexpr long kFluxOne = 3000000;
 // production launches (FW_OPT_FULL_STATE 0) take the flux kernels without
 // the full-state arrays' code.  brk2: the last stage's brk2_fill_body is still due
 // (without dispersion)
@@ -500,7 +501,7 @@ int do_fluxes_as(fw_ctx *c, bool brk2) {
   const int gxx = (g.M + 1 + kFluxXFaces - 1) / kFluxXFaces, gyx = (g.M + 63) / 64, gyy = (g.N + 1 + FY - 1) / FY;
   const dim3 by(64, kFluxYThreadRows);
   const BrkDue<R> due = brk_due<R>(c, brk2);
-  if ((long)g.M * g.N <= kFluxOne<R>) {
+  if (sizeof(R) == 8 || (long)g.M * g.N <= kFluxOne) {
     const dim3 gr(gxx * ((g.N + kFluxYThreadRows - 1) / kFluxYThreadRows) + gyx * gyy + due.on);
     if (disp)
       launch(c, "flux_xy", k_flux_xy<R, true, PROD>, gr, by, d, g, c->prm<R>(), gxx, gyx, due);
@@ -508,13 +509,13 @@ int do_fluxes_as(fw_ctx *c, bool brk2) {
       launch(c, "flux_xy", k_flux_xy<R, false, PROD>, gr, by, d, g, c->prm<R>(), gxx, gyx, due);
     return FW_OK;
   }
-  const dim3 gx(gxx, (g.N + kB2.y - 1) / kB2.y + due.on);
-  if (disp)
-    launch(c, "flux_x", k_flux_x<R, true, PROD>, gx, kB2, d, g, c->prm<R>(), due);
-  else
-    launch(c, "flux_x", k_flux_x<R, false, PROD>, gx, kB2, d, g, c->prm<R>(), due);
   if constexpr (sizeof(R) == 4) {
-    // FP32: columns marched in strips of 4 faces (independent waves)
+    const dim3 gx(gxx, (g.N + kB2.y - 1) / kB2.y + due.on);
+    if (disp)
+      launch(c, "flux_x", k_flux_x<R, true, PROD>, gx, kB2, d, g, c->prm<R>(), due);
+    else
+      launch(c, "flux_x", k_flux_x<R, false, PROD>, gx, kB2, d, g, c->prm<R>(), due);
+    // columns marched in strips of 4 faces (independent waves)
     constexpr int RS = 4;
     const int nt = (g.N + 1 + RS - 1) / RS;
     const dim3 bm(64, 4), gm(gyx, (nt + 3) / 4);
@@ -522,13 +523,6 @@ int do_fluxes_as(fw_ctx *c, bool brk2) {
       launch(c, "flux_y", k_flux_y_march<R, true, RS, PROD>, gm, bm, d, g, c->prm<R>());
     else
       launch(c, "flux_y", k_flux_y_march<R, false, RS, PROD>, gm, bm, d, g, c->prm<R>());
-  } else {
-    // FP64: the LDS tile (the marching window would need 216 VGPRs)
-    const dim3 gy(gyx, gyy);
-    if (disp)
-      launch(c, "flux_y", k_flux_y<R, true, 1, PROD>, gy, by, d, g, c->prm<R>());
-    else
-      launch(c, "flux_y", k_flux_y<R, false, 1, PROD>, gy, by, d, g, c->prm<R>());
   }
   return FW_OK;
 }

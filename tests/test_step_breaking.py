@@ -14,8 +14,8 @@ pytestmark = pytest.mark.gpu
 KEYS = ["Eta", "U", "V", "HU", "HV", "Ubar", "Vbar", "H", "MASK", "MASK9", "AGE_BREAKING", "nu_break"]
 
 
-# 1540 x 1000 cells take the fluxes as two launches in FP32, 900 x 700 in FP64
-@pytest.mark.parametrize("m,n,prec", [(40, 30, "sp"), (340, 342, "sp"), (340, 343, "sp"), (1540, 1000, "sp"),
+# 2100 x 1430 cells take the fluxes as two launches in FP32
+@pytest.mark.parametrize("m,n,prec", [(40, 30, "sp"), (340, 342, "sp"), (340, 343, "sp"), (1540, 1000, "sp"), (2100, 1430, "sp"),
                                       (40, 30, "dp"), (900, 700, "dp")])
 @pytest.mark.parametrize("dispersion", [False, True])
 def test_step_matches_routines(m, n, prec, dispersion, gpu_available):
