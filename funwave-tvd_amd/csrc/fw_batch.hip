@@ -185,7 +185,7 @@ __global__ void __launch_bounds__(WideLB<R>::wg512) kb_disp_terms(FWB_ARGS, int 
 }
 
 template <class R, bool P2>
-__global__ void __launch_bounds__(kDispTX * kDispTY) kb_disp_fused(FWB_ARGS, int pm, int pa, int brk) {
+__global__ void __launch_bounds__(kDispTX<R> * kDispTY<R>) kb_disp_fused(FWB_ARGS, int pm, int pa, int brk) {
   FWB_HEAD
   if (e.x < 0) {  // the previous stage's brk2_fill, as in k_disp_fused
     if (brk) brk2_fill_body<R>(mdev(M, pm ^ 1, pa ^ 1), M.g, M.p, M.clk[0], tile_blk(e));
@@ -524,7 +524,7 @@ int build_queues(fw_batch *b) {
   const dim3 sd = b->shape[G_DISP], sh = b->shape[G_HUV], sc = b->shape[G_CELL];
   if ((rc = make_tiles(b, "disp", sd, sd.x, sd.y, M_, N_))) return rc;
   // (and one workgroup per member for the previous stage's brk2_fill, first)
-  if ((rc = make_tiles(b, "dispf", dim3(kDispTX, kDispTY), kDispTX, kDispTY, M_, N_, true))) return rc;
+  if ((rc = make_tiles(b, "dispf", dim3(kDispTX<R>, kDispTY<R>), kDispTX<R>, kDispTY<R>, M_, N_, true))) return rc;
   if ((rc = make_tiles(b, "huv", sh, sh.x, sh.y, M_, N_))) return rc;
   if ((rc = make_tiles(b, "cell", sc, sc.x, sc.y, M_, N_))) return rc;
   auto M1 = [](const Geo &g) { return g.M + 1; };

@@ -793,7 +793,7 @@ __global__ void __launch_bounds__(WideLB<R>::wg512) k_disp_terms(Dev<R> d, Geo g
 
 // --------------------------------------------------------------------------
 // CAL_DISPERSION in one pass (dispersion.F:62-506), for the production path
-// of a non-periodic domain: the eight second derivatives of a 64 x 8 tile and
+// of a non-periodic domain: the eight second derivatives of a tile of cells and
 // its one-cell ring go to LDS, already as EXCHANGE_DISPERSION leaves them
 // (a ghost cell holds the value of its mirror cell, negated for the arrays
 // odd in that direction, bc.F:306-529), and the terms of k_disp_terms are
@@ -802,7 +802,14 @@ __global__ void __launch_bounds__(WideLB<R>::wg512) k_disp_terms(Dev<R> d, Geo g
 // nonlinear sums, and the four cross derivatives and U1p, V1p unless the RK
 // update forms those itself, p.xd_in_huv).  Same operations on
 // the same operands as k_disp_deriv + ghost fill + k_disp_terms.
-constexpr int kDispTX = 64, kDispTY = 8;
+// Tile of k_disp_fused, one thread per cell.  In FP64 its 138 registers leave a
+// SIMD three waves: one workgroup of 64 x 8 fills a CU and waits at its own
+// barrier, smaller ones overlap.  Step at 96 x 72, 400 x 300, 1021 x 770 and 2048 x
+// 2048 cells of 1.5 m, FP64: 64 x 8 192, 355, 1063, 4486 us; 64 x 4 185, 343, 1050, 4420; 32 x
+// 8 198, 335, 1041, 4375; 32 x 4 191, 337, 1050, 4402 (no size slower).  FP32 (72
+// registers) has three workgroups of 64 x 8 per CU: other tiles are equal or slower.
+template <class R> constexpr int kDispTX = sizeof(R) == 4 ? 64 : 32;
+template <class R> constexpr int kDispTY = sizeof(R) == 4 ? 8 : 4;
 
 // the eight second derivatives at (i, j) after the ghost fill (0 Uxx, 1
 // Vxy, 2 Uxy, 3 Vyy, 4 DUxx, 5 DVxy, 6 DUxy, 7 DVyy)
@@ -841,20 +848,20 @@ __device__ __forceinline__ void second_derivs(const Dev<R> &d, const Geo &g, con
 
 template <class R, bool P2>
 __device__ __forceinline__ void disp_fused_body(Dev<R> d, Geo g, Prm<R> p, R DT, const Blk &B) {
-  constexpr int EX = kDispTX + 2, EY = kDispTY + 2;
+  constexpr int EX = kDispTX<R> + 2, EY = kDispTY<R> + 2;
   __shared__ R sS[8][EY][EX];
   // max(Depth, MinDepthFrc), Ut and Vt of the tile and its ring, formed once
   // per cell (the terms read them at the nine points of their stencil)
   __shared__ R sT[3][EY][EX];
   const Tile tb = xcd_tile(B);
-  const int x0 = 1 + tb.x * kDispTX, y0 = 1 + tb.y * kDispTY;
+  const int x0 = 1 + tb.x * kDispTX<R>, y0 = 1 + tb.y * kDispTY<R>;
   const int tx = threadIdx.x, ty = threadIdx.y;
   // the ring of second derivatives: at most two cells per thread, both
   // formed unconditionally (clamped into the grid, dropped outside it) so
   // that their loads go out together
   {
-    const int t = tx + ty * kDispTX;
-    constexpr int NT = kDispTX * kDispTY, NE = EX * EY;
+    const int t = tx + ty * kDispTX<R>;
+    constexpr int NT = kDispTX<R> * kDispTY<R>, NE = EX * EY;
     static_assert(NE <= 2 * NT, "two ring cells per thread at most");
     const int qa = t, qb = t + NT < NE ? t + NT : NE - 1;
     const R mdf = p.MDF;
@@ -3639,7 +3646,7 @@ __global__ void __launch_bounds__(1024) k_brk2_fill(Dev<R> d, Geo g, Prm<R> p, R
 // would hold up the stream for 5 us (96 x 72) to 39 (2048 x 2048) runs beside it
 // (as the last workgroup it would end 30 us after the others at 2048 x 2048).
 template <class R, bool P2>
-__global__ void __launch_bounds__(kDispTX * kDispTY) k_disp_fused(Dev<R> d, Geo g, Prm<R> p, R DT, const R *dtp,
+__global__ void __launch_bounds__(kDispTX<R> * kDispTY<R>) k_disp_fused(Dev<R> d, Geo g, Prm<R> p, R DT, const R *dtp,
                                                                   BrkDue<R> due) {
   const R dt = dtp ? *dtp : DT;
   Blk B = grid_blk();

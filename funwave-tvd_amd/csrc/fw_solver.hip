@@ -449,7 +449,7 @@ int do_dispersion(fw_ctx *c, bool in_step = false, const R *dtp = nullptr, bool 
   const Geo &g = c->g;
   if (disp_one_pass<R>(c)) {
     // one pass: the second derivatives stay in LDS (k_disp_fused)
-    const dim3 b(kDispTX, kDispTY), gr((g.M + kDispTX - 1) / kDispTX, (g.N + kDispTY - 1) / kDispTY + (brk2 ? 1 : 0));
+    const dim3 b(kDispTX<R>, kDispTY<R>), gr((g.M + kDispTX<R> - 1) / kDispTX<R>, (g.N + kDispTY<R> - 1) / kDispTY<R> + (brk2 ? 1 : 0));
     Prm<R> p = c->prm<R>();
     p.xd_in_huv = in_step ? 1 : 0;
     const BrkDue<R> due = brk_due<R>(c, brk2);
