@@ -121,6 +121,14 @@ __global__ void kb_halo_per(FWB_ARGS, int list, int pm) {
   else halo_body<R>(M.hxf[pm].a[e.y - L.n], M.g, 0, tile_blk(e));
 }
 
+// the same where a member is narrow (k_halo_seq)
+template <class R>
+__global__ void kb_halo_seq(FWB_ARGS, int list, int phase, int pm) {
+  FWB_HEAD
+  const HaloList &L = list == 0 ? M.hx[pm] : M.hd;
+  halo_seq_body<R>(e.y < L.n ? L.a[e.y] : M.hxf[pm].a[e.y - L.n], M.g, M.p.PERIODIC, phase, tile_blk(e));
+}
+
 template <class R>
 __global__ void __launch_bounds__(256) kb_begin(FWB_ARGS, int pm, int pa) {
   FWB_HEAD
@@ -309,6 +317,7 @@ struct fw_batch {
   int n = 0;
   int rb = 4;
   bool periodic = false, disp = false, pow2 = false;
+  bool narrow = false;  // some member is (k_halo_seq)
   std::string err;
   hipStream_t stream = nullptr, side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_fac = nullptr;
@@ -586,11 +595,19 @@ void bl(fw_batch *b, hipStream_t s, const char *qname, K k, A... args) {
   bl_lds<R>(b, s, qname, 0, k, args...);
 }
 
+// ghost fills of list 0 (EXCHANGE) or 1 (CAL_DISPERSION's arrays)
+template <class R>
+void rec_halo(fw_batch *b, int list, int par) {
+  const char *q = list == 0 ? "halo_x" : "halo_d";
+  if (!b->narrow) return bl<R>(b, b->stream, q, kb_halo_per<R>, list, par);
+  for (int phase = 0; phase <= 2; phase++) bl<R>(b, b->stream, q, kb_halo_seq<R>, list, phase, par);
+}
+
 // periodic EXCHANGE (+ SPONGE_DAMPING when sponge) at buffer parity par
 template <class R>
 void rec_exchange(fw_batch *b, int par, int sponge) {
   hipStream_t s = b->stream;
-  bl<R>(b, s, "halo_x", kb_halo_per<R>, 0, par);
+  rec_halo<R>(b, 0, par);
   bl<R>(b, s, "cell", kb_mask_mul<R>, par, par, sponge, 1);
 }
 
@@ -624,7 +641,7 @@ int rec_step(fw_batch *b, int p0, bool first) {
       bl<R>(b, s, "dispf", kb_disp_fused<R, P2>, par, par, st > 0 ? 1 : 0);
     } else if (b->disp) {
       bl<R>(b, s, "disp", kb_disp_deriv<R, P2>, par, par);
-      bl<R>(b, s, "halo_d", kb_halo_per<R>, 1, par);
+      rec_halo<R>(b, 1, par);
       bl<R>(b, s, "disp", kb_disp_terms<R, P2>, par, par);
     }
     if (b->disp) bl<R>(b, s, "flux_x", kb_flux_x<R, true>, par, par);
@@ -1014,6 +1031,7 @@ int fw_batch_create(fw_ctx *const *members, int n, fw_batch **out) {
     b->rb = c0->rb;
     b->disp = c0->cfg.DISPERSION;
     b->periodic = c0->cfg.PERIODIC;
+    for (int m = 0; m < n; m++) b->narrow = b->narrow || narrow(members[m]->g, b->periodic);
     b->pow2 = pow2_of(c0);
     if (hipSetDevice(c0->device) != hipSuccess || hipStreamCreate(&b->stream) != hipSuccess ||
         hipStreamCreate(&b->side) != hipSuccess ||

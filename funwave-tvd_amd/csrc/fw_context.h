@@ -115,6 +115,11 @@ inline void hadd(HaloList &L, void *p, int vtype, int isint = 0, int spec = 0) {
   L.a[L.n++] = HaloArr{p, vtype, isint, spec};
 }
 
+// Fewer than three interior cells across a mirrored direction (k_halo_seq).
+inline bool narrow(const Geo &g, bool periodic) {
+  return g.Ie - g.Ib < 2 || (!periodic && g.Je - g.Jb < 2);
+}
+
 // Line-solve launch: workgroups of x and y lines, whether the lines' d' fit
 // into LDS (TridCfg), dynamic LDS bytes.  n: rows of the longest line.
 struct TridGrid {

@@ -245,6 +245,43 @@ __device__ __forceinline__ void halo_per_body(const HaloArr &A, const Geo &g, co
   if (A.isint) fill((int *)A.p);
   else fill((R *)A.p);
 }
+// Domains of fewer than three interior cells across a mirrored direction: there
+// a ghost cell mirrors another ghost cell, so the reference's order matters (low
+// side, then high side, outermost low cell first) and one pass over all ghost
+// cells would race.  Three launches: phase 0, the periodic y copy of the cell
+// arrays (from interior rows only); phase 1, the x ghosts, one thread per interior
+// row; phase 2, the mirrored y ghosts, one thread per column.
+template <class R>
+__device__ __forceinline__ void halo_seq_body(const HaloArr &A, const Geo &g, bool per, int phase, const Blk &B) {
+  const bool copy = per && A.spec == 0;
+  if (phase == 0) {
+    if (copy) halo_body<R>(A, g, 1, B);
+    return;
+  }
+  if (phase == 2 && copy) return;
+  const HaloSpec s = halo_spec(g, A.spec);
+  const bool x = phase == 1;
+  const int t = B.x * blockDim.x + threadIdx.x;
+  if (t >= (x ? s.Je - s.Jb + 1 : s.Ma)) return;
+  const size_t o = x ? IX(1, s.Jb + t) : IX(1 + t, 1), st = x ? 1 : (size_t)g.P;
+  const int lo = x ? s.Ib : s.Jb, hi = x ? s.Ie : s.Je;
+  const bool odd = A.vtype == (x ? 2 : 3);
+  auto fill = [&](auto *ph) {
+    auto mirror = [&](int to, int from) {
+      const auto v = ph[o + (size_t)(from - 1) * st];
+      ph[o + (size_t)(to - 1) * st] = odd ? -v : v;
+    };
+    for (int k = 1; k <= 3; k++) mirror(k, lo + 3 - k);
+    for (int k = 1; k <= 3; k++) mirror(hi + k, hi - k + 1);
+  };
+  if (A.isint) fill((int *)A.p);
+  else fill((R *)A.p);
+}
+template <class R>
+__global__ void k_halo_seq(HaloList L, HaloList Lf, Geo g, int per, int phase) {
+  const int a = blockIdx.y;
+  halo_seq_body<R>(a < L.n ? L.a[a] : Lf.a[a - L.n], g, per, phase, grid_blk());
+}
 // cell arrays of L periodic, face arrays of Lf mirrored
 template <class R>
 __global__ void k_halo_per(HaloList L, HaloList Lf, Geo g) {

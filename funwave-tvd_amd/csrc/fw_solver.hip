@@ -346,7 +346,11 @@ void halo_exchange_list(fw_ctx *c, HaloList &L, HaloList &Lf) {
   // grid rows = arrays of the list
   const dim3 b(256), gr((cnt + 255) / 256, L.n + Lf.n);
   if (!gr.y) return;
-  if (!c->cfg.PERIODIC) {
+  const bool per = c->cfg.PERIODIC;
+  if (narrow(g, per)) {
+    for (int phase = per ? 0 : 1; phase <= 2; phase++)
+      launch(c, "halo", k_halo_seq<R>, gr, b, L, Lf, g, per ? 1 : 0, phase);
+  } else if (!per) {
     for (int k = 0; k < Lf.n; k++) L.a[L.n++] = Lf.a[k];
     launch(c, "halo", k_halo<R>, gr, b, L, g, 0);
   } else {
