@@ -13,8 +13,9 @@
 // arranges within one domain).  The kernels are the per-domain kernels' own
 // bodies (fw_kernels.h), so every member's arithmetic is exactly that of
 // fw_step on the member alone.
-// As in fw_step, a non-periodic member's step starts with one pass (kb_begin)
-// and what follows the line solves is another (kb_tail).
+// As in fw_step, a walled member's step starts with one pass (kb_begin)
+// and what follows the line solves is another (kb_tail); periodic batches,
+// and those with a member under three cells across, fill ghosts separately.
 //
 // Nothing goes back to the host during a run: each member's DT, TIME and
 // status live on the device (ESTIMATE_DT, misc.F:216-296, with FIXED_DT;
@@ -58,8 +59,8 @@ struct Member {
   Dev<R> d;
   Geo g;
   Prm<R> p;
-  HaloList hx[2];   // periodic: EXCHANGE cell arrays at buffer parity 0 / 1
-  HaloList hxf[2];  // periodic: the face arrays P, Q
+  HaloList hx[2];   // fw_batch::sep: EXCHANGE cell arrays at buffer parity 0 / 1
+  HaloList hxf[2];  // fw_batch::sep: the face arrays P, Q
   HaloList hd;      // periodic: CAL_DISPERSION second derivatives (+ ETAx, ETAy)
   R *clk;           // [0] DT, [1] TIME, [2] max |eta|
   int *st;          // [0] status, [1] steps taken since the wavemaker table
@@ -111,7 +112,7 @@ __global__ void kb_copy3(FWB_ARGS) {
   }
 }
 
-// Periodic fills; list 0: EXCHANGE (queue y = array, then face array), 1:
+// Separate fills; list 0: EXCHANGE (queue y = array, then face array), 1:
 // CAL_DISPERSION's arrays
 template <class R>
 __global__ void kb_halo_per(FWB_ARGS, int list, int pm) {
@@ -318,6 +319,7 @@ struct fw_batch {
   int rb = 4;
   bool periodic = false, disp = false, pow2 = false;
   bool narrow = false;  // some member is (k_halo_seq)
+  bool sep = false;     // fills of their own, as in fw_step: periodic, or some member narrow
   std::string err;
   hipStream_t stream = nullptr, side = nullptr;
   hipEvent_t ev_fork = nullptr, ev_fac = nullptr;
@@ -430,7 +432,7 @@ Member<R> &mem_h(fw_batch *b, int m) {
   return ((Member<R> *)b->members_h.data())[m];
 }
 
-// halo queue of the periodic fills: ghost chunks x arrays
+// halo queue of the separate fills: ghost chunks x arrays
 template <class R>
 int make_halo_queue(fw_batch *b, const std::string &name, int list) {
   Queue &Q = b->q[name];
@@ -486,7 +488,7 @@ int fill_members(fw_batch *b) {
     fw_ctx *c = b->mem[m];
     Member<R> &M = mem_h<R>(b, m);
     M.d = c->dev<R>();
-    if (!c->cfg.PERIODIC) M.d.EtaW = M.d.eta2;  // as in fw_step
+    if (!b->sep) M.d.EtaW = M.d.eta2;  // as in fw_step
     M.g = c->g;
     M.p = c->prm<R>();
     // the one-pass dispersion leaves the cross derivatives and U1p, V1p to
@@ -510,7 +512,7 @@ int fill_members(fw_batch *b) {
     M.wks = b->wk_stride[m];
     M.wk = M.wks ? (const R *)((char *)b->wk + b->wk_off[m]) : nullptr;
     const long ncell = (long)c->g.M * c->g.N;
-    if (c->cfg.PERIODIC) {
+    if (b->sep) {
       M.ndt = (int)std::min<long>(kRedBlocks, (ncell + 255) / 256);
       M.nmax = std::min(256, c->g.Je - c->g.Jb + 1);
     } else {  // the workgroups of kb_begin and kb_tail
@@ -572,10 +574,8 @@ int build_queues(fw_batch *b) {
   b->trid = trid_lds<R>(rows);
   b->trid_fixed = true;
   for (int m = 0; m < b->n; m++) b->trid_fixed = b->trid_fixed && trid_fixed(mem(m).p);
-  if (b->periodic) {
-    if ((rc = make_halo_queue<R>(b, "halo_x", 0))) return rc;
-    if ((rc = make_halo_queue<R>(b, "halo_d", 1))) return rc;
-  }
+  if (b->sep && (rc = make_halo_queue<R>(b, "halo_x", 0))) return rc;
+  if (b->periodic && (rc = make_halo_queue<R>(b, "halo_d", 1))) return rc;
   return FW_OK;
 }
 
@@ -603,7 +603,7 @@ void rec_halo(fw_batch *b, int list, int par) {
   for (int phase = 0; phase <= 2; phase++) bl<R>(b, b->stream, q, kb_halo_seq<R>, list, phase, par);
 }
 
-// periodic EXCHANGE (+ SPONGE_DAMPING when sponge) at buffer parity par
+// EXCHANGE by a fill of its own (+ SPONGE_DAMPING when sponge) at buffer parity par
 template <class R>
 void rec_exchange(fw_batch *b, int par, int sponge) {
   hipStream_t s = b->stream;
@@ -619,9 +619,9 @@ int rec_step(fw_batch *b, int p0, bool first) {
   hipStream_t s = b->stream, sd = b->side;
   const R alpha[3] = {(R)0, (R)3 / (R)4, (R)1 / (R)3};
   const R beta[3] = {(R)1, (R)1 / (R)4, (R)2 / (R)3};
-  const bool per = b->periodic;
+  const bool per = b->periodic, sep = b->sep;
   int par = p0;
-  if (!per) {
+  if (!sep) {
     bl<R>(b, s, "begin", kb_begin<R>, par, par);
   } else {
     bl<R>(b, s, "copy", kb_copy3<R>);
@@ -638,7 +638,7 @@ int rec_step(fw_batch *b, int p0, bool first) {
       BCHK(b, hipEventRecord(b->ev_fac, sd));
     }
     if (b->disp && !per) {
-      bl<R>(b, s, "dispf", kb_disp_fused<R, P2>, par, par, st > 0 ? 1 : 0);
+      bl<R>(b, s, "dispf", kb_disp_fused<R, P2>, par, par, st > 0 && !sep ? 1 : 0);
     } else if (b->disp) {
       bl<R>(b, s, "disp", kb_disp_deriv<R, P2>, par, par);
       rec_halo<R>(b, 1, par);
@@ -664,7 +664,7 @@ int rec_step(fw_batch *b, int p0, bool first) {
       if (per) solve(kb_trid_solve<R, true, true>, kb_trid_solve<R, false, true>);
       else solve(kb_trid_solve<R, true, false>, kb_trid_solve<R, false, false>);
     }
-    if (!per) {
+    if (!sep) {
       bl<R>(b, s, "tail", kb_tail<R, true>, par, par, st == 2 ? 1 : 0);
       if (st == 2 || !b->disp) bl<R>(b, s, "one1024", kb_brk2_fill<R>, par, par);
     } else {
@@ -673,9 +673,9 @@ int rec_step(fw_batch *b, int p0, bool first) {
       bl<R>(b, s, "one1024", kb_brk2<R>, par, par);
     }
     par ^= 1;
-    if (per) rec_exchange<R>(b, par, -1);
+    if (sep) rec_exchange<R>(b, par, -1);
   }
-  if (per) bl<R>(b, s, "max", kb_maxeta_partial<R>);
+  if (sep) bl<R>(b, s, "max", kb_maxeta_partial<R>);
   bl<R>(b, s, "one1024", kb_max_final<R>);
   return FW_OK;
 }
@@ -933,7 +933,7 @@ int autotune(fw_batch *b, int trial, std::string &rep) {
     // the two-pass dispersion kernels run only for periodic members (the
     // others take the fused kernel, whose tile is fixed)
     if (gi == G_DISP && !(b->disp && b->periodic)) continue;
-    if ((gi == G_CELL && !b->periodic) || gi == G_BRK) continue;  // UPDATE_MASK and breaking are in kb_tail
+    if ((gi == G_CELL && !b->sep) || gi == G_BRK) continue;  // UPDATE_MASK and breaking are in kb_tail
     dim3 best = cand[gi][0];
     double best_ms = 1e30;
     for (const dim3 &s : cand[gi]) {
@@ -1032,6 +1032,7 @@ int fw_batch_create(fw_ctx *const *members, int n, fw_batch **out) {
     b->disp = c0->cfg.DISPERSION;
     b->periodic = c0->cfg.PERIODIC;
     for (int m = 0; m < n; m++) b->narrow = b->narrow || narrow(members[m]->g, b->periodic);
+    b->sep = b->periodic || b->narrow;
     b->pow2 = pow2_of(c0);
     if (hipSetDevice(c0->device) != hipSuccess || hipStreamCreate(&b->stream) != hipSuccess ||
         hipStreamCreate(&b->side) != hipSuccess ||

@@ -853,7 +853,9 @@ int do_step_prod(fw_ctx *c, int nsteps) {
   const fw_config &f = c->cfg;
   const Geo &g = c->g;
   const Prm<R> &p = c->prm<R>();
-  const bool per = f.PERIODIC, sponge = f.DIRECT_SPONGE;
+  // a fill of its own (do_exchange) where a ghost cell is no function of one
+  // interior cell: periodic and narrow domains
+  const bool sep = f.PERIODIC || narrow(g, f.PERIODIC), sponge = f.DIRECT_SPONGE;
   const dim3 gb = grid2(g.M, g.N, kB2), gt = grid2(g.M + 1, g.N + 1, kB2);
   // the last stage's breaking ages' ghost cells by the one workgroup of
   // k_brk2_fill, or, on a longer boundary, by a launch after k_brk2's (96 x 72: 5.6 us against 4 + 4;
@@ -865,12 +867,12 @@ int do_step_prod(fw_ctx *c, int nsteps) {
     Dev<R> &d;
     EtaW(Dev<R> &d_, bool own) : d(d_) { if (own) d.EtaW = d.eta2; }
     ~EtaW() { d.EtaW = d.Eta; }
-  } guard(d, !per);
+  } guard(d, !sep);
   int rc = FW_OK;
   for (int s = 0; s < nsteps; s++) {
     const unsigned seq = ++c->pub_seq;
     int nblk = (int)(gb.x * gb.y);
-    if (!per) {
+    if (!sep) {
       launch(c, "begin", k_begin<R>, gb, kB2, d, g, p);
     } else {
       launch(c, "copy3", k_copy3<R>, dim3(2048), dim3(256), d.Eta0, (const R *)d.Eta, d.Ubar0, (const R *)d.Ubar,
@@ -900,7 +902,7 @@ int do_step_prod(fw_ctx *c, int nsteps) {
       if ((rc = do_lines<R>(c, true))) return rc;
       const bool last = st == 3;
       Pub *pub = last ? c->pub_dev + 1 : nullptr;
-      if (!per) {
+      if (!sep) {
         launch(c, "tail", k_tail<R, true>, gt, kB2, d, g, p, (R)c->dt, sponge ? 1 : 0, last ? 1 : 0);
         if (!last) {
           brk2_due = p.SHOW_BRK || p.VISC_BRK;  // beside the next stage's dispersion or fluxes
@@ -922,9 +924,9 @@ int do_step_prod(fw_ctx *c, int nsteps) {
       }
       std::swap(d.MASK, d.MASKn);
       if (p.SHOW_BRK) std::swap(d.AGE_BREAKING, d.AGEn);
-      if (per && (rc = do_exchange<R>(c, sponge))) return rc;
+      if (sep && (rc = do_exchange<R>(c, sponge))) return rc;
     }
-    if (per) {
+    if (sep) {
       launch(c, "maxeta", k_maxeta_partial<R>, dim3(256), dim3(256), d, g);
       launch(c, "max_final", k_max_pub<R>, dim3(1), dim3(1024), d, 256, c->pub_dev + 1, seq);
     }

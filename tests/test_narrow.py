@@ -1,7 +1,10 @@
 """Domains of one and two interior cells across, where ghost cells mirror other
 ghost cells: EXCHANGE against the oracle, whose fills run in the reference's
-order (bc.F:631-1272).  Copies and sign changes only, so the tolerance is
-none: every array bit for bit, ghost cells included."""
+order (bc.F:631-1272); whole steps of the production path and of batches
+against the routine-by-routine path, and that against the oracle.  The same
+operations everywhere, so the tolerance is none: every array bit for bit,
+ghost cells included (against the oracle with the Froude cap's ATAN2, COS and
+SIN left to the host)."""
 import numpy as np
 import pytest
 
@@ -62,3 +65,53 @@ def test_exchange_matches_oracle(periodic, m, n, prec, gpu_available):
                for k in ("Eta", "U", "V", "HU", "HV", "P", "Q", "MASK", "AGE_BREAKING", "nu_break")}
         assert not any(bad.values()), (rep, bad)
     g.close()
+
+
+STEP_KEYS = ["Eta", "Eta0", "U", "V", "U0", "V0", "HU", "HV", "Ubar", "Vbar", "Ubar0", "Vbar0", "H", "MASK", "MASK9",
+             "AGE_BREAKING", "nu_break", "DepthX", "DepthY", "P", "Q"]
+OPTIONS = [{}, {"DISPERSION": False}, {"VISCOSITY_BREAKING": False}, {"DIRECT_SPONGE": True},
+           {"SHOW_BREAKING": False, "DX": 1.5, "DY": 1.5},
+           {"VISCOSITY_BREAKING": False, "DIFFUSION_SPONGE": True, "FRICTION_SPONGE": True}]
+
+
+# (three cells are the least that take the merged passes, whose threads write
+# only the ghost cells that mirror an interior cell)
+@pytest.mark.parametrize("prec", ["sp", "dp"])
+@pytest.mark.parametrize("m,n", [(1, 1), (1, 2), (2, 1), (2, 2), (7, 1), (2, 9), (1, 130), (150, 2), (3, 3), (3, 8), (4, 5)])
+def test_steps_match_routines_and_oracle(m, n, prec, gpu_available):
+    import fwgpu
+    import oracle
+    for opt in OPTIONS:
+        print(f"\n[narrow step] {m} x {n} {prec} {opt}", flush=True)
+        st = narrow_state(m, n, prec, **opt)
+        g, r = fwgpu.Solver(st, prec), fwgpu.Solver(st, prec, full_state=True)
+        h, o = fwgpu.Solver(st, prec, host_math=True), oracle.OracleSolver(st)
+        for steps in (1, 2):
+            assert g.step(steps) == r.step(steps)
+            bad = {k: bitwise_mismatch(g.download(k), r.download(k)) for k in STEP_KEYS}
+            assert not any(bad.values()), bad
+            assert h.step(steps) == (o.run(steps), (o.dt.value, o.time.value))[1]
+            bad = {k: bitwise_mismatch(h.download(k), o[k]) for k in STEP_KEYS}
+            assert not any(bad.values()), bad
+        for s in (g, r, h):
+            s.close()
+
+
+@pytest.mark.parametrize("prec", ["sp", "dp"])
+@pytest.mark.parametrize("opt", OPTIONS[:4])
+def test_batch_matches_members_alone(opt, prec, gpu_available):
+    import fwgpu
+    print(f"\n[narrow batch] {prec} {opt}", flush=True)
+    sts = [narrow_state(m, n, prec, DT_fixed=0.02, **opt) for m, n in ((40, 30), (1, 7), (2, 2), (9, 2), (3, 3))]
+    alone, gs = ([fwgpu.Solver(st, prec) for st in sts] for _ in range(2))
+    b = fwgpu.Batch(gs)
+    for steps in (1, 2, 4):
+        b.step(steps)
+        for g, a in zip(gs, alone):
+            a.step(steps)
+            assert g.clock == a.clock
+            bad = {k: bitwise_mismatch(g.download(k), a.download(k)) for k in STEP_KEYS}
+            assert not any(bad.values()), (g.M, g.N, bad)
+    b.close()
+    for s in gs + alone:
+        s.close()
