@@ -82,6 +82,7 @@ struct fw_ctx {
   // breaking flag (pinned memory, as the host and as the device see it)
   fw::Pub *pub = nullptr, *pub_dev = nullptr;
   unsigned pub_seq = 0;
+  hipError_t launch_err = hipSuccess;  // of a launch since launch_status() last asked
   std::string err;
   bool prof = false;
   std::vector<PendingEvent> pending;

@@ -74,11 +74,18 @@ void launch_lds(fw_ctx *c, const char *name, K k, dim3 grid, dim3 block, size_t 
     b = get_event(c);
     (void)hipEventRecord(a, c->cur);
   }
-  hipLaunchKernelGGL(k, grid, block, lds, c->cur, args...);
+  const hipError_t e = fws::start(k, grid, block, lds, c->cur, args...);
+  if (c->launch_err == hipSuccess) c->launch_err = e;
   if (c->prof) {
     (void)hipEventRecord(b, c->cur);
     c->pending.push_back({name, a, b});
   }
+}
+int launch_status(fw_ctx *c) {
+  const hipError_t e = c->launch_err;
+  c->launch_err = hipSuccess;
+  if (e != hipSuccess) return fail(c, FW_E_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
+  return FW_OK;
 }
 template <typename K, typename... A>
 void launch(fw_ctx *c, const char *name, K k, dim3 grid, dim3 block, A... args) {
@@ -327,6 +334,8 @@ int stage_wavemaker(fw_ctx *c, R &AA) {
 // The host's side of publish(): spins until the kernel has stored seq.  A wait
 // longer than 20 ms goes to the stream, whose error it then reports.
 int wait_pub(fw_ctx *c, const Pub *p, unsigned seq) {
+  const int rc = launch_status(c);
+  if (rc) return rc;
   const auto t0 = std::chrono::steady_clock::now();
   while (__atomic_load_n(&p->seq, __ATOMIC_ACQUIRE) != seq) {
     for (int k = 0; k < 32; k++) __builtin_ia32_pause();
@@ -404,7 +413,6 @@ int do_estimate_dt(fw_ctx *c, bool copy_uv) {
   launch(c, "dt_partial", k_dt_partial<R>, dim3(nblk), dim3(256), d, c->g, c->prm<R>(), copy_uv ? 1 : 0);
   const unsigned seq = ++c->pub_seq;
   launch(c, "dt_final", k_dt_pub<R>, dim3(1), dim3(1024), d, c->prm<R>(), nblk, (R *)c->scal, c->pub_dev, seq);
-  HIPCHK(c, hipGetLastError());
   int rc = wait_pub(c, c->pub, seq);
   if (rc) return rc;
   const R dt = (R)c->pub[0].val;
@@ -420,7 +428,6 @@ int do_max_eta(fw_ctx *c, double *out) {
   launch(c, "maxeta", k_maxeta_partial<R>, dim3(nblk), dim3(256), d, c->g);
   const unsigned seq = ++c->pub_seq;
   launch(c, "max_final", k_max_pub<R>, dim3(1), dim3(1024), d, nblk, c->pub_dev + 1, seq);
-  HIPCHK(c, hipGetLastError());
   int rc = wait_pub(c, c->pub + 1, seq);
   if (rc) return rc;
   *out = c->pub[1].val;
@@ -701,7 +708,6 @@ int do_lines(fw_ctx *c, bool fac) {
       if (tg.res) launch_lds(c, "trid", k_trid_solve<R, true, false>, gr, b, tg.lds, d, g, tg.nx);
       else launch_lds(c, "trid", k_trid_solve<R, false, false>, gr, b, tg.lds, d, g, tg.nx);
     }
-    HIPCHK(c, hipGetLastError());  // (the only launch with more than 64 KB of dynamic LDS)
   }
   return FW_OK;
 }
@@ -1314,7 +1320,6 @@ int fw_wave_breaking(fw_ctx *c) {
   if (rc == FW_OK) rc = DISPATCH(c, do_roller)(c);
   if (rc) return rc;
   if (c->cfg.SHOW_BREAKING) {
-    HIPCHK(c, hipGetLastError());
     if ((rc = wait_pub(c, c->pub + 2, seq))) return rc;
     if (c->pub[2].flag && (rc = read_break_flag(c, c->rb == 8 ? (void *)c->dd.flags : (void *)c->df.flags))) return rc;
   }

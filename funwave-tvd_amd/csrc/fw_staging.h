@@ -17,6 +17,18 @@
 
 namespace fws {
 
+// A launch that returns its own status: what hipGetLastError gives may be the
+// error of an earlier, unrelated call of this thread, and asking clears it.
+template <class T>
+struct Same {
+  using type = T;
+};
+template <class... P>
+hipError_t start(void (*k)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t s, typename Same<P>::type... a) {
+  void *args[] = {(void *)&a...};
+  return hipLaunchKernel((const void *)k, grid, block, args, lds, s);
+}
+
 // Slots are read and written with system-scope accesses, which pass the caches
 // by; once they have completed (the wait, in every wave), one counter and one
 // store tell the host.  With a system-scope fence in every wave instead, which
@@ -115,10 +127,10 @@ class Staging {
       const int q = (int)(next % kSlots);
       if ((e = wait(q, s)) != hipSuccess) break;  // the slot's last copy
       memcpy(ring + q * kSlot, src + k, c * sizeof(T));
-      busy[q] = ++next;
-      hipLaunchKernelGGL(k_slot_up<T>, dim3(kWg), dim3(256), 0, s, dst + k / w * dp, dp, slot(q), w,
-                         (uint32_t)(k % w), (uint32_t)c, count + q, flag_dev + q, next);
-      if ((e = hipGetLastError()) != hipSuccess) busy[q] = 0;
+      ++next;
+      e = start(k_slot_up<T>, dim3(kWg), dim3(256), 0, s, dst + k / w * dp, dp, slot(q), w, (uint32_t)(k % w),
+                (uint32_t)c, count + q, flag_dev + q, next);
+      if (e == hipSuccess) busy[q] = next;
     }
     return e;
   }
@@ -135,10 +147,10 @@ class Staging {
         const int q = (int)(next % kSlots);
         if ((e = wait(q, s)) != hipSuccess) break;
         const size_t k0 = issued * per;
-        busy[q] = ++next;
-        hipLaunchKernelGGL(k_slot_down<T>, dim3(kWg), dim3(256), 0, s, slot(q), src + k0 / w * sp, sp, w,
-                           (uint32_t)(k0 % w), (uint32_t)std::min(per, n - k0), count + q, flag_dev + q, next);
-        if ((e = hipGetLastError()) != hipSuccess) busy[q] = 0;
+        ++next;
+        e = start(k_slot_down<T>, dim3(kWg), dim3(256), 0, s, slot(q), src + k0 / w * sp, sp, w, (uint32_t)(k0 % w),
+                  (uint32_t)std::min(per, n - k0), count + q, flag_dev + q, next);
+        if (e == hipSuccess) busy[q] = next;
       }
       if (e != hipSuccess) break;
       const int q = (int)((first + k) % kSlots);
