@@ -1200,7 +1200,8 @@ static int transfer(fw_ctx *c, int id, void *host, bool up) {
     else
       HIPCHK(c, up ? c->stg.up((uint32_t *)dp, g.P, (const uint32_t *)host, w, h, c->stream)
                    : c->stg.down((uint32_t *)host, (const uint32_t *)dp, g.P, w, h, c->stream));
-    if (up) HIPCHK(c, c->stg.drain(c->stream));
+    // (streams that do not wait for this one may read the field next)
+    if (up) HIPCHK(c, hipStreamSynchronize(c->stream));
     return FW_OK;
   }
   // band tables

@@ -117,7 +117,9 @@ class Staging {
     return hipSuccess;
   }
   // h rows of w elements: dst (device, pitch dp) := src (host, dense), queued
-  // on s; src may be changed on return
+  // on s; src may be changed on return.  A slot's flag says that it has been
+  // read, not that dst can be read from another stream: an XCD's cache is
+  // written back when the kernel ends.
   template <class T>
   hipError_t up(T *dst, size_t dp, const T *src, uint32_t w, size_t h, hipStream_t s) {
     hipError_t e = init();
@@ -157,12 +159,6 @@ class Staging {
       if ((e = wait(q, s)) != hipSuccess) break;
       memcpy(dst + k * per, ring + q * kSlot, std::min(per, n - k * per) * sizeof(T));
     }
-    return e;
-  }
-  // until everything copied up has left the ring
-  hipError_t drain(hipStream_t s) {
-    hipError_t e = hipSuccess;
-    for (int q = 0; e == hipSuccess && q < kSlots; q++) e = wait(q, s);
     return e;
   }
   // (after the owner's stream has been synchronised)
