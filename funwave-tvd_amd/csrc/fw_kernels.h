@@ -3283,7 +3283,7 @@ template <class R>
 __global__ void __launch_bounds__(1024) k_brk2(Dev<R> d, Geo g, Prm<R> p, R DT, int nblk, Pub *pub, unsigned seq) {
   if (p.SHOW_BRK) brk2_body<R>(d, g, p, DT, grid_blk());
   if (!pub) return;
-  __syncthreads();
+  __syncthreads();  // (publish releases the workgroup's stores)
   R m = (R)0;
   if (nblk) m = extreme1024<R, true>(d.red, nblk, (R)0);
   if (threadIdx.x == 0) publish(pub, (double)m, d.flags[0], seq);

@@ -1324,6 +1324,8 @@ int fw_wave_breaking(fw_ctx *c) {
     if ((rc = wait_pub(c, c->pub + 2, seq))) return rc;
     if (c->pub[2].flag && (rc = read_break_flag(c, c->rb == 8 ? (void *)c->dd.flags : (void *)c->df.flags))) return rc;
   }
+  // (the roller's kernel follows the one that has told the host)
+  if (c->rb == 8 ? c->pd.full_state : c->pf.full_state) HIPCHK(c, hipStreamSynchronize(c->stream));
   return c->prof ? collect_profile(c) : FW_OK;
 }
 int fw_sponge_damping(fw_ctx *c) { ENTRY(c, DISPATCH(c, do_sponge_only)(c)); }

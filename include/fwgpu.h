@@ -16,8 +16,8 @@
  * from one host thread at a time.  Work runs on the context's own HIP stream
  * (default priority); calls return after the work is queued, except those
  * that hand a value back to the host (fw_estimate_dt, fw_step,
- * fw_check_blowup, fw_download, fw_reduce_stats) and fw_upload, which wait
- * for it.
+ * fw_check_blowup, fw_download, fw_reduce_stats), fw_upload and
+ * fw_wave_breaking (which reports FW_E_BREAK_ITER), which wait for it.
  */
 #ifndef FWGPU_H
 #define FWGPU_H

@@ -58,3 +58,29 @@ def test_upload(m, n, prec, gpu_available):
         assert idle(g)
         assert on_side_stream(g, "Eta").tobytes() == a.tobytes(), rep
     g.close()
+
+
+@pytest.mark.parametrize("full", [False, True])
+@pytest.mark.parametrize("m,n,prec", [(60, 40, "sp"), (1500, 1000, "sp"), (700, 500, "dp")])
+def test_breaking(m, n, prec, full, gpu_available):
+    """Ages and viscosities, and with every intermediate kept the roller flux,
+    whose kernel is the last of WAVE_BREAKING."""
+    print(f"\n[visibility] breaking {m} x {n} {prec} full={full}", flush=True)
+    g = solver(m, n, prec, full_state=full)
+    rng = np.random.default_rng(m)
+    shape = g.shape_of("Eta")
+    g.set_clock(0.1, 0.0)
+    g.upload("H", np.full(shape, 2.0))
+    names = ["AGE_BREAKING", "nu_break"] + (["ROLLER_FLUX"] if full else [])
+    for rep in range(8):
+        for k in ("ETAT", "ETAx", "ETAy", "U", "V", "Eta"):  # (the roller flux is proportional to Eta - ETAmean)
+            g.upload(k, 6.0 * rng.standard_normal(shape))
+        g.breaking()
+        if full:
+            assert idle(g)
+        seen = {k: on_side_stream(g, k) for k in names}
+        g.synchronize()
+        for k, v in seen.items():
+            assert v.tobytes() == g.download(k).tobytes(), (k, rep)
+    assert all(np.count_nonzero(v) > 0 for v in seen.values())
+    g.close()
