@@ -69,6 +69,7 @@ struct Member {
   int wks;          // stride of wk (0: no per-step wavemaker source)
   int show_brk;
   int ndt, nmax;    // block extremes that ESTIMATE_DT / CHECK_BLOWUP reduce
+  int pl;           // periodic y lines of a workgroup of the line solves
   size_t pe;        // elements of one plane
 };
 
@@ -247,7 +248,7 @@ __global__ void __launch_bounds__(kTridThreads) kb_trid_fac(FWB_ARGS, int pm, in
 template <class R, bool RES, bool PER>
 __global__ void __launch_bounds__(kTridThreads) kb_trid_solve(FWB_ARGS, int pm, int pa) {
   FWB_HEAD
-  trid_lines_body<R, RES, PER>(mdev(M, pm, pa), M.g, e.aux, tile_blk(e));
+  trid_lines_body<R, RES, PER>(mdev(M, pm, pa), M.g, e.aux, M.pl, tile_blk(e));
 }
 
 template <class R>
@@ -484,6 +485,17 @@ inline int tiles(int n) { return (n + 63) / 64; }
 template <class R>
 int fill_members(fw_batch *b) {
   b->members_h.assign(sizeof(Member<R>) * b->n, 0);
+  int rows = 0;  // of the longest line over all members
+  long wgs = 0;    // of x lines, and one for each wavefront of periodic y lines
+  for (fw_ctx *c : b->mem) {
+    const int nx = c->g.Ie - c->g.Ib + 1, ny = c->g.Je - c->g.Jb + 1;
+    rows = std::max(rows, b->periodic ? nx : std::max(nx, ny));
+    wgs += (ny + kTridL - 1) / kTridL + (nx + 63) / 64;
+  }
+  b->trid = trid_lds<R>(rows);
+  // 24 members of 1024 x 200, FP32, one workgroup per CU: 5.7 ms per step with 64
+  // lines of each, 4.7 with 320; 12 of them 3.1 and 3.0; 4 of up to 400 x 300 1.7 and 1.8
+  const bool whole = wgs > 256 * (long)(TridCfg<R>::lds_max / b->trid.lds);
   for (int m = 0; m < b->n; m++) {
     fw_ctx *c = b->mem[m];
     Member<R> &M = mem_h<R>(b, m);
@@ -520,6 +532,7 @@ int fill_members(fw_batch *b) {
       M.nmax = tiles(c->g.M + 1) * ((c->g.N + 4) / 4);
     }
     M.pe = plane_elems(c->g);
+    M.pl = whole ? kTridThreads : per_lines<R>(c->g.Ie - c->g.Ib + 1, c->g.Je - c->g.Jb + 1, kTridThreads);
   }
   BCHK(b, hipMemcpy(b->members, b->members_h.data(), b->members_h.size(), hipMemcpyHostToDevice));
   return FW_OK;
@@ -559,19 +572,16 @@ int build_queues(fw_batch *b) {
   auto chunks = [&](int m) { return (int)std::min<size_t>(2048, (mem(m).pe + 2047) / 2048); };
   if ((rc = make_line(b, "copy", dim3(256), chunks, chunks))) return rc;
   auto nx = [&](int m) { return trid_grid<R>(mem(m).g, b->periodic).nx; };
-  auto nxy = [&](int m) { const TridGrid t = trid_grid<R>(mem(m).g, b->periodic); return t.nx + t.ny; };
+  auto nxy = [&](int m) {
+    const TridGrid t = trid_grid<R>(mem(m).g, b->periodic);
+    return t.nx + (b->periodic ? (mem(m).g.Ie - mem(m).g.Ib + mem(m).pl) / mem(m).pl : t.ny);
+  };
   if ((rc = make_line(b, "trid", dim3(kTridThreads), nxy, nx))) return rc;
   if (b->periodic) {  // c' of the x lines only
     if ((rc = make_line(b, "trid_fac", dim3(kTridThreads), nx, nx))) return rc;
   } else {
     if ((rc = make_line(b, "trid_fac", dim3(kTridThreads), nxy, nx))) return rc;
   }
-  int rows = 0;  // of the longest line over all members
-  for (int m = 0; m < b->n; m++) {
-    const Geo &g = mem(m).g;
-    rows = std::max(rows, b->periodic ? g.Ie - g.Ib + 1 : std::max(g.Ie - g.Ib + 1, g.Je - g.Jb + 1));
-  }
-  b->trid = trid_lds<R>(rows);
   b->trid_fixed = true;
   for (int m = 0; m < b->n; m++) b->trid_fixed = b->trid_fixed && trid_fixed(mem(m).p);
   if (b->sep && (rc = make_halo_queue<R>(b, "halo_x", 0))) return rc;

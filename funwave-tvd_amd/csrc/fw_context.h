@@ -140,7 +140,8 @@ inline TridGrid trid_grid(const Geo &g, bool periodic) {
   const int nx = g.Ie - g.Ib + 1, ny = g.Je - g.Jb + 1;
   TridGrid t = trid_lds<R>(periodic ? nx : (nx > ny ? nx : ny));
   t.nx = (ny + kTridL - 1) / kTridL;
-  t.ny = periodic ? (nx + kTridThreads - 1) / kTridThreads : (nx + kTridL - 1) / kTridL;
+  const int yl = periodic ? per_lines<R>(nx, ny, kTridThreads) : kTridL;
+  t.ny = (nx + yl - 1) / yl;
   return t;
 }
 

@@ -2597,8 +2597,22 @@ __device__ __forceinline__ void trid_solve_body(const Dev<R> &d, const Geo &g, i
 }
 
 // TRIDy_periodic (tridiagnal.F:59-325, serial path): Sherman-Morrison, one
-// thread per line (its lines are short).  The RK update keeps a, c, d
-// themselves in ya, yc, yd for it.
+// thread per line.  The RK update keeps a, c, d themselves in ya, yc, yd for it.
+// What bounds it is the latency of one dependent row after another.  A domain
+// whose lines fit one workgroup is solved by one: the wavefronts share the
+// cache lines that their columns straddle.  Beyond 128 KB of a plane those have
+// left the cache before the way back, and wider domains have more wavefronts
+// than one CU's path to the L2 feeds: there a workgroup takes one wavefront of
+// lines.  (A batch whose wavefronts would outnumber what the chip holds at a
+// time takes whole workgroups again: Member::pl.)  Line solves of a stage (x lines beside them), one workgroup of 320
+// against 64 lines each, columns x rows: FP32 96 x 64 96 and 109 us, 200 x 128 195
+// and 217, 300 x 64 105 and 110, 300 x 300 556 and 490; FP64 256 x 64 114 and 117,
+// 200 x 128 234 and 226, 300 x 300 634 and 524.  320 lines of each workgroup against
+// 64 at 1024 x 300: FP32 608 and 512, FP64 709 and 560; up to eight rows no difference.
+template <class R>
+__host__ __device__ constexpr int per_lines(int lines, int rows, int n) {
+  return lines <= n && (long)lines * rows * (long)sizeof(R) <= 128 * 1024 ? n : 64;
+}
 template <class R>
 __device__ __forceinline__ void thomas(R *A, R *C, R *D, R *Z, size_t o0, ptrdiff_t s, int n) {
   R cprev = C[o0], dprev = D[o0];
@@ -2626,10 +2640,10 @@ __device__ __forceinline__ void thomas(R *A, R *C, R *D, R *Z, size_t o0, ptrdif
   }
 }
 template <class R>
-__device__ __forceinline__ void trid_per_body(const Dev<R> &d, const Geo &g, int blk) {
+__device__ __forceinline__ void trid_per_body(const Dev<R> &d, const Geo &g, int blk, int pl) {
   const int ny = g.Je - g.Jb + 1;
-  const int i = g.Ib + blk * blockDim.x + threadIdx.x;
-  if (i > g.Ie) return;
+  const int i = g.Ib + blk * pl + threadIdx.x;
+  if ((int)threadIdx.x >= pl || i > g.Ie) return;
   const ptrdiff_t s = (ptrdiff_t)g.P;
   R *a = d.ya, *c = d.yc, *dd = d.yd;
   size_t ob = IX(i, g.Jb), oe = IX(i, g.Je);
@@ -2650,14 +2664,14 @@ __device__ __forceinline__ void trid_per_body(const Dev<R> &d, const Geo &g, int
     d.V[o] = d.y1[o] + beta * d.y2[o];
   }
 }
-// PER: the y lines are periodic (workgroups from nxblk on)
+// PER: the y lines are periodic (pl of each workgroup from nxblk on)
 template <class R, bool RES, bool PER>
-__device__ __forceinline__ void trid_lines_body(const Dev<R> &d, const Geo &g, int nxblk, const Blk &B) {
+__device__ __forceinline__ void trid_lines_body(const Dev<R> &d, const Geo &g, int nxblk, int pl, const Blk &B) {
   extern __shared__ __attribute__((aligned(16))) char trid_smem[];
   if (PER) {
     const int b = line_block(B);
     if (b >= nxblk) {
-      trid_per_body<R>(d, g, b - nxblk);
+      trid_per_body<R>(d, g, b - nxblk, pl);
       return;
     }
   }
@@ -2665,7 +2679,7 @@ __device__ __forceinline__ void trid_lines_body(const Dev<R> &d, const Geo &g, i
 }
 template <class R, bool RES, bool PER>
 __global__ void __launch_bounds__(kTridThreads) k_trid_solve(Dev<R> d, Geo g, int nxblk) {
-  trid_lines_body<R, RES, PER>(d, g, nxblk, grid_blk());
+  trid_lines_body<R, RES, PER>(d, g, nxblk, per_lines<R>(g.Ie - g.Ib + 1, g.Je - g.Jb + 1, kTridThreads), grid_blk());
 }
 
 // ---- the whole solve in one sweep, for fw_estimate_huv, where a, c and d all
@@ -2896,11 +2910,11 @@ __device__ __forceinline__ void trid_lds_body(Dev<R> d, Geo g, int nxblk, const 
   }
   if (w >= 2) bwd_store(0, 0);
 }
-// PER: the y lines are periodic (256 per workgroup from nxblk on)
+// PER: the y lines are periodic (per_lines of each workgroup from nxblk on)
 template <class R, int L, int CH, bool PER>
 __global__ void __launch_bounds__(256) k_trid_lds(Dev<R> d, Geo g, int nxblk) {
   if (PER && (int)blockIdx.x >= nxblk) {
-    trid_per_body<R>(d, g, blockIdx.x - nxblk);
+    trid_per_body<R>(d, g, blockIdx.x - nxblk, per_lines<R>(g.Ie - g.Ib + 1, g.Je - g.Jb + 1, 256));
     return;
   }
   trid_lds_body<R, L, CH>(d, g, nxblk, grid_blk());

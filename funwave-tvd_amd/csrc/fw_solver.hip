@@ -694,8 +694,9 @@ int do_lines(fw_ctx *c, bool fac) {
     // 48 rows (125 KB)
     constexpr int L = kTridL, CH = sizeof(R) == 4 ? 64 : 48;
     const int ny = g.Je - g.Jb + 1, nx = g.Ie - g.Ib + 1, nxblk = (ny + L - 1) / L;
+    const int pl = per_lines<R>(nx, ny, 256);
     if (c->cfg.PERIODIC)
-      launch(c, "trid", k_trid_lds<R, L, CH, true>, dim3(nxblk + (nx + 255) / 256), dim3(256), d, g, nxblk);
+      launch(c, "trid", k_trid_lds<R, L, CH, true>, dim3(nxblk + (nx + pl - 1) / pl), dim3(256), d, g, nxblk);
     else
       launch(c, "trid", k_trid_lds<R, L, CH, false>, dim3(nxblk + (nx + L - 1) / L), dim3(256), d, g, nxblk);
   } else if (c->cfg.DISPERSION) {

@@ -192,3 +192,25 @@ def test_untuned_batch_starts_with_whole_wavefronts(gpu_available):
     b.close()
     for g in gs:
         g.close()
+
+
+@pytest.mark.parametrize("prec", ["sp", "dp"])
+def test_periodic_members_beyond_the_chip(prec, gpu_available):
+    """Sixteen periodic members whose line solves take more workgroups than
+    there are CUs (their y lines then go by whole workgroups), and three
+    whose y lines go by wavefronts, by both launch rules the members' own
+    results bit for bit."""
+    import fwcases
+    import fwgpu
+    for sizes in ([(1000, 3)] * 15 + [(333, 5)], [(400, 4), (300, 40), (64, 64)]):
+        print(f"\n[batch periodic] {prec} {len(sizes)} members", flush=True)
+        sts = {s: fixed_dt_state(fwcases.beach_1d(mglob=s[0], nglob=s[1], xslp=0.4 * s[0], xc_wk=0.2 * s[0],
+                                                  sponge_west=0.1 * s[0]), prec) for s in set(sizes)}
+        ref = {s: run_alone([st], prec, 3)[0] for s, st in sts.items()}
+        gs = [fwgpu.Solver(sts[s], prec) for s in sizes]
+        b = fwgpu.Batch(gs)
+        b.step(3)
+        compare(gs, [ref[s] for s in sizes], "periodic batch")
+        b.close()
+        for g in gs:
+            g.close()

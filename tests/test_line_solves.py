@@ -79,3 +79,27 @@ def test_periodic_lines_match_oracle(m, n, prec, gpu_available):
     bad = {k: bitwise_mismatch(g.download(k), o[k]) for k in KEYS}
     assert not any(bad.values()), bad
     g.close()
+
+
+# periodic y lines: all in one workgroup (up to 320 columns in fw_step, 256 by
+# routine, 128 KB of a plane), one more column, one more row, a remainder of a
+# wavefront, and many
+@pytest.mark.parametrize("m,n,prec", [(64, 16, "sp"), (256, 20, "sp"), (257, 20, "sp"), (320, 102, "sp"), (320, 103, "sp"),
+                                      (321, 20, "sp"), (130, 252, "sp"), (130, 253, "sp"), (700, 33, "sp"),
+                                      (320, 51, "dp"), (320, 52, "dp"), (321, 17, "dp"), (129, 130, "dp")])
+def test_periodic_y_lines_match_oracle(m, n, prec, gpu_available):
+    import fwgpu
+    import oracle
+    print(f"\n[line solves] periodic y {m} x {n} {prec}", flush=True)
+    st = _state(m, n, prec, True, False, periodic=True)
+    g, o = fwgpu.Solver(st, prec, host_math=True), oracle.OracleSolver(st)
+    assert g.step(2) == (o.run(2), (o.dt.value, o.time.value))[1]
+    bad = {k: bitwise_mismatch(g.download(k), o[k]) for k in KEYS}
+    assert not any(bad.values()), bad
+    g.dispersion(); o.dispersion()
+    g.fluxes(); o.fluxes()
+    g.sources(); o.sources()
+    g.estimate_huv(2); o.estimate_huv(2)
+    bad = {k: bitwise_mismatch(g.download(k), o[k]) for k in ("Eta", "U", "V", "HU", "HV")}
+    assert not any(bad.values()), bad
+    g.close()
