@@ -137,6 +137,8 @@ __global__ void __launch_bounds__(256) kb_begin(FWB_ARGS, int pm, int pa) {
   begin_body<R>(mdev(M, pm, pa), M.g, M.p, tile_blk(e, e.aux));
 }
 
+// (64 x 4 threads: with 64 x 8 an FP32 batch of 16 members of about 640 x 448 takes
+// 2634 us per step instead of 2594, FP64 as long)
 template <class R, bool FILL>
 __global__ void __launch_bounds__(256) kb_tail(FWB_ARGS, int pm, int pa, int last) {
   FWB_HEAD
@@ -293,15 +295,15 @@ __global__ void kb_reset_steps(int *const *st, int n) {
 
 // tunable workgroup shapes (the kernels take any shape within their
 // launch bounds); names as reported by fw_batch_autotune
-enum Group { G_DISP = 0, G_HUV, G_CELL, G_BRK, G_COUNT };
+enum Group { G_DISP = 0, G_HUV, G_CELL, G_COUNT };
 const char *kGroupName[G_COUNT] = {"disp (disp_deriv, disp_terms; periodic members)", "src_huv",
-                                   "cell (mask_mul; periodic members)", "mask/brk (part of the fixed-shape tail)"};
+                                   "cell (mask_mul; separate fills)"};
 
 // The shapes a batch starts with: the single-domain step's (64 x 8 for the
 // neighbour-reading kernels, 64 x 4 elsewhere).  They are set explicitly: a
 // default-constructed dim3 is 1 x 1, one thread per workgroup, which ran
 // sixteen members of 640 x 448 cells at 32.6 ms per step instead of 3.0.
-const dim3 kGroupShape[G_COUNT] = {dim3(64, 8), dim3(64, 4), dim3(64, 4), dim3(64, 8)};
+const dim3 kGroupShape[G_COUNT] = {dim3(64, 8), dim3(64, 4), dim3(64, 4)};
 
 struct Queue {
   std::vector<QEnt> h;
@@ -338,7 +340,7 @@ struct fw_batch {
   // queues
   std::map<std::string, Queue> q;
   TridGrid trid{};  // LDS of the line solves
-  dim3 shape[G_COUNT] = {kGroupShape[0], kGroupShape[1], kGroupShape[2], kGroupShape[3]};
+  dim3 shape[G_COUNT] = {kGroupShape[0], kGroupShape[1], kGroupShape[2]};
   // graphs of one step per starting parity, and of the first step of a call
   hipGraphExec_t gx[3] = {nullptr, nullptr, nullptr};
   bool trid_fixed = false;  // trid_fixed() holds for every member
@@ -913,9 +915,8 @@ int autotune(fw_batch *b, int trial, std::string &rep) {
   std::vector<dim3> cand[G_COUNT] = {
       {dim3(64, 8), dim3(64, 4), dim3(128, 4), dim3(128, 2), dim3(64, 16)},
       {dim3(64, 4), dim3(64, 2), dim3(128, 2), dim3(64, 8), dim3(256, 1)},
-      {dim3(64, 4), dim3(64, 2), dim3(128, 2), dim3(256, 1), dim3(64, 8)},
-      {dim3(64, 8), dim3(64, 4), dim3(128, 4), dim3(128, 2)}};
-  const int lim[G_COUNT] = {lim_disp, lim_huv, 1024, 1024};
+      {dim3(64, 4), dim3(64, 2), dim3(128, 2), dim3(256, 1), dim3(64, 8)}};
+  const int lim[G_COUNT] = {lim_disp, lim_huv, 1024};
   std::vector<double> dt0, tm0;
   std::vector<int> st0 = b->status;
   std::vector<Dev<R>> dev0;  // the contexts' buffer assignment (trial runs swap it)
@@ -943,7 +944,7 @@ int autotune(fw_batch *b, int trial, std::string &rep) {
     // the two-pass dispersion kernels run only for periodic members (the
     // others take the fused kernel, whose tile is fixed)
     if (gi == G_DISP && !(b->disp && b->periodic)) continue;
-    if ((gi == G_CELL && !b->sep) || gi == G_BRK) continue;  // UPDATE_MASK and breaking are in kb_tail
+    if (gi == G_CELL && !b->sep) continue;  // (part of kb_tail, whose tile is fixed)
     dim3 best = cand[gi][0];
     double best_ms = 1e30;
     for (const dim3 &s : cand[gi]) {
@@ -1128,9 +1129,13 @@ int fw_batch_autotune(fw_batch *b, int trial_steps, char *report, int len) {
 
 int fw_batch_get_shapes(const fw_batch *b, int *shapes) {
   if (!b || !shapes) return FW_E_INVALID;
-  for (int k = 0; k < G_COUNT; k++) {
-    shapes[2 * k] = (int)b->shape[k].x;
-    shapes[2 * k + 1] = (int)b->shape[k].y;
+  // of the queues that a step launches
+  const char *disp = b->periodic ? "disp" : "dispf";
+  const char *q[4] = {disp, "huv", b->sep ? "cell" : "tail", b->disp && !b->sep ? disp : "one1024"};
+  for (int k = 0; k < 4; k++) {
+    const dim3 s = b->q.at(q[k]).block;
+    shapes[2 * k] = (int)s.x;
+    shapes[2 * k + 1] = (int)s.y;
   }
   return FW_OK;
 }

@@ -214,13 +214,16 @@ int fw_batch_status(const fw_batch *b, int *status /* n entries */);
 int fw_batch_time_steps(fw_batch *b, int nsteps, double *ms);
 /* 1 (default): replay the captured step graphs; 0: launch eagerly */
 int fw_batch_set_graph(fw_batch *b, int on);
-/* Workgroup shapes of the tunable kernels (the RK update and, in periodic
- * batches, the dispersion stencils and the velocity tail) chosen by timing
+/* Workgroup shapes of the tunable kernels (the RK update; in periodic batches
+ * also the dispersion stencils and EXCHANGE's mask multiply) chosen by timing
  * trial_steps steps per candidate on a snapshot of the members' state,
  * restored afterwards; report: one line per trial. */
 int fw_batch_autotune(fw_batch *b, int trial_steps, char *report, int len);
-/* the shapes in use: 4 groups x (x, y): dispersion, RK update, velocity tail,
- * UPDATE_MASK and breaking (the last two fixed unless periodic) */
+/* the shapes launched, 4 groups x (x, y): dispersion; RK update; EXCHANGE's
+ * mask multiply (batches of walled members: the pass after the line solves,
+ * which contains it, the velocity tail, UPDATE_MASK and breaking's first
+ * pass); breaking's fixed point, one workgroup per member (walled members
+ * with dispersion: of the next dispersion launch) */
 int fw_batch_get_shapes(const fw_batch *b, int *shapes);
 
 #ifdef __cplusplus

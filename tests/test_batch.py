@@ -214,3 +214,25 @@ def test_periodic_members_beyond_the_chip(prec, gpu_available):
         b.close()
         for g in gs:
             g.close()
+
+
+def test_reported_shapes_are_those_launched(gpu_available):
+    """fw_batch_get_shapes takes the shapes from the launches themselves: walled
+    FP64 members' dispersion runs in tiles of 32 x 4, breaking's fixed point is
+    a workgroup of that launch or, without it, one of 1024 threads, and
+    periodic batches report the mask multiply's shape."""
+    import fwcases
+    import fwgpu
+    print("\n[batch] shapes launched", flush=True)
+    base = fixed_dt_state(fwcases.member(5, mrange=(60, 60), nrange=(40, 40)), "dp")
+    per = fixed_dt_state(fwcases.beach_1d(mglob=100, nglob=4, xslp=40.0, xc_wk=20.0, sponge_west=10.0), "sp")
+    swe = dict(fixed_dt_state(fwcases.member(5, mrange=(60, 60), nrange=(40, 40)), "sp"), DISPERSION=0)
+    for st, prec, want in ((base, "dp", {"disp": (32, 4), "cell": (64, 4), "mask_brk": (32, 4)}),
+                           (per, "sp", {"disp": (64, 8), "cell": (64, 4), "mask_brk": (1024, 1)}),
+                           (swe, "sp", {"cell": (64, 4), "mask_brk": (1024, 1)})):
+        g = fwgpu.Solver(st, prec)
+        b = fwgpu.Batch([g])
+        got = b.shapes()
+        assert {k: got[k] for k in want} == want, got
+        b.close()
+        g.close()
