@@ -223,3 +223,52 @@ def test_conserving_correction_moves_no_water(gpu_available):
     assert abs(np.sum((e1 - e0)[wet])) <= 1e-3 * moved
     net.close()
     g.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,W", [(8, 4, 1024), (1, 8, 4128), (9, 61, 70)])
+def test_gradient_of_many_tiles_matches_numpy(B, H, W, gpu_available):
+    """Weight gradients are summed over tiles of 4 x 64 pixels by at most 128
+    workgroups: exactly one tile each, two workgroups with a second one, and
+    288 tiles ragged both ways.  Tolerance as above."""
+    import fwcnn
+    rng = np.random.default_rng(B + H + W)
+    p = random_params(17)
+    x = rng.standard_normal((B, 5, H, W)).astype(np.float32)
+    tgt = rng.standard_normal((B, 3, H, W)).astype(np.float32)
+    print(f"\n[cnn gradient] B={B} H={H} W={W}", flush=True)
+    net = fwcnn.Net(H, W, B, fwcnn.flatten(p))
+    loss, g = net.train_step(x, tgt, lr=0.0, want_grad=True)
+    ref_loss, ref_g = cn.loss_and_grad(p, x, tgt)
+    assert loss == pytest.approx(ref_loss, rel=1e-2)
+    gd = fwcnn.unflatten(g)
+    for name, _ in fwcnn.SHAPES:
+        e = rel_l2(gd[name], ref_g[name])
+        print(f"  {name}: rel L2 {e:.2e}")
+        assert e < 1e-2, name
+    net.close()
+
+
+@pytest.mark.gpu
+def test_packs_follow_the_parameters(gpu_available):
+    """A training step writes each new parameter into the forward and the
+    data-gradient weight packs itself: outputs and gradients are then those of
+    a network made from the parameters, bit for bit."""
+    import fwcnn
+    rng = np.random.default_rng(31)
+    B, H, W = 3, 21, 70
+    x = rng.standard_normal((B, 5, H, W)).astype(np.float32)
+    tgt = rng.standard_normal((B, 3, H, W)).astype(np.float32)
+    print(f"\n[cnn packs] B={B} H={H} W={W}", flush=True)
+    net = fwcnn.Net(H, W, B, fwcnn.flatten(random_params(32)))
+    before = net.params()
+    for _ in range(3):
+        net.train_step(x, tgt, lr=1e-2)
+    after = net.params()
+    assert np.mean(after != before) > 0.9
+    fresh = fwcnn.Net(H, W, B, after)
+    assert net.forward(x).tobytes() == fresh.forward(x).tobytes()
+    (l0, g0), (l1, g1) = (n.train_step(x, tgt, lr=0.0, want_grad=True) for n in (net, fresh))
+    assert l0 == l1 and g0.tobytes() == g1.tobytes()
+    net.close()
+    fresh.close()
