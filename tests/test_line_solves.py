@@ -103,3 +103,84 @@ def test_periodic_y_lines_match_oracle(m, n, prec, gpu_available):
     bad = {k: bitwise_mismatch(g.download(k), o[k]) for k in ("Eta", "U", "V", "HU", "HV")}
     assert not any(bad.values()), bad
     g.close()
+
+
+# x lines too long for LDS (FP32 beyond 2112 rows, FP64 beyond 1024): their d'
+# goes through memory, periodic domains and batches included
+@pytest.mark.parametrize("m,n,prec", [(2112, 4, "sp"), (2113, 4, "sp"), (3000, 5, "sp"), (1024, 4, "dp"), (1025, 4, "dp"),
+                                      (2300, 5, "dp")])
+def test_long_periodic_lines_match_oracle(m, n, prec, gpu_available):
+    import fwgpu
+    import oracle
+    print(f"\n[line solves] long periodic {m} x {n} {prec}", flush=True)
+    for visc in (True, False):
+        st = _state(m, n, prec, visc, False, periodic=True)
+        g, o = fwgpu.Solver(st, prec, host_math=True), oracle.OracleSolver(st)
+        assert g.step(2) == (o.run(2), (o.dt.value, o.time.value))[1]
+        bad = {k: bitwise_mismatch(g.download(k), o[k]) for k in KEYS}
+        assert not any(bad.values()), bad
+        g.close()
+        # and the production kernels against the routine-by-routine path
+        g, r = fwgpu.Solver(st, prec), fwgpu.Solver(st, prec, full_state=True)
+        assert g.step(3) == r.step(3)
+        bad = {k: bitwise_mismatch(g.download(k), r.download(k)) for k in KEYS}
+        assert not any(bad.values()), bad
+        g.close()
+        r.close()
+
+
+@pytest.mark.parametrize("prec", ["sp", "dp"])
+@pytest.mark.parametrize("periodic", [False, True])
+def test_batch_with_a_long_member(periodic, prec, gpu_available):
+    """One member past the LDS limit puts every member's lines on the path
+    through memory: each as alone, where the short ones stay in LDS."""
+    import fwgpu
+    long = 2113 if prec == "sp" else 1025
+    sizes = [(long, 4), (65, 7), (130, 20), (16, 5)] if periodic else [(long, 4), (65, 7), (7, 130), (5, long)]
+    print(f"\n[line solves] batch {sizes} {prec}", flush=True)
+    sts = [dict(_state(m, n, prec, True, False, periodic=periodic), FIXED_DT=1, DT_fixed=0.03125) for m, n in sizes]
+    gs, alone = ([fwgpu.Solver(st, prec) for st in sts] for _ in range(2))
+    b = fwgpu.Batch(gs)
+    b.step(3)
+    for g, a in zip(gs, alone):
+        a.step(3)
+        assert g.clock == a.clock
+        bad = {k: bitwise_mismatch(g.download(k), a.download(k)) for k in KEYS}
+        assert not any(bad.values()), (g.M, g.N, bad)
+    b.close()
+    for s in gs + alone:
+        s.close()
+
+
+# whole steps of the production path at the sizes whose edge cells mirror across
+# several walls, against the routine-by-routine path; wet everywhere (MASK9
+# stays 1, and the second stage forms no c') or drying
+@pytest.mark.parametrize("prec", ["sp", "dp"])
+@pytest.mark.parametrize("m,n", [(3, 3), (3, 8), (8, 3), (4, 5), (6, 6), (7, 31), (33, 5), (64, 16), (65, 129)])
+@pytest.mark.parametrize("dry", [False, True])
+def test_small_production_steps_match_routines(dry, m, n, prec, gpu_available):
+    import fwgpu
+    for visc, sponge in ((True, True), (False, True), (True, False), (False, False)):
+        print(f"\n[line solves] production {m} x {n} {prec} dry={dry} viscosity={visc} sponge={sponge}", flush=True)
+        st = _state(m, n, prec, visc, False)
+        if not dry:
+            st.update(_wet(st))
+        st = dict(st, DIRECT_SPONGE=int(sponge))
+        st["SPONGE"] = 1.0 + 0.5 * np.random.default_rng(m).random(st["SPONGE"].shape).astype(st["SPONGE"].dtype)
+        g, r = fwgpu.Solver(st, prec), fwgpu.Solver(st, prec, full_state=True)
+        for steps in (1, 2, 3):
+            assert g.step(steps) == r.step(steps)
+            bad = {k: bitwise_mismatch(g.download(k), r.download(k)) for k in KEYS}
+            assert not any(bad.values()), bad
+        g.close()
+        r.close()
+
+
+def _wet(st):
+    """The state's waves over a flat bottom."""
+    N, M = st["Depth"].shape
+    d = {k: np.full_like(st[k], 3.0) for k in ("Depth", "DepthX", "DepthY")}
+    d.update(MASK=np.ones((N, M), np.int32), MASK9=np.ones((N, M), np.int32))
+    d["Eta"] = np.where(st["MASK"] > 0, st["Eta"], 0).astype(st["Eta"].dtype)
+    d["H"] = (d["Eta"] + d["Depth"]).astype(st["H"].dtype)
+    return d

@@ -51,3 +51,12 @@ def test_step_matches_routines(m, n, prec, dispersion, gpu_available):
     assert np.count_nonzero(g.download("nu_break")) > 0
     g.close()
     r.close()
+
+
+# ghost cells included, 6 (Mloc + Nloc) = 4092 of them go with the fixed point, 4098
+# by a launch of their own
+@pytest.mark.parametrize("m,n", [(330, 340), (330, 341), (9, 661), (662, 9)])
+@pytest.mark.parametrize("dispersion", [False, True])
+def test_step_on_both_sides_of_the_fill_limit(m, n, dispersion, gpu_available):
+    for prec in ("sp", "dp"):
+        test_step_matches_routines(m, n, prec, dispersion, gpu_available)
