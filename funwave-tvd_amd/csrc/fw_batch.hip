@@ -120,7 +120,7 @@ __global__ void kb_halo_per(FWB_ARGS, int list, int pm) {
   FWB_HEAD
   const HaloList &L = list == 0 ? M.hx[pm] : M.hd;
   if (e.y < L.n) halo_per_body<R>(L.a[e.y], M.g, tile_blk(e));
-  else halo_body<R>(M.hxf[pm].a[e.y - L.n], M.g, 0, tile_blk(e));
+  else halo_body<R>(M.hxf[pm].a[e.y - L.n], M.g, false, tile_blk(e));
 }
 
 // the same where a member is narrow (k_halo_seq)

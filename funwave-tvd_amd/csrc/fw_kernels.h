@@ -140,7 +140,7 @@ template <bool P2, class R> __device__ __forceinline__ Dv<R> dvy(const Prm<R> &p
 // a pure function of one interior value: phi(mi, mj) times the mirror signs.
 // With PERIODIC, the y ghost rows are copied first over all columns (the
 // x-ghost columns still holding their previous values) and the x ghosts are
-// filled afterwards; that takes two ordered launches (modes 1 and 2).
+// filled afterwards (halo_per_body).
 struct HaloArr {
   void *p;
   int vtype;   // 1 even, 2 odd in x, 3 odd in y
@@ -164,41 +164,38 @@ __device__ __forceinline__ HaloSpec halo_spec(const Geo &g, int spec) {
 }
 
 // ghost index t -> (i, j); bottom rows, top rows, then left/right columns of
-// interior rows.  Returns false past the end.
-__device__ __forceinline__ bool halo_pos(const HaloSpec &s, int t, int mode, int &i, int &j) {
+// interior rows (ycopy: the first two only).  Returns false past the end.
+__device__ __forceinline__ bool halo_pos(const HaloSpec &s, int t, bool ycopy, int &i, int &j) {
   int rows = 3 * s.Ma;
   int nr = s.Je - s.Jb + 1;
-  if (mode != 2) {
-    if (t < rows) { j = 1 + t / s.Ma; i = 1 + t % s.Ma; return true; }
-    t -= rows;
-    if (t < rows) { j = s.Je + 1 + t / s.Ma; i = 1 + t % s.Ma; return true; }
-    t -= rows;
-    if (mode == 1) return false;
-  }
+  if (t < rows) { j = 1 + t / s.Ma; i = 1 + t % s.Ma; return true; }
+  t -= rows;
+  if (t < rows) { j = s.Je + 1 + t / s.Ma; i = 1 + t % s.Ma; return true; }
+  t -= rows;
+  if (ycopy) return false;
   if (t < 3 * nr) { j = s.Jb + t / 3; i = 1 + t % 3; return true; }
   t -= 3 * nr;
   if (t < 3 * nr) { j = s.Jb + t / 3; i = s.Ie + 1 + t % 3; return true; }
   return false;
 }
 
-// Ghost fill of one array A; the workgroup's x tile picks its ghost cells.
+// Mirror fill of one array A, or with ycopy its periodic y copy; the workgroup's
+// x tile picks its ghost cells.
 template <class R>
-__device__ __forceinline__ void halo_body(const HaloArr &A, Geo g, int mode, const Blk &B) {
+__device__ __forceinline__ void halo_body(const HaloArr &A, Geo g, bool ycopy, const Blk &B) {
   int t = B.x * blockDim.x + threadIdx.x;
   HaloSpec s = halo_spec(g, A.spec);
   int i, j;
-  if (!halo_pos(s, t, mode, i, j)) return;
+  if (!halo_pos(s, t, ycopy, i, j)) return;
   int si = i, sj = j;
   bool neg = false;
-  if (mode == 1) {  // periodic y copy (raw, no sign)
+  if (ycopy) {  // raw, no sign
     sj = (j <= 3) ? (s.Je - 3 + j) : (3 + (j - s.Je));
   } else {
     if (i < s.Ib) { si = 2 * s.Ib - 1 - i; neg ^= (A.vtype == 2); }
     if (i > s.Ie) { si = 2 * s.Ie + 1 - i; neg ^= (A.vtype == 2); }
-    if (mode == 0) {
-      if (j < s.Jb) { sj = 2 * s.Jb - 1 - j; neg ^= (A.vtype == 3); }
-      if (j > s.Je) { sj = 2 * s.Je + 1 - j; neg ^= (A.vtype == 3); }
-    }
+    if (j < s.Jb) { sj = 2 * s.Jb - 1 - j; neg ^= (A.vtype == 3); }
+    if (j > s.Je) { sj = 2 * s.Je + 1 - j; neg ^= (A.vtype == 3); }
   }
   if (A.isint) {
     int *ph = (int *)A.p;
@@ -209,15 +206,14 @@ __device__ __forceinline__ void halo_body(const HaloArr &A, Geo g, int mode, con
     ph[IX(i, j)] = neg ? -v : v;
   }
 }
-// One array of the list per grid row (blockIdx.y): within a mode every ghost
-// value is read from interior cells only, so the arrays are independent and
-// their fills run side by side instead of one load-store round trip after
-// another.
+// One array of the list per grid row (blockIdx.y): every ghost value is read
+// from interior cells only, so the arrays are independent and their fills run
+// side by side instead of one load-store round trip after another.
 template <class R>
-__global__ void k_halo(HaloList L, Geo g, int mode) {
-  halo_body<R>(L.a[blockIdx.y], g, mode, grid_blk());
+__global__ void k_halo(HaloList L, Geo g) {
+  halo_body<R>(L.a[blockIdx.y], g, false, grid_blk());
 }
-// Periodic fill of one cell array (modes 1 and 2 in one pass).  An x-ghost
+// Periodic fill of one cell array in one pass.  An x-ghost
 // cell of an interior row first gives the value it holds to the y-ghost rows
 // that copy its row, as the reference's y copy does before its x fill, and
 // then takes its mirror value; the y-ghost rows of the interior columns copy
@@ -255,7 +251,7 @@ template <class R>
 __device__ __forceinline__ void halo_seq_body(const HaloArr &A, const Geo &g, bool per, int phase, const Blk &B) {
   const bool copy = per && A.spec == 0;
   if (phase == 0) {
-    if (copy) halo_body<R>(A, g, 1, B);
+    if (copy) halo_body<R>(A, g, true, B);
     return;
   }
   if (phase == 2 && copy) return;
@@ -286,7 +282,7 @@ __global__ void k_halo_seq(HaloList L, HaloList Lf, Geo g, int per, int phase) {
 template <class R>
 __global__ void k_halo_per(HaloList L, HaloList Lf, Geo g) {
   if ((int)blockIdx.y < L.n) halo_per_body<R>(L.a[blockIdx.y], g, grid_blk());
-  else halo_body<R>(Lf.a[blockIdx.y - L.n], g, 0, grid_blk());
+  else halo_body<R>(Lf.a[blockIdx.y - L.n], g, false, grid_blk());
 }
 
 // --------------------------------------------------------------------------
@@ -2086,10 +2082,10 @@ __global__ void __launch_bounds__(WideLB<R>::wg256) k_huv(Dev<R> d, Geo g, Prm<R
 // the c' chain (12 dependent operations, the correctly rounded division
 // among them, ~116 cycles per row) set the pace and d' followed; with den
 // known ahead, the quotient d' is four dependent operations (below).
-// Measured at 2048 x 2048 rows, FP32, x and y lines together: 164 -> 117 us per
-// solve beside UPDATE_MASK and WAVE_BREAKING (106 alone); k_trid_fac takes
-// 157 us beside the dispersion and the fluxes of two stages per call.  1024 x 4
-// periodic (x lines one per thread before): 456 -> 40 us; 96 x 72: 43 -> 11;
+// Measured at 2048 x 2048 rows, FP32, x and y lines together: 103 us per solve
+// (the one sweep took 164, beside UPDATE_MASK and WAVE_BREAKING); k_trid_fac takes
+// 140 us beside the dispersion and the fluxes of two stages per call.  1024 x 4
+// periodic (x lines one per thread before): 456 -> 37 us; 96 x 72: 43 -> 9;
 // FP64 1021 x 770: 105 -> 70.
 constexpr int kTridL = 16;    // lines per workgroup: 2 x 2042 lines fill the 256 CUs once
 constexpr int kTridNS = 256;  // staging threads (four waves)
@@ -3666,7 +3662,7 @@ __device__ __forceinline__ void brk2_fill_body(const Dev<R> &d, const Geo &g, co
     for (int k = 0; k < K; k++) {
       int i, j;
       const int t = min(t0 + k * nt, cnt - 1);
-      halo_pos(s, t, 0, i, j);
+      halo_pos(s, t, false, i, j);
       const int si = i < g.Ib ? 2 * g.Ib - 1 - i : (i > g.Ie ? 2 * g.Ie + 1 - i : i);
       const int sj = j < g.Jb ? 2 * g.Jb - 1 - j : (j > g.Je ? 2 * g.Je + 1 - j : j);
       dst[k] = IX(i, j);

@@ -361,7 +361,7 @@ void halo_exchange_list(fw_ctx *c, HaloList &L, HaloList &Lf) {
       launch(c, "halo", k_halo_seq<R>, gr, b, L, Lf, g, per ? 1 : 0, phase);
   } else if (!per) {
     for (int k = 0; k < Lf.n; k++) L.a[L.n++] = Lf.a[k];
-    launch(c, "halo", k_halo<R>, gr, b, L, g, 0);
+    launch(c, "halo", k_halo<R>, gr, b, L, g);
   } else {
     launch(c, "halo", k_halo_per<R>, gr, b, L, Lf, g);
   }
