@@ -34,7 +34,9 @@ enum { FW_CNN_NPARAMS = 9 * 5 * 32 + 32 + 2 * (9 * 32 * 32 + 32) + 9 * 32 * 3 + 
 
 typedef struct fw_cnn fw_cnn;
 
-/* Buffers for batches of up to max_batch samples of H x W cells. */
+/* Buffers for batches of up to max_batch samples of H x W cells, and 2 MB of
+ * pinned host memory for the host arrays.  Calls that take those poll it while
+ * they wait, for up to 20 ms before they block on the stream. */
 int fw_cnn_create(int H, int W, int max_batch, fw_cnn **out);
 int fw_cnn_destroy(fw_cnn *net);
 const char *fw_cnn_strerror(const fw_cnn *net);

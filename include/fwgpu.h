@@ -18,6 +18,10 @@
  * that hand a value back to the host (fw_estimate_dt, fw_step,
  * fw_check_blowup, fw_download, fw_reduce_stats), fw_upload and
  * fw_wave_breaking (which reports FW_E_BREAK_ITER), which wait for it.
+ * Most waits poll a word of pinned host memory, which keeps the calling
+ * thread's CPU busy, for up to 20 ms each before they block on the stream.
+ * Field transfers go through 2 MB of pinned host memory per context, taken
+ * at its first transfer and given back by fw_destroy.
  */
 #ifndef FWGPU_H
 #define FWGPU_H
